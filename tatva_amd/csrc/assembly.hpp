@@ -345,7 +345,7 @@ __device__ __forceinline__ void elem_diag(const double (&X)[Elem<KIND>::NNE][Ele
 
 // Hex8 local node -> sign index i + 2j + 4k (sx, sy, sz > 0 -> i, j, k = 1).
 __host__ __device__ constexpr int hex_bin(int a) {
-  return a == 2 ? 3 : a == 3 ? 2 : a == 6 ? 7 : a == 7 ? 6 : a;
+  return a ^ ((a >> 1) & 1);  // 2 <-> 3 and 6 <-> 7
 }
 
 // In-place sign-product transform v <- H v (unnormalised), stages x, y, z.

@@ -22,6 +22,8 @@ template <int D, class T>
 struct Poisson {
   static constexpr int NC = 1;
   static constexpr bool kSource = true;
+  static constexpr bool kLinear = true;  // the tangent does not depend on the state
+  __device__ __forceinline__ T modulus() const { return T(1); }
   T f;
   const double *ep = nullptr;  // per-element f (n_elements), or NULL
   __device__ __forceinline__ Poisson at(int64_t e) const {
@@ -59,6 +61,7 @@ template <int D, class T>
 struct LinearElastic {
   static constexpr int NC = D;
   static constexpr bool kSource = false;
+  static constexpr bool kLinear = true;
   T mu, lam;
   const double *ep = nullptr;  // per-element (mu, lambda) pairs (n_elements x 2), or NULL
   __device__ __forceinline__ LinearElastic at(int64_t e) const {
@@ -101,6 +104,23 @@ struct LinearElastic {
   __device__ __forceinline__ void dP(const Lin &, const T dG[NC][D], T out[NC][D]) const {
     stress(dG, out);
   }
+  // S[c][k] = sum w B_a,c B_b,k of two nodes -> their stiffness block
+  // mu (tr S) I + mu S^T + lambda S, in place (row-major)
+  __device__ __forceinline__ void row_block(T (&S)[D * D]) const {
+    T tr = T(0);
+#pragma unroll
+    for (int i = 0; i < D; ++i) tr += S[i * D + i];
+    T K[D * D];
+#pragma unroll
+    for (int c = 0; c < D; ++c)
+#pragma unroll
+      for (int k = 0; k < D; ++k) {
+        K[c * D + k] = mu * S[k * D + c] + lam * S[c * D + k];
+        if (c == k) K[c * D + k] += mu * tr;
+      }
+#pragma unroll
+    for (int i = 0; i < D * D; ++i) S[i] = K[i];
+  }
   // w dP (the quadrature weight folded into the moduli)
   __device__ __forceinline__ void dPw(const Lin &, const T dG[NC][D], T w, T out[NC][D]) const {
     stress_with(w * mu, w * lam, dG, out);
@@ -122,6 +142,7 @@ template <int D, class T>
 struct NeoHookean {
   static constexpr int NC = D;
   static constexpr bool kSource = false;
+  static constexpr bool kLinear = false;
   T mu, lam;
   const double *ep = nullptr;  // per-element (mu, lambda) pairs (n_elements x 2), or NULL
   __device__ __forceinline__ NeoHookean at(int64_t e) const {
@@ -132,6 +153,10 @@ struct NeoHookean {
     }
     return r;
   }
+  // the moduli of the tangent: mu, mu - lambda ln J and lambda
+  __device__ __forceinline__ T modulus() const { return mu; }
+  __device__ __forceinline__ T shear_modulus(T J) const { return mu - lam * tlog<T>(J); }
+  __device__ __forceinline__ T bulk_modulus() const { return lam; }
   struct Lin {
     T Fi[D][D];  // F^-1
     T c1;        // mu - lambda ln J

@@ -23,6 +23,7 @@
 #include "common.hpp"
 #include "density.hpp"
 #include "element.hpp"
+#include "hessian.hpp"
 #include "mesh.hpp"
 
 namespace tatva {
@@ -1020,6 +1021,29 @@ extern "C" int tatva_mesh_create(int device, int elem_kind, const double *coords
     }
     m->hex_affine = affine ? 1 : 0;
   }
+  // affine Hex8: the reference element's gradient products over the quadrature
+  // rule (hex8_affine_row_blocks)
+  std::vector<double> ref;
+  if (m->hex_affine) {
+    ref.assign(9 * 64, 0.0);
+    for (int q = 0; q < nq; ++q) {
+      double dn[8][3];
+      for (int b = 0; b < 8; ++b)
+        for (int k = 0; k < 3; ++k) {
+          double v = 0.125;
+          for (int j = 0; j < 3; ++j) {
+            const double sj = (b >> j) & 1 ? 1.0 : -1.0;
+            v *= j == k ? sj : 1.0 + sj * m->quad.xi[q][j];
+          }
+          dn[b][k] = v;
+        }
+      for (int k = 0; k < 3; ++k)
+        for (int l = 0; l < 3; ++l)
+          for (int a = 0; a < 8; ++a)
+            for (int b = 0; b < 8; ++b)
+              ref[(size_t)((k * 3 + l) * 64 + a * 8 + b)] += m->quad.w[q] * dn[a][k] * dn[b][l];
+    }
+  }
   hipError_t err = hipSetDevice(device);
   if (err != hipSuccess) return fail(err, "hipSetDevice");
   if ((err = hipStreamCreateWithFlags(&up, hipStreamNonBlocking)) != hipSuccess) {
@@ -1046,6 +1070,8 @@ extern "C" int tatva_mesh_create(int device, int elem_kind, const double *coords
     if ((err = upload(&m->t_inc_end, T.inc_end, "tiles")) != hipSuccess) return fail(err, "tiles");
     if ((err = upload(&m->t_inc_list, T.inc_list, "tiles")) != hipSuccess) return fail(err, "tiles");
   }
+  if (m->hex_affine && (err = upload(&m->hex_ref, ref, "reference element")) != hipSuccess)
+    return fail(err, "reference element");
   m->tiles = TileSet{T.n_tiles, T.max_local, T.max_colors, 0, m->t_lnodes,
                      m->t_color_off, m->t_node_ptr, m->t_slot_ptr, m->t_slot_pos,
                      m->t_tnodes, m->t_inc_end, m->t_inc_list, m->t_elem};
@@ -1093,7 +1119,7 @@ extern "C" int tatva_mesh_destroy(tatva_mesh *m) {
   for (void *p : {(void *)m->t_lnodes, (void *)m->t_color_off,
                   (void *)m->t_node_ptr, (void *)m->t_slot_ptr, (void *)m->t_slot_pos,
                   (void *)m->t_tnodes, (void *)m->t_inc_end, (void *)m->t_inc_list,
-                  (void *)m->t_elem,
+                  (void *)m->t_elem, (void *)m->hex_ref,
                   (void *)m->loc_ptr, (void *)m->loc_elems})
     if (p) (void)hipFree(p);
   delete m;
@@ -1459,20 +1485,48 @@ extern "C" int tatva_colored_hessian(tatva_mesh *m, const tatva_density *d, cons
   TATVA_REQUIRE(n_colors >= 1 && n_colors <= kMaxColors, "n_colors must be in [1, 2048]");
   TATVA_REQUIRE((dof_map == nullptr) == (red_to_full == nullptr),
                 "dof_map and red_to_full must be given together");
+  TATVA_REQUIRE(n_rows > 0, "the pattern has no rows");
   const int nc = density_ncomp(m, d);
   if (!dof_map) TATVA_REQUIRE(n_rows == m->n_nodes * nc, "pattern size does not match the mesh dofs");
   const int64_t need = tatva_colored_hessian_workspace(m, nc);
   TATVA_REQUIRE(workspace && ws_bytes >= need, "colored Hessian workspace too small");
   (void)nnz;
   hipStream_t s = (hipStream_t)stream;
-  double *Ke = (double *)workspace;
-  const int rows_per_block = kBlock / kWave;
-  const size_t lds = (size_t)rows_per_block * n_colors * sizeof(double);
   return with_kind(m->kind, [&](auto kc) -> int {
     constexpr int K = decltype(kc)::value;
     return with_density<Elem<K>::D, double>(d, [&](auto dens) -> int {
       using Dens = decltype(dens);
       constexpr int NNE = Elem<K>::NNE, NC = Dens::NC;
+      using Sh = RowsShape<K, NC>;
+      // node rows: as many nodes per block as its LDS holds, in whole waves
+      const size_t wave_lds = (kWave / Sh::LG) * Sh::lds_bytes(n_colors);
+      const int waves = (int)std::min<size_t>(kBlock / kWave, kTileLdsMax / wave_lds);
+      if (waves >= 1) {
+        const int threads = waves * kWave, per = threads / Sh::LG;
+        const auto launch = [&](auto affine, auto mapped) {
+          k_node_rows<K, Dens, decltype(affine)::value, decltype(mapped)::value>
+              <<<grid_for(m->n_nodes, per), threads, per * Sh::lds_bytes(n_colors), s>>>(
+                  m->n_nodes, n_rows, m->coords, m->conn, m->quad, m->hex_ref, dens, u, dof_map,
+                  colors, n_colors, indptr, indices, m->inv_ptr, m->inv_list, data);
+        };
+        const auto with_map = [&](auto affine) {
+          if (dof_map) launch(affine, std::true_type{});
+          else launch(affine, std::false_type{});
+        };
+        if constexpr (K == TATVA_HEX8 && Dens::kLinear) {
+          if (m->hex_affine) with_map(std::true_type{});
+          else with_map(std::false_type{});
+        } else {
+          with_map(std::false_type{});
+        }
+        TATVA_CHECK_LAUNCH();
+        return TATVA_OK;
+      }
+      // so many colors that a wave's rows do not fit: one row per wave, from
+      // the element stiffness
+      double *Ke = (double *)workspace;
+      const int rows_per_block = kBlock / kWave;
+      const size_t lds = (size_t)rows_per_block * n_colors * sizeof(double);
       const int64_t nthreads = m->n_elements * NNE * NC;
       k_elem_stiffness<K, Dens><<<grid_for(nthreads), kBlock, 0, s>>>(
           m->n_elements, m->coords, m->conn, m->quad, dens, u, Ke);

@@ -1,0 +1,132 @@
+"""GPU kernels at the sizes where their work splits: tile and lane remainders,
+quadrature rules of other lengths, nodes shared by many elements, patterns with
+many colors.  Each against the FP64 oracle; FP64 results to 1e-12 relative to
+the largest entry (summation order and cofactor inverses, as the parity tests)."""
+
+import numpy as np
+import pytest
+import scipy.sparse as sps
+
+import tatva_amd as ta
+from oracle import fem
+from tatva_amd import energies, lifter, sparse
+
+pytestmark = pytest.mark.gpu
+
+RTOL = 1e-12
+ORACLE_EL = {ta.Tri3: fem.Tri3, ta.Tetrahedron4: fem.Tet4, ta.Hexahedron8: fem.Hex8}
+
+
+def to_np(t):
+    return t.detach().cpu().numpy()
+
+
+def rel_err(a, b):
+    a, b = np.asarray(a, dtype=np.float64), np.asarray(b, dtype=np.float64)
+    return np.max(np.abs(a - b)) / max(np.max(np.abs(b)), 1e-300)
+
+
+def gauss(points_1d, dim=3):
+    x, w = np.polynomial.legendre.leggauss(points_1d)
+    g = np.meshgrid(*[x] * dim, indexing="ij")
+    h = np.meshgrid(*[w] * dim, indexing="ij")
+    return np.stack([a.ravel() for a in g], -1), np.prod([a.ravel() for a in h], axis=0)
+
+
+def fan(kind, k):
+    """k elements around one node or axis: triangles around a center, tetrahedra
+    around a center (a triangulated sphere of k caps, two rings), hexahedra
+    around a vertical axis (two layers)."""
+    t = 2 * np.pi * np.arange(k) / k
+    if kind == "tri3":
+        X = np.vstack([[0.0, 0.0], np.c_[np.cos(t), np.sin(t)]])
+        i = np.arange(k)
+        return ta.Mesh(X, np.c_[np.zeros(k, int), 1 + i, 1 + (i + 1) % k])
+    if kind == "tet4":
+        ring = np.c_[np.cos(t), np.sin(t), np.zeros(k)]
+        X = np.vstack([[0.0, 0.0, 0.0], [0.1, 0.0, 0.9], [0.0, -0.1, -1.1], ring])
+        i = np.arange(k)
+        a, b, o = 3 + i, 3 + (i + 1) % k, np.zeros(k, int)
+        return ta.Mesh(X, np.vstack([np.c_[o, a, b, o + 1], np.c_[o, b, a, o + 2]]))
+    # k quads (center, two spokes and the corner between them), extruded twice
+    r = np.vstack([[0.0, 0.0], np.c_[np.cos(t), np.sin(t)],
+                   1.3 * np.c_[np.cos(t + np.pi / k), np.sin(t + np.pi / k)]])
+    n = r.shape[0]
+    X = np.vstack([np.c_[r * s, np.full(n, z)] for z, s in ((0.0, 1.0), (0.7, 1.1), (1.5, 0.9))])
+    i = np.arange(k)
+    quad = np.c_[np.zeros(k, int), 1 + i, 1 + k + i, 1 + (i + 1) % k]
+    return ta.Mesh(X, np.vstack([np.c_[quad + l * n, quad + (l + 1) * n] for l in (0, 1)]))
+
+
+def hessian_pair(mesh, el, density, od, colors=None, fixed=None):
+    """Colored Hessian data on the GPU, and the oracle's element stiffness summed
+    into the same pattern."""
+    nc = density.ncomp(el.dim)
+    n = mesh.n_nodes * nc
+    rng = np.random.default_rng(7)
+    u = 0.02 * rng.standard_normal(n)
+    E = ta.Operator(mesh, el).energy(density)
+    S = sparse.pattern_from_mesh(mesh, nc)
+    prob = fem.Problem(ORACLE_EL[type(el)](el.quad_points, el.quad_weights), mesh.coords,
+                       mesh.elements, od)
+    fixed = np.zeros(0, int) if fixed is None else fixed
+    L = lifter.Lifter(n, lifter.Fixed(fixed, 0.0))
+    u[fixed] = 0.0
+    cm = sparse.ColoredMatrix.from_csr(L.adapt_sparsity(S),
+                                       None if colors is None else colors(L.size_reduced))
+    E_red = E.reduced(L) if fixed.size else E
+    K = sparse.jacfwd(E_red.grad, cm)(u[L.free_dofs] if fixed.size else u)
+    dofs = (mesh.elements[:, :, None] * nc + np.arange(nc)).reshape(mesh.n_elements, -1)
+    Ke = prob.element_stiffness(u).reshape(mesh.n_elements, dofs.shape[1], dofs.shape[1])
+    pair = L.dof_map[np.stack(np.broadcast_arrays(dofs[:, :, None], dofs[:, None, :]))]
+    keep = (pair >= 0).all(axis=0)
+    ref = sps.coo_matrix((Ke[keep], (pair[0][keep], pair[1][keep])), shape=cm.shape).tocsr()
+    ref.sort_indices()
+    assert np.array_equal(ref.indices, K.to_csr().indices)
+    return to_np(K.data), ref.data
+
+
+LE, NH, PO = (energies.LinearElasticity(0.7, 1.3), energies.NeoHookean(0.7, 1.3),
+              energies.Poisson(1.5))
+ORACLE = {LE: fem.LinearElasticity(0.7, 1.3), NH: fem.NeoHookean(0.7, 1.3), PO: fem.Poisson(1.5)}
+
+
+@pytest.mark.parametrize("density", [LE, NH, PO], ids=["le", "nh", "poisson"])
+@pytest.mark.parametrize("kind,k", [("tri3", 3), ("tri3", 16), ("tri3", 17), ("tri3", 40),
+                                    ("tet4", 3), ("tet4", 16), ("tet4", 17), ("tet4", 40),
+                                    ("hex8", 3), ("hex8", 4), ("hex8", 5), ("hex8", 9)])
+def test_hessian_rows_of_a_node_in_many_elements(kind, k, density):
+    """Nodes in fewer, exactly and more elements than a node's lanes hold at a
+    time (16 triangles, 32 tetrahedra, 8 hexahedra)."""
+    el = {"tri3": ta.Tri3, "tet4": ta.Tetrahedron4, "hex8": ta.Hexahedron8}[kind]()
+    got, ref = hessian_pair(fan(kind, k), el, density, ORACLE[density])
+    assert rel_err(got, ref) < RTOL
+
+
+@pytest.mark.parametrize("density", [LE, NH, PO], ids=["le", "nh", "poisson"])
+@pytest.mark.parametrize("jitter", [0.0, 0.15])
+@pytest.mark.parametrize("points", [1, 2, 3])
+def test_hessian_rows_hex8_quadrature_rules(points, jitter, density):
+    """1, 8 and 27 points over eight lanes; parallelepipeds and general elements;
+    rows and columns of constrained dofs left out."""
+    qp, qw = gauss(points)
+    mesh = ta.Mesh.box((4, 3, 5), jitter=jitter, seed=2)
+    nc = density.ncomp(3)
+    fixed = np.r_[0:4 * nc, [11 * nc, 30 * nc + nc - 1]]
+    got, ref = hessian_pair(mesh, ta.Hexahedron8(qp, qw), density, ORACLE[density], fixed=fixed)
+    assert rel_err(got, ref) < RTOL
+
+
+@pytest.mark.parametrize("kind,shape", [("tri3", (29, 30)), ("tet4", (8, 8, 7)), ("hex8", (8, 8, 7))])
+def test_hessian_rows_of_many_colors(kind, shape):
+    """Almost 2048 colors: one wave's rows fill the LDS (Hex8) or do not fit and
+    the rows come from the element stiffness (Tri3, Tet4)."""
+    if kind == "tri3":
+        mesh, el = ta.Mesh.unit_square(*shape), ta.Tri3()
+    elif kind == "tet4":
+        mesh, el = ta.Mesh.box(shape, type="tetrahedron", jitter=0.1, seed=3), ta.Tetrahedron4()
+    else:
+        mesh, el = ta.Mesh.box(shape, jitter=0.1, seed=3), ta.Hexahedron8()
+    assert 1800 < mesh.n_nodes * el.dim <= 2048
+    got, ref = hessian_pair(mesh, el, LE, ORACLE[LE], colors=np.arange)
+    assert rel_err(got, ref) < RTOL
