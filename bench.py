@@ -417,7 +417,8 @@ def hvp_tile_bytes(op, dens_ncomp=3, cached_lin=0, geo=False, defer_n=0, mapped=
     """Algorithmic bytes of one FP32 HVP tile-kernel launch (k_tile_assemble,
     matrix-free PCG operator), from the mesh's device layout: per element its
     nne uint16 local node numbers (+ cached linearisation floats per quadrature
-    point, + its 44-byte geometry cache entry, if any), per (tile, local node)
+    point, + its geometry cache entry, if any: geo bytes, True for the 44 of a
+    parallelepiped; a box along the axes has 20), per (tile, local node)
     slot its global node (int32), the node's FP64 coordinates (not with the
     geometry cache), FP32 state and tangent, the tangent's dof-map entries
     (int32) and the slot's FP32 partial sums written and the int32 position it
@@ -435,7 +436,7 @@ def hvp_tile_bytes(op, dens_ncomp=3, cached_lin=0, geo=False, defer_n=0, mapped=
     nne = 8 if op.element.kind == 2 else (4 if op.element.kind == 1 else 3)
     d = 3 if nne != 3 else 2
     nc = dens_ncomp
-    b = 2 * nne * E + 4 * cached_lin * lay["n_quad"] * E + (44 * E if geo else 0)
+    b = 2 * nne * E + 4 * cached_lin * lay["n_quad"] * E + (44 if geo is True else int(geo)) * E
     b += S * (4 + (0 if geo else 8 * d) + 4 * nc * (0 if cached_lin else 1)
               + (4 if mapped else 0) * nc + 4 * nc + 4 * nc + 4)
     incidence = nne in (4, 8)
@@ -586,7 +587,7 @@ def headline(args):
     defer = not args.no_defer
     full_vec = not args.no_full_vectors
     n_vec = mesh.n_nodes * 3 if full_vec else n_free   # length of the CG vectors
-    tile_bytes, lay = hvp_tile_bytes(op, cached_lin=10 if cached else 0, geo=geo,
+    tile_bytes, lay = hvp_tile_bytes(op, cached_lin=10 if cached else 0, geo=20 if geo else False,
                                      defer_n=n_vec if defer else 0, mapped=not full_vec)
     hbm_rate = tile_bytes / (tile_us * 1e-6) / 1e9 if tile_us else None
     # the profile's counters are those of the default kernel on this workload
@@ -618,7 +619,7 @@ def headline(args):
         "roofline": {
             "kernel": (f"k_tile_assemble<HEX8, NeoHookean<3,float>, float, "
                        f"{'kModeHvpLin' if cached else 'kModeHvp'}, "
-                       f"{'kGeomCache' if geo else 'kGeomAffine'}> (FP32 HVP tile kernel of the "
+                       f"{'kGeomBoxCache' if geo else 'kGeomBox'}> (FP32 HVP tile kernel of the "
                        "matrix-free PCG operator)"),
             "bound": "valu",
             "achieved": achieved,

@@ -93,7 +93,8 @@ int tatva_set_profiling(int enable);
  * TATVA_OPT_MATFREE_GEOM_CACHE: whether tatva_pcg_matfree_f32 on an affine
  * Hex8 mesh (every element a parallelepiped) writes each element's Jacobian
  * inverse (FP32) and det J (FP64) once per solve, 44 bytes per element in the
- * workspace, so that every HVP reads them instead of the node coordinates (the
+ * workspace (20 on meshes of boxes along the axes, where it is diagonal), so
+ * that every HVP reads them instead of the node coordinates (the
  * values the product computes itself, so the same result bit for bit): 1
  * (default) on affine Hex8 meshes, 0 never.  Both caches are in the workspace
  * only when selected: set the options before querying its size.

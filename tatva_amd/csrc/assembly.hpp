@@ -65,15 +65,23 @@ enum { kModeResidual = 0, kModeHvp = 1, kModeDiag = 2, kModeLinearize = 3, kMode
 // every quadrature point from the node coordinates.  kGeomAffine: a Hex8
 // parallelepiped, its Jacobian inverted once per element.  kGeomCache: an
 // affine Hex8 mesh whose geometry is read from a cache written once per solve
-// (FP32 HVP / linearisation only).
-enum { kGeomGeneral = 0, kGeomAffine = 1, kGeomCache = 2 };
+// (FP32 HVP / linearisation only).  kGeomBox, kGeomBoxCache: the same where
+// every element is a box along the coordinate axes (a structured grid): the
+// Jacobian is diagonal, so a gradient takes three products instead of nine of
+// three terms, and the geometry is three edge lengths (against kGeomAffine /
+// kGeomCache: 160^3 Neo-Hookean FP32 product 341 -> 287 us, in the PCG 299 -> 268
+// us; 64^3 linear elastic in the PCG 18.8 -> 17.0 us; 64^3 Neo-Hookean FP64
+// 47.5 -> 42.8 us).
+enum { kGeomGeneral = 0, kGeomAffine = 1, kGeomCache = 2, kGeomBox = 3, kGeomBoxCache = 4 };
+constexpr bool geom_cached(int geom) { return geom == kGeomCache || geom == kGeomBoxCache; }
+constexpr bool geom_box(int geom) { return geom == kGeomBox || geom == kGeomBoxCache; }
 
 // Geometry cache layout (affine Hex8): value k of the element in tile slot t
-// of tile b at geo[(b * kGeoFloats + k) * kTile + t] (a tile's threads read
-// consecutive floats): the FP32 cast of the FP64 Jacobian inverse (9 values,
-// row-major) and the FP64 det J as two 32-bit words, the values the kernels
-// computing the geometry themselves use.
-constexpr int kGeoFloats = 11;
+// of tile b at geo[(b * G + k) * kTile + t] (a tile's threads read consecutive
+// floats): the FP32 cast of the FP64 Jacobian inverse (9 values, row-major;
+// boxes: the 3 on its diagonal) and the FP64 det J as two 32-bit words, the
+// values the kernels computing the geometry themselves use.
+constexpr int geo_floats(bool box) { return box ? 5 : 11; }
 
 // The p and x updates of an FP32 conjugate-gradient iteration, which its step
 // kernel leaves to the next operator launch (nothing reads p or x in between):
@@ -441,18 +449,38 @@ __device__ __forceinline__ double hex8_affine_inverse(const double (&X)[8][3], T
   return det;
 }
 
+// The same for a box along the axes, from two opposite nodes: with equal edges
+// the modes above are exactly half an edge length, and the zeros of the Jacobian
+// leave det = J00 (J11 J22) and the diagonal of the inverse.
+template <class T>
+__device__ __forceinline__ double hex8_box_inverse(const double (&lo)[3], const double (&hi)[3],
+                                                   T (&iv)[3]) {
+#pragma clang fp contract(off)
+  double J[3];
+#pragma unroll
+  for (int j = 0; j < 3; ++j) J[j] = 0.5 * (hi[j] - lo[j]);
+  const double c00 = J[1] * J[2];
+  const double det = J[0] * c00;
+  const double r = 1.0 / det;
+  iv[0] = T(c00 * r);
+  iv[1] = T((J[0] * J[2]) * r);
+  iv[2] = T((J[0] * J[1]) * r);
+  return det;
+}
+
 // Hex8 residual (MODE = kModeResidual: S = P(G), plus the Poisson source) or
 // Hessian-vector product (S = dP(G(u); G(v))): ye = sum_q w_q B_q^T S_q.
 // Geometry in FP64, physics in T.
 // MODE kModeLinearize / kModeHvpLin: as elem_hvp (cache at lin, stride kTile).
-// GEO (affine only): J^-1 and det J read from geo (this element's geometry
-// cache, stride kTile) instead of computed from X.
-template <class Dens, class T, int MODE, bool AFFINE, bool GEO = false>
+// GEOM: AFFINE for all but kGeomGeneral; the cached ones read J^-1 and det J
+// from geo (this element's geometry cache, stride kTile) instead of computing
+// them from X, the box ones hold the diagonal of J^-1 only (X: nodes 0 and 6).
+template <class Dens, class T, int MODE, int GEOM>
 __device__ __forceinline__ void hex8_element(const double (&X)[8][3], const T (&ue)[8][Dens::NC],
                                              const T (&ve)[8][Dens::NC], const QuadRule &quad,
                                              const Dens &dens, T (&ye)[8][Dens::NC],
                                              T *lin = nullptr, const T *geo = nullptr) {
-  static_assert(!GEO || AFFINE, "the Hex8 geometry cache holds one inverse per element");
+  constexpr bool AFFINE = GEOM != kGeomGeneral, GEO = geom_cached(GEOM), BOX = geom_box(GEOM);
   constexpr int NC = Dens::NC;
   constexpr bool kUsesU = MODE != kModeHvpLin;
   constexpr bool kUsesV = MODE == kModeHvp || MODE == kModeHvpLin;
@@ -474,7 +502,18 @@ __device__ __forceinline__ void hex8_element(const double (&X)[8][3], const T (&
   // values each point would cast from the FP64 inverse)
   T iv0[3][3] = {};
   double det0 = 0.0;
-  if constexpr (GEO) {
+  if constexpr (GEO && BOX) {
+#pragma unroll
+    for (int j = 0; j < 3; ++j) iv0[j][j] = geo[j * kTile];
+    const uint32_t lo = __float_as_uint(float(geo[3 * kTile]));
+    const uint32_t hi = __float_as_uint(float(geo[4 * kTile]));
+    det0 = __hiloint2double((int)hi, (int)lo);
+  } else if constexpr (BOX) {
+    T iv[3];
+    det0 = hex8_box_inverse<T>(X[0], X[6], iv);
+#pragma unroll
+    for (int j = 0; j < 3; ++j) iv0[j][j] = iv[j];
+  } else if constexpr (GEO) {
 #pragma unroll
     for (int i = 0; i < 3; ++i)
 #pragma unroll
@@ -526,7 +565,8 @@ __device__ __forceinline__ void hex8_element(const double (&X)[8][3], const T (&
         T h[3];
         hex_dmodes<T>(UM[c], xt, yt, zt, yz, xz, xy, h);
 #pragma unroll
-        for (int j = 0; j < 3; ++j) G[c][j] = h[0] * iv[j][0] + h[1] * iv[j][1] + h[2] * iv[j][2];
+        for (int j = 0; j < 3; ++j)
+          G[c][j] = BOX ? h[j] * iv[j][j] : h[0] * iv[j][0] + h[1] * iv[j][1] + h[2] * iv[j][2];
       }
     }
     T *lq = (MODE == kModeLinearize || MODE == kModeHvpLin)
@@ -544,7 +584,8 @@ __device__ __forceinline__ void hex8_element(const double (&X)[8][3], const T (&
         T h[3];
         hex_dmodes<T>(VM[c], xt, yt, zt, yz, xz, xy, h);
 #pragma unroll
-        for (int j = 0; j < 3; ++j) dG[c][j] = h[0] * iv[j][0] + h[1] * iv[j][1] + h[2] * iv[j][2];
+        for (int j = 0; j < 3; ++j)
+          dG[c][j] = BOX ? h[j] * iv[j][j] : h[0] * iv[j][0] + h[1] * iv[j][1] + h[2] * iv[j][2];
       }
       // S = w dP(G; dG): the weight folded into the density's moduli
       if constexpr (MODE == kModeHvpLin) {
@@ -563,7 +604,8 @@ __device__ __forceinline__ void hex8_element(const double (&X)[8][3], const T (&
       T Q[3];
 #pragma unroll
       for (int k = 0; k < 3; ++k) {
-        const T sk = S[c][0] * iv[0][k] + S[c][1] * iv[1][k] + S[c][2] * iv[2][k];
+        const T sk = BOX ? S[c][k] * iv[k][k]
+                         : S[c][0] * iv[0][k] + S[c][1] * iv[1][k] + S[c][2] * iv[2][k];
         Q[k] = MODE == kModeResidual ? w * sk : sk;
       }
       A[c][1] += Q[0];
@@ -598,9 +640,11 @@ __device__ __forceinline__ void hex8_element(const double (&X)[8][3], const T (&
   }
 }
 
-// True when the element's bilinear coordinate modes are all exactly zero
-// (computed with the same butterfly as hex_modes).
-inline bool hex_is_affine_host(const double (&X)[8][3]) {
+// 1 when the element's bilinear coordinate modes are all exactly zero (computed
+// with the same butterfly as hex_modes), 2 when its Jacobian is diagonal too
+// (a box along the axes, whose edges along an axis are then equal), else 0.
+inline int hex_affine_host(const double (&X)[8][3]) {
+  int kind = 2;
   for (int j = 0; j < 3; ++j) {
     double v[8];
     for (int a = 0; a < 8; ++a) v[hex_bin(a)] = X[a][j];
@@ -611,9 +655,11 @@ inline bool hex_is_affine_host(const double (&X)[8][3]) {
           v[b] = hi + lo;
           v[b | h] = hi - lo;
         }
-    if (v[3] != 0.0 || v[5] != 0.0 || v[6] != 0.0 || v[7] != 0.0) return false;
+    if (v[3] != 0.0 || v[5] != 0.0 || v[6] != 0.0 || v[7] != 0.0) return 0;
+    for (int k = 0; k < 3; ++k)
+      if (k != j && v[1 << k] != 0.0) kind = 1;
   }
-  return true;
+  return kind;
 }
 
 // ------------------------------------------------------ tile assembly ------
@@ -647,9 +693,8 @@ constexpr size_t tile_lds_bytes(int kind, int max_local, int D, int nne, int NC,
 constexpr size_t kTileLdsMax = 65536;  // LDS one workgroup may allocate
 
 // Body of one tile (one workgroup of kTile threads; lds of tile_lds_bytes).
-// GEOM (kGeomGeneral / kGeomAffine / kGeomCache): how the elements' geometry
-// is taken; with kGeomCache the FP32 HVP and linearisation read it from geo
-// instead of the node coordinates.  u: full state; v (HVP): tangent read through dof_map
+// GEOM: how the elements' geometry is taken; with a cached one the FP32 HVP and
+// linearisation read it from geo instead of the node coordinates.  u: full state; v (HVP): tangent read through dof_map
 // (reduced, zero on constrained dofs).  The tile's local nodes are loaded into
 // LDS once (one thread per node), so each element reads its nodes from LDS
 // instead of gathering them from global memory.  Writes the sums of local node
@@ -668,9 +713,11 @@ __device__ __forceinline__ void tile_assemble(int tile, const double *__restrict
   using El = Elem<KIND>;
   constexpr int D = El::D, NNE = El::NNE, NC = Dens::NC;
   // a geometry cache (affine Hex8 HVP / linearisation) replaces the coordinates
-  constexpr bool kAffine = KIND == TATVA_HEX8 && GEOM != kGeomGeneral;
-  constexpr bool kGeo = KIND == TATVA_HEX8 && GEOM == kGeomCache && sizeof(T) == 4 &&
-                        (MODE == kModeHvp || MODE == kModeHvpLin || MODE == kModeLinearize);
+  constexpr bool kGeo = geom_cached(GEOM);
+  static_assert(GEOM == kGeomGeneral || KIND == TATVA_HEX8, "the geometry variants are Hex8");
+  static_assert(!kGeo || (sizeof(T) == 4 && (MODE == kModeHvp || MODE == kModeHvpLin ||
+                                             MODE == kModeLinearize)),
+                "a geometry cache serves the FP32 product");
   constexpr bool uses_x = !kGeo;
   const int32_t nb = ts.node_ptr[tile];
   const int nloc = ts.node_ptr[tile + 1] - nb;
@@ -794,14 +841,15 @@ __device__ __forceinline__ void tile_assemble(int tile, const double *__restrict
     }
     // this thread's cached linearisation (kModeLinearize / kModeHvpLin)
     T *lp = lin ? lin + (int64_t)tile * quad.nq * Dens::kLin * kTile + threadIdx.x : nullptr;
-    const T *gp = kGeo ? geo + (int64_t)tile * kGeoFloats * kTile + threadIdx.x : nullptr;
+    const T *gp =
+        kGeo ? geo + (int64_t)tile * geo_floats(geom_box(GEOM)) * kTile + threadIdx.x : nullptr;
     if constexpr (KIND == TATVA_HEX8 && MODE == kModeResidual) {
-      hex8_element<Dens, T, kModeResidual, kAffine>(X, ue, ue, quad, de, ye);
+      hex8_element<Dens, T, kModeResidual, GEOM>(X, ue, ue, quad, de, ye);
     } else if constexpr (MODE == kModeResidual) {
       elem_residual<KIND, Dens>(X, ue, quad, de, ye);
     } else if constexpr (MODE == kModeHvp || MODE == kModeHvpLin || MODE == kModeLinearize) {
       if constexpr (KIND == TATVA_HEX8)
-        hex8_element<Dens, T, MODE, kAffine, kGeo>(X, ue, ve, quad, de, ye, lp, gp);
+        hex8_element<Dens, T, MODE, GEOM>(X, ue, ve, quad, de, ye, lp, gp);
       else elem_hvp<KIND, Dens, T, MODE>(X, ue, ve, quad, de, ye, lp);
     } else {
       elem_diag<KIND, Dens, T>(X, ue, quad, de, ye);

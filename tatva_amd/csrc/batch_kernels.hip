@@ -4,7 +4,7 @@
 // share the launches instead of queueing behind each other.
 //
 // Per iteration (tick t), with one class = slots of equal (element kind,
-// density kind, quadrature rule, affine Hex8 flag):
+// density kind, quadrature rule, Hex8 geometry variant):
 //   per class  A  tile assembly of H(u_s) z_s into the slot's tile partials
 //   per class  G  slot gather -> w_s = H z_s (reduced) and the shares of z.w
 //   all slots  S  the single-reduction CG step of each slot (the scalars from
@@ -66,7 +66,7 @@ __device__ __forceinline__ Dens make_density(const tatva_density &d) {
   else return Dens{float(d.p0), float(d.p1), d.elem_params};
 }
 
-template <int KIND, class Dens, bool AFFINE>
+template <int KIND, class Dens, int GEOM>
 __global__ __launch_bounds__(kTile) void k_batch_assemble(const BatchSlot *__restrict__ slots,
                                                           const int32_t *__restrict__ bmap,
                                                           QuadRule quad) {
@@ -75,9 +75,8 @@ __global__ __launch_bounds__(kTile) void k_batch_assemble(const BatchSlot *__res
   if (S.st->done) return;
   extern __shared__ unsigned char lds_raw[];
   const Dens dens = make_density<Dens>(S.dens);
-  // AFFINE: a Hex8 parallelepiped mesh (no geometry cache here)
-  tile_assemble<KIND, Dens, float, kModeHvp,
-                (AFFINE && KIND == TATVA_HEX8) ? kGeomAffine : kGeomGeneral>(
+  // (no geometry cache here)
+  tile_assemble<KIND, Dens, float, kModeHvp, GEOM>(
       b - S.a_blk0, S.coords, quad, dens, S.u, S.z, S.dof_map, S.tiles, S.partial, lds_raw);
 }
 
@@ -555,7 +554,7 @@ extern "C" int tatva_batch_start(tatva_batch *B, int32_t slot, tatva_mesh *m,
   mi.dkind = d->kind;
   mi.ncomp = ncomp;
   mi.quad = m->quad;
-  mi.affine = m->hex_affine;
+  mi.affine = m->hex_box ? kGeomBox : m->hex_affine ? kGeomAffine : kGeomGeneral;
   mi.lds = lds;
   mi.mesh = m;
   B->dirty = true;
@@ -609,9 +608,13 @@ int build_iterations(tatva_batch *B, int iters, hipGraph_t *out) {
         const int32_t *bm_g = B->d_bmap + L.g_off;
         QuadRule quad = L.quad;
         void *a_args[] = {(void *)&slots, (void *)&bm_a, (void *)&quad};
-        const void *fa = (K == TATVA_HEX8 && L.affine)
-                             ? reinterpret_cast<const void *>(&k_batch_assemble<K, Dens, true>)
-                             : reinterpret_cast<const void *>(&k_batch_assemble<K, Dens, false>);
+        const void *fa = reinterpret_cast<const void *>(&k_batch_assemble<K, Dens, kGeomGeneral>);
+        if constexpr (K == TATVA_HEX8) {
+          if (L.affine == kGeomBox)
+            fa = reinterpret_cast<const void *>(&k_batch_assemble<K, Dens, kGeomBox>);
+          else if (L.affine == kGeomAffine)
+            fa = reinterpret_cast<const void *>(&k_batch_assemble<K, Dens, kGeomAffine>);
+        }
         err = add(fa, L.a_n, kTile, L.lds, a_args);
         if (err != hipSuccess) return TATVA_OK;
         void *g_args[] = {(void *)&slots, (void *)&bm_g};

@@ -1012,14 +1012,15 @@ extern "C" int tatva_mesh_create(int device, int elem_kind, const double *coords
   }
   m->n_slots = T.node_ptr.back();
   if (elem_kind == TATVA_HEX8) {
-    bool affine = true;
+    int affine = 2;
     for (int64_t e = 0; e < n_elements && affine; ++e) {
       double X[8][3];
       for (int a = 0; a < 8; ++a)
         for (int j = 0; j < 3; ++j) X[a][j] = coords[(int64_t)elements[e * 8 + a] * 3 + j];
-      affine = hex_is_affine_host(X);
+      affine = std::min(affine, hex_affine_host(X));
     }
     m->hex_affine = affine ? 1 : 0;
+    m->hex_box = affine == 2 ? 1 : 0;
   }
   // affine Hex8: the reference element's gradient products over the quadrature
   // rule (hex8_affine_row_blocks)
@@ -1301,18 +1302,27 @@ static int launch_assembly(tatva_mesh *m, const tatva_density *d, const T *u, co
         return TATVA_EINVAL;
       }
       const int grid = tile_grid(m->tiles.n_tiles, dx.n != 0);
-      if (geo) {
-        if constexpr (kCacheable)
-          k_tile_assemble<K, Dens, T, MODE, kGeomCache><<<grid, kTile, lds, s>>>(
-              m->coords, m->quad, dens, u, v, dof_map, m->tiles, partial, skip, rev, lin, geo, dx);
-      } else if (K == TATVA_HEX8 && m->hex_affine) {
-        k_tile_assemble<K, Dens, T, MODE, kGeomAffine><<<grid, kTile, lds, s>>>(
-            m->coords, m->quad, dens, u, v, dof_map, m->tiles, partial, skip, rev, lin, nullptr,
-            dx);
+      const auto launch = [&](auto geom) {
+        constexpr int G = decltype(geom)::value;
+        k_tile_assemble<K, Dens, T, MODE, G><<<grid, kTile, lds, s>>>(
+            m->coords, m->quad, dens, u, v, dof_map, m->tiles, partial, skip, rev, lin, geo, dx);
+      };
+      using std::integral_constant;
+      if constexpr (K == TATVA_HEX8 && MODE != kModeDiag) {  // (the diagonal works nodal)
+        if (geo) {
+          if constexpr (kCacheable) {
+            if (m->hex_box) launch(integral_constant<int, kGeomBoxCache>{});
+            else launch(integral_constant<int, kGeomCache>{});
+          }
+        } else if (m->hex_box) {
+          launch(integral_constant<int, kGeomBox>{});
+        } else if (m->hex_affine) {
+          launch(integral_constant<int, kGeomAffine>{});
+        } else {
+          launch(integral_constant<int, kGeomGeneral>{});
+        }
       } else {
-        k_tile_assemble<K, Dens, T, MODE, kGeomGeneral><<<grid, kTile, lds, s>>>(
-            m->coords, m->quad, dens, u, v, dof_map, m->tiles, partial, skip, rev, lin, nullptr,
-            dx);
+        launch(integral_constant<int, kGeomGeneral>{});
       }
       if constexpr (MODE == kModeLinearize) {
         TATVA_CHECK_LAUNCH();
@@ -1359,41 +1369,53 @@ int launch_linearize_f32(tatva_mesh *m, const tatva_density *d, const float *u, 
                                                 nullptr, nullptr, 0, 0, nullptr, lin, geo);
 }
 
-// Writes the geometry cache of an affine Hex8 mesh (layout at kGeoFloats):
+// Writes the geometry cache of an affine Hex8 mesh (layout at geo_floats):
 // one thread per tile slot, its element's nodes gathered from conn.
+template <bool BOX>
 __global__ __launch_bounds__(kTile) void k_geometry_cache_hex8(const double *__restrict__ coords,
                                                                const int32_t *__restrict__ conn,
                                                                TileSet ts,
                                                                float *__restrict__ geo) {
+  constexpr int kFloats = geo_floats(BOX);
   const int tile = blockIdx.x;
   const int64_t slot = (int64_t)tile * kTile + threadIdx.x;
   const int32_t e = ts.elem[slot];
-  float *gp = geo + (int64_t)tile * kGeoFloats * kTile + threadIdx.x;
+  float *gp = geo + (int64_t)tile * kFloats * kTile + threadIdx.x;
   if (e < 0) {  // padding slot: zeros, never read
 #pragma unroll
-    for (int k = 0; k < kGeoFloats; ++k) gp[k * kTile] = 0.0f;
+    for (int k = 0; k < kFloats; ++k) gp[k * kTile] = 0.0f;
     return;
   }
   double X[8][3];
 #pragma unroll
   for (int a = 0; a < 8; ++a) {
+    if (BOX && a != 0 && a != 6) continue;
     const int64_t g = conn[(int64_t)e * 8 + a];
 #pragma unroll
     for (int k = 0; k < 3; ++k) X[a][k] = coords[g * 3 + k];
   }
-  float iv[3][3];
-  const double det = hex8_affine_inverse<float>(X, iv);
+  double det;
+  int at = 0;
+  if constexpr (BOX) {
+    float iv[3];
+    det = hex8_box_inverse<float>(X[0], X[6], iv);
 #pragma unroll
-  for (int i = 0; i < 3; ++i)
+    for (int j = 0; j < 3; ++j) gp[at++ * kTile] = iv[j];
+  } else {
+    float iv[3][3];
+    det = hex8_affine_inverse<float>(X, iv);
 #pragma unroll
-    for (int j = 0; j < 3; ++j) gp[(i * 3 + j) * kTile] = iv[i][j];
-  gp[9 * kTile] = __uint_as_float((uint32_t)__double2loint(det));
-  gp[10 * kTile] = __uint_as_float((uint32_t)__double2hiint(det));
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+      for (int j = 0; j < 3; ++j) gp[at++ * kTile] = iv[i][j];
+  }
+  gp[at * kTile] = __uint_as_float((uint32_t)__double2loint(det));
+  gp[(at + 1) * kTile] = __uint_as_float((uint32_t)__double2hiint(det));
 }
 
 int64_t geo_cache_floats(const tatva_mesh *m) {
   if (!m || m->kind != TATVA_HEX8 || !m->hex_affine) return 0;
-  return (int64_t)m->tiles.n_tiles * kTile * kGeoFloats;
+  return (int64_t)m->tiles.n_tiles * kTile * geo_floats(m->hex_box);
 }
 
 int launch_geometry_cache_f32(tatva_mesh *m, float *geo, hipStream_t s) {
@@ -1401,7 +1423,10 @@ int launch_geometry_cache_f32(tatva_mesh *m, float *geo, hipStream_t s) {
     set_error("a geometry cache needs an affine Hex8 mesh");
     return TATVA_EINVAL;
   }
-  k_geometry_cache_hex8<<<m->tiles.n_tiles, kTile, 0, s>>>(m->coords, m->conn, m->tiles, geo);
+  if (m->hex_box)
+    k_geometry_cache_hex8<true><<<m->tiles.n_tiles, kTile, 0, s>>>(m->coords, m->conn, m->tiles, geo);
+  else
+    k_geometry_cache_hex8<false><<<m->tiles.n_tiles, kTile, 0, s>>>(m->coords, m->conn, m->tiles, geo);
   TATVA_CHECK_LAUNCH();
   return TATVA_OK;
 }

@@ -28,6 +28,7 @@ struct tatva_mesh {
   double *partials;      // reduction partials, kMaxReduceBlocks * 4
   int max_incident;      // largest number of elements sharing a node
   int hex_affine;        // Hex8 mesh of parallelepipeds only (constant Jacobian per element)
+  int hex_box;           // ... of boxes along the coordinate axes (diagonal Jacobian)
   double *hex_ref;       // affine Hex8: reference gradient products (hessian.hpp), 9 x 8 x 8
   // LDS tiling (assembly.hpp)
   tatva::TileSet tiles;

@@ -130,3 +130,40 @@ def test_hessian_rows_of_many_colors(kind, shape):
     assert 1800 < mesh.n_nodes * el.dim <= 2048
     got, ref = hessian_pair(mesh, el, LE, ORACLE[LE], colors=np.arange)
     assert rel_err(got, ref) < RTOL
+
+
+def hex_variant(form, shape=(5, 7, 9)):
+    """Hex8 meshes that take each geometry variant of the tile kernels: boxes
+    along the axes, the same boxes with their local axes turned (parallelepipeds
+    whose Jacobian is a permutation), sheared boxes, and boxes of which one is
+    distorted (the whole mesh is general)."""
+    m = ta.Mesh.box(shape, lengths=(1.0, 0.7, 1.9), origin=(-0.3, 0.1, 2.0))
+    if form == "turned":
+        return ta.Mesh(m.coords, m.elements[:, [1, 2, 3, 0, 5, 6, 7, 4]])
+    if form == "sheared":
+        return m.set_coords(m.coords @ np.array([[1.0, 0.2, 0.0], [0.0, 1.0, 0.1], [0.3, 0.0, 1.0]]))
+    X = m.coords.copy()
+    if form == "general":
+        X[X.shape[0] // 2] += 0.01
+    return m.set_coords(X)
+
+
+@pytest.mark.parametrize("density", [LE, NH, PO], ids=["le", "nh", "poisson"])
+@pytest.mark.parametrize("form", ["box", "turned", "sheared", "general"])
+def test_hex8_geometry_variants(form, density):
+    """Residual and product (FP64 to 1e-12; FP32 to 2e-6 of the largest entry: some
+    tens of roundings of 6e-8) of every Hex8 geometry variant against the oracle."""
+    import torch
+
+    mesh = hex_variant(form)
+    E = ta.Operator(mesh, ta.Hexahedron8()).energy(density)
+    if form != "sheared":  # (rounding may leave a sheared box's bilinear modes nonzero)
+        assert E.op.device_layout()["hex_affine"] == (form != "general")
+    prob = fem.Problem(fem.Hex8(), mesh.coords, mesh.elements, ORACLE[density])
+    rng = np.random.default_rng(5)
+    u, v = 0.005 * rng.standard_normal(E.size), rng.standard_normal(E.size)
+    assert rel_err(to_np(E.grad(u)), prob.residual(u)) < RTOL
+    assert rel_err(to_np(E.hvp(u, v)), prob.hvp(u, v)) < RTOL
+    u32, v32 = (torch.as_tensor(a, dtype=torch.float32, device="cuda") for a in (u, v))
+    ref = prob.hvp(to_np(u32).astype(float), to_np(v32).astype(float))
+    assert rel_err(to_np(E.hvp(u32, v32)), ref) < 2e-6
