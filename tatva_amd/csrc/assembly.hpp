@@ -692,6 +692,35 @@ constexpr size_t tile_lds_bytes(int kind, int max_local, int D, int nne, int NC,
 }
 constexpr size_t kTileLdsMax = 65536;  // LDS one workgroup may allocate
 
+// Block sum of the threads' shares to *out, through the tile's own LDS (free
+// once every thread is done with it).
+__device__ __forceinline__ void tile_share(double share, unsigned char *__restrict__ lds,
+                                           double *__restrict__ out) {
+  double *red = reinterpret_cast<double *>(lds);
+  share = wave_sum(share);
+  __syncthreads();
+  if (threadIdx.x % kWave == 0) red[threadIdx.x / kWave] = share;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double s = 0.0;
+#pragma unroll
+    for (int w = 0; w < kTile / kWave; ++w) s += red[w];
+    *out = s;
+  }
+}
+
+// v at a node through the dof map (0 on a constrained dof).
+template <int NC, class T>
+__device__ __forceinline__ void tile_tangent(int64_t node, const T *__restrict__ v,
+                                             const int32_t *__restrict__ dof_map, T (&out)[NC]) {
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    const int64_t dof = node * NC + c;
+    const int64_t r = dof_map ? (int64_t)dof_map[dof] : dof;
+    out[c] = r >= 0 ? v[r] : T(0);
+  }
+}
+
 // Body of one tile (one workgroup of kTile threads; lds of tile_lds_bytes).
 // GEOM: how the elements' geometry is taken; with a cached one the FP32 HVP and
 // linearisation read it from geo instead of the node coordinates.  u: full state; v (HVP): tangent read through dof_map
@@ -699,6 +728,9 @@ constexpr size_t kTileLdsMax = 65536;  // LDS one workgroup may allocate
 // LDS once (one thread per node), so each element reads its nodes from LDS
 // instead of gathering them from global memory.  Writes the sums of local node
 // j to partial[slot_pos[node_ptr[tile] + j] * NC + c] (node-major order).
+// dot (FP32 Hex8 HVP): the tile's share of v . H v, the sums of its local nodes
+// times v there, goes to dot[tile]; summed over the tiles it is the CG's v . H v
+// without a pass over the assembled product.
 template <int KIND, class Dens, class T, int MODE, int GEOM>
 __device__ __forceinline__ void tile_assemble(int tile, const double *__restrict__ coords,
                                               const QuadRule &quad, const Dens &dens,
@@ -707,13 +739,15 @@ __device__ __forceinline__ void tile_assemble(int tile, const double *__restrict
                                               const TileSet &ts, T *__restrict__ partial,
                                               unsigned char *__restrict__ lds,
                                               T *__restrict__ lin = nullptr,
-                                              const T *__restrict__ geo = nullptr) {
+                                              const T *__restrict__ geo = nullptr,
+                                              double *__restrict__ dot = nullptr) {
   constexpr bool kUsesU = MODE != kModeHvpLin;
   constexpr bool kUsesV = MODE == kModeHvp || MODE == kModeHvpLin;
   using El = Elem<KIND>;
   constexpr int D = El::D, NNE = El::NNE, NC = Dens::NC;
   // a geometry cache (affine Hex8 HVP / linearisation) replaces the coordinates
   constexpr bool kGeo = geom_cached(GEOM);
+  constexpr bool kDot = KIND == TATVA_HEX8 && sizeof(T) == 4 && kUsesV;
   static_assert(GEOM == kGeomGeneral || KIND == TATVA_HEX8, "the geometry variants are Hex8");
   static_assert(!kGeo || (sizeof(T) == 4 && (MODE == kModeHvp || MODE == kModeHvpLin ||
                                              MODE == kModeLinearize)),
@@ -732,6 +766,8 @@ __device__ __forceinline__ void tile_assemble(int tile, const double *__restrict
   // (a constrained dof, r < 0, reads a valid dummy address and stores 0, so
   // that no load sits behind a branch).
   const T *dummy = reinterpret_cast<const T *>(coords);
+  // the tangent at this thread's first two local nodes, for the dot
+  T v01[2][NC];
   const auto stage = [&](auto mapped) {
     constexpr bool kMapped = decltype(mapped)::value;
     for (int j0 = threadIdx.x; j0 < nloc; j0 += 2 * kTile) {
@@ -762,6 +798,7 @@ __device__ __forceinline__ void tile_assemble(int tile, const double *__restrict
           for (int c = 0; c < NC; ++c) {
             const T val = *(r[h][c] >= 0 ? v + r[h][c] : dummy);
             vv[h][c] = r[h][c] >= 0 ? val : T(0);
+            if (kDot && j0 == (int)threadIdx.x) v01[h][c] = vv[h][c];
           }
       }
 #pragma unroll
@@ -877,7 +914,17 @@ __device__ __forceinline__ void tile_assemble(int tile, const double *__restrict
     __syncthreads();
     // one local node per thread, its components together: one read of each
     // incidence entry serves all NC sums (each still in ascending entry order)
+    double share = 0.0;
     for (int j = threadIdx.x; j < nloc; j += kTile) {
+      T vj[NC];  // v at the node
+      if constexpr (kDot) {
+        if (dot && j >= 2 * kTile) {
+          tile_tangent<NC, T>(ts.tnodes[nb + j], v, dof_map, vj);
+        } else {
+#pragma unroll
+          for (int c = 0; c < NC; ++c) vj[c] = j < kTile ? v01[0][c] : v01[1][c];
+        }
+      }
       const int q0 = j > 0 ? (int)ie[j - 1] : 0;
       const int q1 = ie[j];
       T sum[NC];
@@ -892,6 +939,15 @@ __device__ __forceinline__ void tile_assemble(int tile, const double *__restrict
       const int64_t pos = (int64_t)ts.slot_pos[nb + j] * NC;
 #pragma unroll
       for (int c = 0; c < NC; ++c) partial[pos + c] = sum[c];
+      if constexpr (kDot) {
+        if (dot) {
+#pragma unroll
+          for (int c = 0; c < NC; ++c) share += (double)sum[c] * (double)vj[c];
+        }
+      }
+    }
+    if constexpr (kDot) {
+      if (dot) tile_share(share, lds, dot + tile);
     }
     return;
   }
@@ -923,7 +979,8 @@ __global__ __launch_bounds__(kTile) void k_tile_assemble(const double *__restric
                                                          TileSet ts, T *__restrict__ partial,
                                                          const int *__restrict__ skip, int rev,
                                                          T *__restrict__ lin,
-                                                         const T *__restrict__ geo, CgDefer dx) {
+                                                         const T *__restrict__ geo, CgDefer dx,
+                                                         double *__restrict__ dot) {
   if (skip && *skip) return;
   extern __shared__ unsigned char lds_raw[];
   // dx (FP32 HVP): a CG step's p and x streams, run by the launch's streaming
@@ -948,7 +1005,7 @@ __global__ __launch_bounds__(kTile) void k_tile_assemble(const double *__restric
   int tile = (int)xcd_block(b, ts.n_tiles);
   if (rev) tile = ts.n_tiles - 1 - tile;
   tile_assemble<KIND, Dens, T, MODE, GEOM>(tile, coords, quad, dens, u, v, dof_map, ts, partial,
-                                           lds_raw, lin, geo);
+                                           lds_raw, lin, geo, dot);
 }
 
 // Sum of node i's tile slots (ascending tile): the tiles wrote them to the

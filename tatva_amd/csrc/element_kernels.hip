@@ -1267,6 +1267,9 @@ extern "C" int tatva_energy(tatva_mesh *m, const tatva_density *d, const double 
 namespace tatva {
 
 // Tile assembly + slot gather for one mode; out is reduced through dof_map.
+// With part_dot the shares of v . H v go there: over gather_blocks blocks of the
+// gather, or (gather_blocks 0) from the tiles, the gather being left to the
+// caller (slot sums in m->scratch; out unused).
 template <class T, int MODE>
 static int launch_assembly(tatva_mesh *m, const tatva_density *d, const T *u, const T *v,
                            const int32_t *dof_map, const double *f_ext, T *out, hipStream_t s,
@@ -1305,7 +1308,8 @@ static int launch_assembly(tatva_mesh *m, const tatva_density *d, const T *u, co
       const auto launch = [&](auto geom) {
         constexpr int G = decltype(geom)::value;
         k_tile_assemble<K, Dens, T, MODE, G><<<grid, kTile, lds, s>>>(
-            m->coords, m->quad, dens, u, v, dof_map, m->tiles, partial, skip, rev, lin, geo, dx);
+            m->coords, m->quad, dens, u, v, dof_map, m->tiles, partial, skip, rev, lin, geo, dx,
+            gather_blocks ? nullptr : part_dot);
       };
       using std::integral_constant;
       if constexpr (K == TATVA_HEX8 && MODE != kModeDiag) {  // (the diagonal works nodal)
@@ -1330,10 +1334,10 @@ static int launch_assembly(tatva_mesh *m, const tatva_density *d, const T *u, co
       }
       // optional event between the tile kernel and the gather (kernel timing)
       if (between) TATVA_TRY_HIP(hipEventRecord(between, s));
-      if (part_dot)
+      if (part_dot && gather_blocks)
         k_slot_gather_dot<NC, T><<<gather_blocks, kBlock, 0, s>>>(
             m->n_nodes, m->t_slot_ptr, partial, dof_map, v, out, part_dot, skip);
-      else
+      else if (!part_dot)
         k_slot_gather<NC, T><<<grid_for(m->n_nodes), kBlock, 0, s>>>(
             m->n_nodes, m->t_slot_ptr, partial, f_ext, dof_map, out, skip);
       TATVA_CHECK_LAUNCH();
@@ -1448,6 +1452,17 @@ int launch_hvp_dot_f32(tatva_mesh *m, const tatva_density *d, const float *u, co
                                                const_cast<float *>(lin), geo, defer);
   return launch_assembly<float, kModeHvp>(m, d, u, v, dof_map, nullptr, y, s, skip, part_dot,
                                           hvp_gather_blocks(m), rev, between, nullptr, geo, defer);
+}
+
+int launch_hvp_tiles_f32(tatva_mesh *m, const tatva_density *d, const float *u, const float *v,
+                         const int32_t *dof_map, double *part_dot, hipStream_t s, const int *skip,
+                         int rev, const float *lin, const float *geo, const CgDefer &dx) {
+  if (lin)
+    return launch_assembly<float, kModeHvpLin>(m, d, u, v, dof_map, nullptr, nullptr, s, skip,
+                                               part_dot, 0, rev, nullptr, const_cast<float *>(lin),
+                                               geo, dx);
+  return launch_assembly<float, kModeHvp>(m, d, u, v, dof_map, nullptr, nullptr, s, skip, part_dot,
+                                          0, rev, nullptr, nullptr, geo, dx);
 }
 
 }  // namespace tatva

@@ -36,17 +36,6 @@
 
 namespace tatva {
 
-// Value of the lane that a DPP control pairs with this one.
-template <int CTRL>
-__device__ __forceinline__ double dpp_f64(double v) {
-  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true);
-  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true);
-  return __hiloint2double(hi, lo);
-}
-constexpr int kDppXor1 = 0xB1;        // quad_perm [1, 0, 3, 2]
-constexpr int kDppXor2 = 0x4E;        // quad_perm [2, 3, 0, 1]
-constexpr int kDppHalfMirror = 0x141; // lane ^ 7 inside each group of 8
-
 // Lanes of one wave writing and then reading the same LDS.
 __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -214,20 +203,20 @@ __device__ __forceinline__ void hex8_row_blocks(const double *__restrict__ xs, i
       block(j, v);
       block(7 - j, send);
 #pragma unroll
-      for (int i = 0; i < NV; ++i) v[i] += dpp_f64<kDppHalfMirror>(send[i]);
+      for (int i = 0; i < NV; ++i) v[i] += dpp_move<kDppHalfMirror>(send[i]);
     };
     const auto quarter = [&](int j, double (&v)[NV]) {  // j in 0, 1
       double send[NV];
       half(j, v);
       half(j ^ 2, send);
 #pragma unroll
-      for (int i = 0; i < NV; ++i) v[i] += dpp_f64<kDppXor2>(send[i]);
+      for (int i = 0; i < NV; ++i) v[i] += dpp_move<kDppXor2>(send[i]);
     };
     double v0[NV], v1[NV];
     quarter(0, v0);
     quarter(1, v1);
 #pragma unroll
-    for (int i = 0; i < NV; ++i) out[i] += v0[i] + dpp_f64<kDppXor1>(v1[i]);
+    for (int i = 0; i < NV; ++i) out[i] += v0[i] + dpp_move<kDppXor1>(v1[i]);
   }
   if constexpr (NC > 1 && Dens::kLinear) dens.row_block(out);
 }
@@ -330,13 +319,13 @@ __device__ __forceinline__ void hex8_affine_row_blocks(const double (&X)[3], int
 #pragma unroll
   for (int c = 0; c < 3; ++c) {
     const auto diff = [](double v, double other, bool high) { return high ? v - other : other - v; };
-    const double o1 = dpp_f64<kDppXor1>(X[c]);
+    const double o1 = dpp_move<kDppXor1>(X[c]);
     const double s1 = X[c] + o1, d1 = diff(X[c], o1, b0);
-    const double os = dpp_f64<kDppXor2>(s1), od = dpp_f64<kDppXor2>(d1);
+    const double os = dpp_move<kDppXor2>(s1), od = dpp_move<kDppXor2>(d1);
     const double s12 = s1 + os, m1 = d1 + od, m2 = diff(s1, os, b1);
-    J[0][c] = 0.125 * (m1 + dpp_f64<kDppHalfMirror>(m1));
-    J[1][c] = 0.125 * (m2 + dpp_f64<kDppHalfMirror>(m2));
-    J[2][c] = 0.125 * diff(s12, dpp_f64<kDppHalfMirror>(s12), b2);
+    J[0][c] = 0.125 * (m1 + dpp_move<kDppHalfMirror>(m1));
+    J[1][c] = 0.125 * (m2 + dpp_move<kDppHalfMirror>(m2));
+    J[2][c] = 0.125 * diff(s12, dpp_move<kDppHalfMirror>(s12), b2);
   }
   const double det = det_inv(J, inv);
   if constexpr (NC == 1) {

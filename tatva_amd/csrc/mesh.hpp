@@ -84,6 +84,13 @@ int launch_hvp_dot_f32(tatva_mesh *m, const tatva_density *d, const float *u, co
                        const float *lin = nullptr, const float *geo = nullptr,
                        const CgDefer *dx = nullptr);
 int hvp_gather_blocks(const tatva_mesh *m);
+// The tile kernel of y = H(u) v (FP32) alone: the slots' sums go to m->scratch
+// (the caller's next kernel gathers them per node, slot_sum) and the tiles'
+// shares of v . y to part_dot (n_tiles, Hex8 only); rev: tiles in reverse order (same
+// result); dx: a CG step's deferred p and x update, applied by the kernel.
+int launch_hvp_tiles_f32(tatva_mesh *m, const tatva_density *d, const float *u, const float *v,
+                         const int32_t *dof_map, double *part_dot, hipStream_t s, const int *skip,
+                         int rev, const float *lin, const float *geo, const CgDefer &dx);
 int density_ncomp(const tatva_mesh *m, const tatva_density *d);
 // Drops cached solver graphs that captured this mesh's arrays.
 void forget_mesh_graphs(const tatva_mesh *m);

@@ -629,6 +629,146 @@ __global__ __launch_bounds__(kBlock) void k_cg_step(int64_t n, T *__restrict__ x
   }
 }
 
+// KB of the FP32 matrix-free form on Hex8 meshes: the step by nodes.  w = H z is
+// summed here from the tiles' slots (ascending tile) instead of by a gather
+// kernel of its own: the tile kernel's shares give w.u, so nothing needs w before
+// the scalars are known, and w is neither written nor read back.  dof_map: the
+// vectors are reduced (an index outside [0, n) is skipped), or NULL: full-length,
+// D^-1 = 0 on the dofs outside the system.
+// kDefer: as in k_cg_step.
+// A thread takes kStepNodes nodes at a time (a stride apart), loaded before the
+// scalars are summed, their slot lists walked side by side.  Four consecutive
+// nodes in 16-byte vectors measured no faster (105 against 102 us at 160^3),
+// non-temporal stores slower (124 us: a thread's 12 bytes are no whole line).
+constexpr int kStepNodes = 2;
+
+template <int NC, bool kDefer>
+__global__ __launch_bounds__(kBlock) void k_node_step(
+    int64_t n_nodes, int64_t n, const int32_t *__restrict__ slot_ptr,
+    const float *__restrict__ partial, const int32_t *__restrict__ dof_map, float *__restrict__ x,
+    float *__restrict__ r, float *__restrict__ z, float *__restrict__ p, float *__restrict__ s,
+    const float *__restrict__ dinv, const double *__restrict__ part_delta, int n_delta,
+    const double *__restrict__ part_g_old, const double *__restrict__ part_rr_old, int n_old,
+    double *__restrict__ part_g_new, double *__restrict__ part_rr_new, int q,
+    PcgState *__restrict__ st) {
+  if (st->done) return;
+  const int iter = st->it[q ^ 1];
+  constexpr int K = kStepNodes, M = K * NC;
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  struct Nodes {
+    float w[M], s[M], r[M], d[M], z[M], p[M], x[M];
+    int64_t at[M];  // -1: nothing to write
+  };
+  const auto load = [&](int64_t i, Nodes &N) {
+    int32_t b[K], len[K], longest = 0;
+    // (past the end the last node again, and nothing written)
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int64_t node = i + k * stride;
+      const int64_t g = node < n_nodes ? node : n_nodes - 1;
+      b[k] = slot_ptr[g];
+      len[k] = slot_ptr[g + 1];
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        const int64_t dof = g * NC + c;
+        const int64_t at = dof_map ? (int64_t)dof_map[dof] : dof;
+        N.at[k * NC + c] = at >= 0 && at < n ? at : -1;
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < M; ++j) {
+      const int64_t at = N.at[j] >= 0 ? N.at[j] : 0;
+      N.s[j] = s[at];
+      N.r[j] = r[at];
+      N.d[j] = dinv[at];
+      if constexpr (!kDefer) {
+        N.z[j] = z[at];
+        N.p[j] = p[at];
+        N.x[j] = x[at];
+      }
+      if (i + (j / NC) * stride >= n_nodes) N.at[j] = -1;
+      N.w[j] = 0.0f;
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      len[k] -= b[k];
+      longest = max(longest, len[k]);
+    }
+    for (int32_t j = 0; j < longest; ++j)
+#pragma unroll
+      for (int k = 0; k < K; ++k)
+        if (j < len[k]) {
+          const float *src = partial + (int64_t)(b[k] + j) * NC;
+#pragma unroll
+          for (int c = 0; c < NC; ++c) N.w[k * NC + c] += src[c];
+        }
+  };
+  const int64_t i0 = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+  Nodes pre;
+  load(i0, pre);
+  double gamma, rr, delta;
+  sum_partials3(part_g_old, n_old, part_rr_old, n_old, part_delta, n_delta, gamma, rr, delta);
+  const bool first = iter == 0;
+  const double beta = first ? 0.0 : gamma / st->gamma[q ^ 1];
+  const double denom = first ? delta : delta - beta * gamma / st->alpha[q ^ 1];
+  const bool converged = rr <= st->tol2;
+  const bool spent = iter >= st->maxiter;
+  const bool bad = !(denom > 0.0) || !isfinite(denom) || !isfinite(gamma) || !isfinite(rr);
+  if (converged || spent || bad) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      st->done = 1;
+      st->rr = rr;
+      st->iter = iter;
+      st->status = converged ? TATVA_OK : spent ? TATVA_ENOTCONV : TATVA_EBREAKDOWN;
+    }
+    return;
+  }
+  const double alpha = gamma / denom;
+  const float a = float(alpha), bt = float(beta);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    st->alpha[q] = alpha;
+    st->gamma[q] = gamma;
+    st->it[q] = iter + 1;
+    st->iter = iter + 1;
+    st->rr = rr;
+    if constexpr (kDefer) st->defer[q] = CgDeferCoef{a, bt, first ? 1 : 2, 0};
+  }
+  double sg = 0.0, srr = 0.0;
+  // the expressions of k_cg_step (p and s hold no values before iteration 0)
+  const auto update = [&](const Nodes &N) {
+#pragma unroll
+    for (int j = 0; j < M; ++j) {
+      const int64_t k = N.at[j];
+      if (k < 0) continue;
+      if constexpr (!kDefer) {
+        const float pn = first ? N.z[j] : N.z[j] + bt * N.p[j];
+        p[k] = pn;
+        x[k] = N.x[j] + a * pn;
+      }
+      const float sn = first ? N.w[j] : N.w[j] + bt * N.s[j];
+      const float rn = N.r[j] - a * sn;
+      const float zn = N.d[j] * rn;
+      s[k] = sn;
+      r[k] = rn;
+      z[k] = zn;
+      sg += (double)rn * (double)zn;
+      // D^-1 = 0 marks a dof outside the system: its r is not part of the residual
+      srr += N.d[j] != 0.0f ? (double)rn * (double)rn : 0.0;
+    }
+  };
+  update(pre);
+  for (int64_t i = i0 + K * stride; i < n_nodes; i += K * stride) {
+    Nodes N;
+    load(i, N);
+    update(N);
+  }
+  block_sum2(sg, srr);
+  if (threadIdx.x == 0) {
+    part_g_new[blockIdx.x] = sg;
+    part_rr_new[blockIdx.x] = srr;
+  }
+}
+
 // r given: z = D^-1 r, p = z, shares of r.z (into the parity-1 slot, read by
 // iteration 0 as "previous"), r.r and b.b.
 template <class T>
@@ -992,6 +1132,32 @@ __global__ __launch_bounds__(kBlock) void k_sum_shares(const double *__restrict_
   for (int i = lo + threadIdx.x; i < hi; i += kBlock) v += p[i];
   v = block_sum(v);
   if (threadIdx.x == 0) out[blockIdx.x] = v;
+}
+
+// The three sums of a step at once, each folded to kShareBlocks partials (out,
+// out + kShareBlocks, ...): with many shares a step block then sums 64 of each
+// instead of all, and the step's grid is free.
+__global__ __launch_bounds__(kBlock) void k_fold_shares(const double *__restrict__ a, int na,
+                                                       const double *__restrict__ b,
+                                                       const double *__restrict__ c, int nbc,
+                                                       double *__restrict__ out,
+                                                       const PcgState *__restrict__ st) {
+  if (st->done) return;
+  const auto part = [&](const double *p, int n) {
+    const int per = (n + kShareBlocks - 1) / kShareBlocks;
+    const int lo = blockIdx.x * per, hi = min(lo + per, n);
+    double v = 0.0;
+    for (int i = lo + threadIdx.x; i < hi; i += kBlock) v += p[i];
+    return v;
+  };
+  double va = part(a, na), vb = part(b, nbc), vc = part(c, nbc);
+  va = block_sum(va);
+  block_sum2(vb, vc);
+  if (threadIdx.x == 0) {
+    out[blockIdx.x] = va;
+    out[kShareBlocks + blockIdx.x] = vb;
+    out[2 * kShareBlocks + blockIdx.x] = vc;
+  }
 }
 
 // Typed views of a workspace; base is the workspace's first byte.
@@ -1392,16 +1558,27 @@ int matfree_pcg_setup(tatva_mesh *m, const tatva_density *d, const float *u,
 // and the affine Hex8 geometry (each 0 bytes when not selected)
 constexpr int kMatfreeVecs = 10;
 
+// Shares that a step's blocks sum themselves.
+constexpr int kStepShares = 2048;
+static int64_t vec_blocks(int64_t n, int per_thread) {
+  const int64_t per_block = (int64_t)kBlock * per_thread;
+  return (n + per_block - 1) / per_block;
+}
+
 // Length of the CG vectors the workspace is sized for: with full-length
 // vectors the larger of n and the full dof count.
 static int64_t matfree_vec_len(const tatva_mesh *m, const tatva_density *d, int64_t n) {
   return g_full_vectors.load() == 1 ? std::max<int64_t>(n, m->n_nodes * density_ncomp(m, d)) : n;
 }
 
-static size_t matfree_u_offset(int64_t n) { return ws_layout(n, kMatfreeVecs, sizeof(float)).total; }
+// (the workspace also holds the tiles' shares of z.w)
+static WsLayout matfree_layout(const tatva_mesh *m, int64_t n) {
+  return ws_layout(n, kMatfreeVecs, sizeof(float), m->tiles.n_tiles);
+}
+static size_t matfree_u_offset(const tatva_mesh *m, int64_t n) { return matfree_layout(m, n).total; }
 
 static size_t matfree_lin_offset(const tatva_mesh *m, int64_t n) {
-  return matfree_u_offset(n) + align256((size_t)(m->n_nodes * m->dim) * sizeof(float));
+  return matfree_u_offset(m, n) + align256((size_t)(m->n_nodes * m->dim) * sizeof(float));
 }
 
 // Bytes of the two caches under the current options.
@@ -1438,7 +1615,7 @@ extern "C" int tatva_pcg_matfree_f32(tatva_mesh *m, const tatva_density *d, cons
   const bool full = dof_map && g_full_vectors.load() == 1;
   const int64_t nv = full ? n_full : n;
   const int32_t *op_map = full ? nullptr : dof_map;
-  const WsLayout L = ws_layout(nv, kMatfreeVecs, sizeof(float));
+  const WsLayout L = matfree_layout(m, nv);
   chunk += chunk & 1;
   TATVA_TRY_HIP(hipSetDevice(m->device));
   DeviceRes *res = nullptr;
@@ -1456,7 +1633,7 @@ extern "C" int tatva_pcg_matfree_f32(tatva_mesh *m, const tatva_density *d, cons
   float *b = ws_vec<float>(wsb, L, 7);
   float *diag = ws_vec<float>(wsb, L, 8);
   float *z2 = ws_vec<float>(wsb, L, 9);
-  float *u = reinterpret_cast<float *>(wsb + matfree_u_offset(nv));
+  float *u = reinterpret_cast<float *>(wsb + matfree_u_offset(m, nv));
   // the state is fixed during the solve: the density may be linearised once and
   // read back by every product (option; off by default: on the 160^3 Hex8 cube
   // the product reading 40 bytes per point ran at 515 us against 433 us for the
@@ -1488,7 +1665,20 @@ extern "C" int tatva_pcg_matfree_f32(tatva_mesh *m, const tatva_density *d, cons
   // (full-length: the reduced diagonal is copied as is and read through the map)
   TATVA_TRY_HIP(hipMemcpyAsync(diag, diag_in, n * sizeof(float), hipMemcpyDeviceToDevice, s));
   TATVA_TRY_HIP(hipMemcpyAsync(u, u_in, n_full * sizeof(float), hipMemcpyDeviceToDevice, s));
-  const int gv = step_grid(nv, step_prefetch<float>());
+  const int nc = density_ncomp(m, d);
+  // Hex8: the step gathers the product by nodes (k_node_step) and the tiles give
+  // the shares of z.w.  With many of those every block of a step would sum them
+  // all, so they and the step's own are folded first (a launch of its own), and
+  // the step's grid is as large as its share buffers.  Other elements: a gather
+  // kernel with the dot, then the step (a Tet4 tile's work is so short that its
+  // share cost more than the pass saved: 64^3 x 6 tiles 32.0 -> 37.4 us, gather
+  // and step 15.9 -> 14.4 us).
+  const bool by_node = m->kind == TATVA_HEX8;
+  const int n_shares = m->tiles.n_tiles;
+  const bool fold = by_node && n_shares > kStepShares;
+  const int gv = !by_node ? step_grid(nv, step_prefetch<float>())
+                 : fold   ? (int)std::min<int64_t>(kMaxReduceBlocks, vec_blocks(m->n_nodes, kStepNodes))
+                          : step_grid(m->n_nodes, kStepNodes);
   const bool profiling = g_profiling.load() != 0;
   // r = b - H x, z = D^-1 r, shares of r.z, r.r, b.b (w is scratch here)
   if (geo) {
@@ -1502,7 +1692,6 @@ extern "C" int tatva_pcg_matfree_f32(tatva_mesh *m, const tatva_density *d, cons
   rc = matfree_pcg_setup(m, d, u, op_map, nv, diag, b, x, r, z, w, dinv, P.rz(1), P.rr(1), P.bb,
                          gv, tol, maxiter, st, s, lin, geo, full ? dof_map : nullptr, n);
   if (rc) return rc;
-  const int g_op = hvp_gather_blocks(m);
   // deferred p and x (option, on by default): iteration i's z sits in zb[i % 2];
   // the step of iteration i writes z_{i+1} to the other buffer and leaves
   // p_i = z_i + beta p_{i-1}, x_{i+1} = x_i + alpha p_i to the tile kernel of
@@ -1510,26 +1699,59 @@ extern "C" int tatva_pcg_matfree_f32(tatva_mesh *m, const tatva_density *d, cons
   // iteration i + 1 overwrites it.  The solve is the same bits either way.
   const bool defer = g_cg_defer.load() == 1;
   float *const zb[2] = {z, defer ? z2 : z};
-  // KA: w = H z with the shares of z.w; the tiles run in alternating order
-  // (iteration parity), as the CSR SpMV streams its matrix
+  // KA: w = H z with the shares of z.w (Hex8: the slot sums of w and the tiles'
+  // shares); the tiles run in alternating order (iteration parity), as the CSR
+  // SpMV streams its matrix
+  const int g_op = hvp_gather_blocks(m);
+  double *shares = by_node ? reinterpret_cast<double *>(wsb + L.op_parts) : P.pap;
   const auto op = [&](int q, hipEvent_t between) -> int {
     const CgDefer dx{zb[q ^ 1], p, x, &st->defer[q ^ 1], defer ? nv : 0};
-    return launch_hvp_dot_f32(m, d, u, zb[q], op_map, w, P.pap, s, &st->done, q, between, lin,
+    if (by_node) {
+      const int e = launch_hvp_tiles_f32(m, d, u, zb[q], op_map, shares, s, &st->done, q, lin, geo, dx);
+      if (e) return e;
+      if (between) TATVA_TRY_HIP(hipEventRecord(between, s));
+      if (fold)
+        k_fold_shares<<<kShareBlocks, kBlock, 0, s>>>(shares, n_shares, P.rz(q ^ 1), P.rr(q ^ 1), gv,
+                                                      P.pap, st);
+      TATVA_CHECK_LAUNCH();
+      return TATVA_OK;
+    }
+    return launch_hvp_dot_f32(m, d, u, zb[q], op_map, w, shares, s, &st->done, q, between, lin,
                               geo, &dx);
   };
   // the sampled operator also times its tile kernel alone (prof_a to prof_m)
   const std::function<int()> sampled_op = [&]() -> int { return op(0, res->prof_m); };
+  const auto node_step = [&](int q) {
+    const auto launch = [&](auto ncc, auto deferred) {
+      constexpr int NC = decltype(ncc)::value;
+      constexpr bool kDefer = decltype(deferred)::value;
+      k_node_step<NC, kDefer><<<gv, kBlock, 0, s>>>(
+          m->n_nodes, nv, m->t_slot_ptr, (const float *)m->scratch, op_map, kDefer ? nullptr : x, r,
+          zb[q ^ 1], kDefer ? nullptr : p, sv, dinv, fold ? P.pap : shares,
+          fold ? kShareBlocks : n_shares, fold ? P.pap + kShareBlocks : P.rz(q ^ 1),
+          fold ? P.pap + 2 * kShareBlocks : P.rr(q ^ 1), fold ? kShareBlocks : gv, P.rz(q), P.rr(q),
+          q, st);
+    };
+    const auto with_nc = [&](auto deferred) {
+      if (density_ncomp(m, d) == 1) launch(std::integral_constant<int, 1>{}, deferred);
+      else launch(std::integral_constant<int, 3>{}, deferred);
+    };
+    if (defer) with_nc(std::true_type{});
+    else with_nc(std::false_type{});
+  };
   const std::function<int(int, bool)> step = [&](int q, bool with_op) -> int {
     if (with_op) {
       const int e = op(q, nullptr);
       if (e) return e;
     }
-    if (defer)
+    if (by_node)
+      node_step(q);
+    else if (defer)
       k_cg_step<float, true><<<gv, kBlock, 0, s>>>(nv, nullptr, r, zb[q ^ 1], nullptr, sv, w, dinv,
-                                                   P.pap, g_op, P.rz(q ^ 1), P.rr(q ^ 1), P.rz(q),
+                                                   shares, g_op, P.rz(q ^ 1), P.rr(q ^ 1), P.rz(q),
                                                    P.rr(q), q, st);
     else
-      k_cg_step<float><<<gv, kBlock, 0, s>>>(nv, x, r, z, p, sv, w, dinv, P.pap, g_op, P.rz(q ^ 1),
+      k_cg_step<float><<<gv, kBlock, 0, s>>>(nv, x, r, z, p, sv, w, dinv, shares, g_op, P.rz(q ^ 1),
                                              P.rr(q ^ 1), P.rz(q), P.rr(q), q, st);
     return TATVA_OK;
   };
@@ -1615,7 +1837,7 @@ __global__ __launch_bounds__(kBlock) void k_reduce_rows_dot_f32(int64_t n, const
 extern "C" int64_t tatva_pcg_matfree_mapped_workspace(tatva_mesh *m, int64_t n) {
   if (!m || n <= 0) return -1;
   const int64_t n_full = m->n_nodes * m->dim;
-  return (int64_t)(matfree_u_offset(n) + 3 * align256((size_t)n_full * sizeof(float)));
+  return (int64_t)(matfree_u_offset(m, n) + 3 * align256((size_t)n_full * sizeof(float)));
 }
 
 extern "C" int tatva_pcg_matfree_f32_mapped(tatva_mesh *m, const tatva_density *d, const float *u_in,
@@ -1629,7 +1851,7 @@ extern "C" int tatva_pcg_matfree_f32_mapped(tatva_mesh *m, const tatva_density *
                     n > 0,
                 "invalid arguments");
   TATVA_REQUIRE(chunk >= 1 && chunk <= 4096, "chunk must be in [1, 4096]");
-  const WsLayout L = ws_layout(n, kMatfreeVecs, sizeof(float));
+  const WsLayout L = matfree_layout(m, n);
   TATVA_REQUIRE(((uintptr_t)workspace & 255) == 0, "PCG workspace must be 256-byte aligned");
   TATVA_REQUIRE(workspace && ws_bytes >= tatva_pcg_matfree_mapped_workspace(m, n),
                 "PCG workspace too small");
@@ -1651,9 +1873,9 @@ extern "C" int tatva_pcg_matfree_f32_mapped(tatva_mesh *m, const tatva_density *
   float *b = ws_vec<float>(wsb, L, 7);
   float *diag = ws_vec<float>(wsb, L, 8);
   const size_t full_bytes = align256((size_t)m->n_nodes * m->dim * sizeof(float));
-  float *u = reinterpret_cast<float *>(wsb + matfree_u_offset(n));
-  float *v_full = reinterpret_cast<float *>(wsb + matfree_u_offset(n) + full_bytes);
-  float *y_full = reinterpret_cast<float *>(wsb + matfree_u_offset(n) + 2 * full_bytes);
+  float *u = reinterpret_cast<float *>(wsb + matfree_u_offset(m, n));
+  float *v_full = reinterpret_cast<float *>(wsb + matfree_u_offset(m, n) + full_bytes);
+  float *y_full = reinterpret_cast<float *>(wsb + matfree_u_offset(m, n) + 2 * full_bytes);
   const PcgParts P = parts_at(wsb, L);
   PcgState *st = ws_state(wsb, L);
   hipStream_t caller = (hipStream_t)stream;

@@ -167,3 +167,43 @@ def test_hex8_geometry_variants(form, density):
     u32, v32 = (torch.as_tensor(a, dtype=torch.float32, device="cuda") for a in (u, v))
     ref = prob.hvp(to_np(u32).astype(float), to_np(v32).astype(float))
     assert rel_err(to_np(E.hvp(u32, v32)), ref) < 2e-6
+
+
+@pytest.mark.parametrize("full", [True, False])
+@pytest.mark.parametrize("shape,density", [((6, 5, 4), LE), ((9, 7, 5), PO), ((82, 81, 80), PO),
+                                           ((82, 81, 80), LE)],
+                         ids=["le-small", "poisson-small", "poisson-folded", "le-folded"])
+def test_matfree_pcg_step_by_nodes(shape, density, full):
+    """Hex8 FP32 PCG whose step gathers the product by nodes: one and three
+    components, full-length and reduced vectors, few and more than 2048 tiles
+    (their shares folded first), deferred updates on and off (the same bits).
+    Stopped at a recurrence residual of 1e-4; the true FP64 residual may differ
+    from it by FP32 rounding over the iterations (some 1e2 of 6e-8 relative to
+    b, so 2e-4 bounds the sum)."""
+    import torch
+
+    from tatva_amd import solvers
+
+    mesh = ta.Mesh.box(shape)
+    E = ta.Operator(mesh, ta.Hexahedron8()).energy(density)
+    x0 = np.where(mesh.coords[:, 0] == 0.0)[0]
+    nc = density.ncomp(3)
+    L = lifter.Lifter(E.size, lifter.Fixed((x0[:, None] * nc + np.arange(nc)).ravel(), 0.0))
+    red = E.reduced(L)
+    u = torch.zeros(E.size, dtype=torch.float32, device="cuda")
+    g = torch.Generator(device="cuda").manual_seed(3)
+    b = torch.randn(red.size, dtype=torch.float32, device="cuda", generator=g)
+    out = []
+    solvers.set_full_vectors(full)
+    try:
+        for defer in (True, False):
+            solvers.set_deferred_update(defer)
+            x, info = solvers.pcg_matfree(red, u, b, tol=1e-4)
+            assert info.converged
+            out.append((info.iterations, x))
+    finally:
+        solvers.set_deferred_update(True)   # the defaults
+        solvers.set_full_vectors(True)
+    assert out[0][0] == out[1][0] and torch.equal(out[0][1], out[1][1])
+    r = b.double() - red.hvp_full_state(u.double(), out[0][1].double())
+    assert float(r.norm() / b.double().norm()) < 2e-4
