@@ -728,10 +728,10 @@ __device__ __forceinline__ void tile_tangent(int64_t node, const T *__restrict__
 // LDS once (one thread per node), so each element reads its nodes from LDS
 // instead of gathering them from global memory.  Writes the sums of local node
 // j to partial[slot_pos[node_ptr[tile] + j] * NC + c] (node-major order).
-// dot (FP32 Hex8 HVP): the tile's share of v . H v, the sums of its local nodes
-// times v there, goes to dot[tile]; summed over the tiles it is the CG's v . H v
-// without a pass over the assembled product.
-template <int KIND, class Dens, class T, int MODE, int GEOM>
+// DOT, dot (HVP): the tile's share of v . H v, the sums of its local nodes times
+// v there, goes to dot[tile]; summed over the tiles it is the CG's v . H v without
+// a pass over the assembled product.
+template <int KIND, class Dens, class T, int MODE, int GEOM, bool DOT = false>
 __device__ __forceinline__ void tile_assemble(int tile, const double *__restrict__ coords,
                                               const QuadRule &quad, const Dens &dens,
                                               const T *__restrict__ u, const T *__restrict__ v,
@@ -747,7 +747,7 @@ __device__ __forceinline__ void tile_assemble(int tile, const double *__restrict
   constexpr int D = El::D, NNE = El::NNE, NC = Dens::NC;
   // a geometry cache (affine Hex8 HVP / linearisation) replaces the coordinates
   constexpr bool kGeo = geom_cached(GEOM);
-  constexpr bool kDot = KIND == TATVA_HEX8 && sizeof(T) == 4 && kUsesV;
+  constexpr bool kDot = DOT && kUsesV;
   static_assert(GEOM == kGeomGeneral || KIND == TATVA_HEX8, "the geometry variants are Hex8");
   static_assert(!kGeo || (sizeof(T) == 4 && (MODE == kModeHvp || MODE == kModeHvpLin ||
                                              MODE == kModeLinearize)),
@@ -964,9 +964,14 @@ __device__ __forceinline__ void tile_assemble(int tile, const double *__restrict
     }
     __syncthreads();
   }
+  double share = 0.0;
   for (int i = threadIdx.x; i < nloc * NC; i += kTile) {
     const int j = i / NC;
     partial[(int64_t)ts.slot_pos[nb + j] * NC + (i - j * NC)] = acc[i];
+    if constexpr (kDot) share += (double)acc[i] * (double)vs[i];
+  }
+  if constexpr (kDot) {
+    if (dot) tile_share(share, lds, dot + tile);
   }
 }
 
@@ -1004,8 +1009,9 @@ __global__ __launch_bounds__(kTile) void k_tile_assemble(const double *__restric
   // previous one; every tile writes its own slots, so the result is the same)
   int tile = (int)xcd_block(b, ts.n_tiles);
   if (rev) tile = ts.n_tiles - 1 - tile;
-  tile_assemble<KIND, Dens, T, MODE, GEOM>(tile, coords, quad, dens, u, v, dof_map, ts, partial,
-                                           lds_raw, lin, geo, dot);
+  constexpr bool kDot = KIND == TATVA_HEX8 && sizeof(T) == 4;
+  tile_assemble<KIND, Dens, T, MODE, GEOM, kDot>(tile, coords, quad, dens, u, v, dof_map, ts,
+                                                 partial, lds_raw, lin, geo, dot);
 }
 
 // Sum of node i's tile slots (ascending tile): the tiles wrote them to the

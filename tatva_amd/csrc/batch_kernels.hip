@@ -4,11 +4,15 @@
 // share the launches instead of queueing behind each other.
 //
 // Per iteration (tick t), with one class = slots of equal (element kind,
-// density kind, quadrature rule, Hex8 geometry variant):
-//   per class  A  tile assembly of H(u_s) z_s into the slot's tile partials
-//   per class  G  slot gather -> w_s = H z_s (reduced) and the shares of z.w
-//   all slots  S  the single-reduction CG step of each slot (the scalars from
-//                 its partials, p, s, x, r, z updates, shares of r.z and r.r)
+// quadrature rule, Hex8 geometry variant), whatever their densities:
+//   per class  A  tile assembly of H(u_s) z_s into the slot's tile partials and
+//                 the tiles' shares of z.w
+//   all slots  S  the single-reduction CG step of each slot by nodes (w_s = H z_s
+//                 gathered from the tiles, the scalars from its partials, p, s, x,
+//                 r, z updates, shares of r.z and r.r)
+// (A launch per density and a gather launch of its own per class ran the mixed
+// stream of linear elastic and Neo-Hookean cubes in five launches an iteration,
+// 44 us of kernels at six requests of 8^3 to 40^3; now two, 23.5 us.)
 // with the recurrences of the single-solve PCG (solver_kernels.hip).  A block
 // finds its slot through a per-block table (one load) and works on that
 // slot's arrays only; the slot's own blocks re-sum its partials across the
@@ -34,14 +38,6 @@
 
 namespace tatva {
 
-// Gather blocks of one slot: grid-stride over nodes beyond kMaxReduceBlocks.
-inline int gather_grid(int64_t n_nodes) {
-  int64_t b = (n_nodes + kBlock - 1) / kBlock;
-  if (b < 1) b = 1;
-  if (b > kMaxReduceBlocks) b = kMaxReduceBlocks;
-  return (int)b;
-}
-
 struct BatchSlot {
   const double *coords;
   const int32_t *conn;
@@ -56,8 +52,9 @@ struct BatchSlot {
   double *pap, *rz0, *rz1, *rr0, *rr1, *bb;
   PcgState *st;
   int64_t start_tick;  // batch tick of the slot's first iteration
-  int32_t g_blocks, v_blocks;
-  int32_t a_blk0, g_blk0, v_blk0;
+  int32_t ncomp;
+  int32_t v_blocks;
+  int32_t a_blk0, v_blk0;
 };
 
 template <class Dens>
@@ -66,7 +63,16 @@ __device__ __forceinline__ Dens make_density(const tatva_density &d) {
   else return Dens{float(d.p0), float(d.p1), d.elem_params};
 }
 
-template <int KIND, class Dens, int GEOM>
+template <int KIND, int GEOM, class Dens>
+__device__ __forceinline__ void batch_tile(const BatchSlot &S, int tile, const QuadRule &quad,
+                                           unsigned char *__restrict__ lds) {
+  // (no geometry cache here)
+  tile_assemble<KIND, Dens, float, kModeHvp, GEOM, true>(
+      tile, S.coords, quad, make_density<Dens>(S.dens), S.u, S.z, S.dof_map, S.tiles, S.partial,
+      lds, nullptr, nullptr, S.pap);
+}
+
+template <int KIND, int GEOM>
 __global__ __launch_bounds__(kTile) void k_batch_assemble(const BatchSlot *__restrict__ slots,
                                                           const int32_t *__restrict__ bmap,
                                                           QuadRule quad) {
@@ -74,47 +80,21 @@ __global__ __launch_bounds__(kTile) void k_batch_assemble(const BatchSlot *__res
   const BatchSlot &S = slots[bmap[b]];
   if (S.st->done) return;
   extern __shared__ unsigned char lds_raw[];
-  const Dens dens = make_density<Dens>(S.dens);
-  // (no geometry cache here)
-  tile_assemble<KIND, Dens, float, kModeHvp, GEOM>(
-      b - S.a_blk0, S.coords, quad, dens, S.u, S.z, S.dof_map, S.tiles, S.partial, lds_raw);
-}
-
-template <int NC>
-__global__ __launch_bounds__(kBlock) void k_batch_gather(const BatchSlot *__restrict__ slots,
-                                                         const int32_t *__restrict__ bmap) {
-  const int b = (int)xcd_block(blockIdx.x, gridDim.x);
-  const BatchSlot &S = slots[bmap[b]];
-  if (S.st->done) return;
-  const int lb = b - S.g_blk0;
-  const int32_t *__restrict__ dof_map = S.dof_map;
-  const float *__restrict__ z = S.z;
-  float *__restrict__ w = S.w;
-  double dot = 0.0;
-  for (int64_t i = (int64_t)lb * kBlock + threadIdx.x; i < S.n_nodes;
-       i += (int64_t)S.g_blocks * kBlock) {
-    float acc[NC];
-    slot_sum<NC, float>(i, S.tiles.slot_ptr, S.partial, acc);
-#pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      const int64_t dof = i * NC + c;
-      const int64_t r = dof_map ? (int64_t)dof_map[dof] : dof;
-      if (r >= 0) {
-        w[r] = acc[c];
-        dot += (double)acc[c] * (double)z[r];
-      }
-    }
+  constexpr int D = Elem<KIND>::D;
+  const int tile = b - S.a_blk0;
+  // (the slot, and so its density, is the same for the whole block)
+  switch (S.dens.kind) {
+    case TATVA_DENSITY_POISSON: batch_tile<KIND, GEOM, Poisson<D, float>>(S, tile, quad, lds_raw); break;
+    case TATVA_DENSITY_LINEAR_ELASTIC:
+      batch_tile<KIND, GEOM, LinearElastic<D, float>>(S, tile, quad, lds_raw);
+      break;
+    default: batch_tile<KIND, GEOM, NeoHookean<D, float>>(S, tile, quad, lds_raw); break;
   }
-  dot = block_sum(dot);
-  if (threadIdx.x == 0) S.pap[lb] = dot;
 }
 
 // Iteration k of a batch launch sequence runs at batch tick *tick + k (the
 // tick advances by the sequence length at its end, k_batch_tick), so the
 // graph of a sequence replays with no per-launch arguments.
-// Elements per thread the batched CG step loads before its share sums.
-constexpr int kBatchPrefetch = 4;
-
 __global__ __launch_bounds__(kBlock) void k_batch_step(const BatchSlot *__restrict__ slots,
                                                        const int32_t *__restrict__ bmap,
                                                        const int64_t *__restrict__ tick, int k) {
@@ -124,97 +104,15 @@ __global__ __launch_bounds__(kBlock) void k_batch_step(const BatchSlot *__restri
   if (st->done) return;
   const int lb = blk - S.v_blk0;
   const int q = (int)((*tick + k - S.start_tick) & 1);
-  const int iter = st->it[q ^ 1];
-  float *__restrict__ x = S.x;
-  float *__restrict__ r = S.r;
-  float *__restrict__ z = S.z;
-  float *__restrict__ p = S.p;
-  float *__restrict__ s = S.s;
-  const float *__restrict__ w = S.w;
-  const float *__restrict__ dinv = S.dinv;
-  // the first kBatchPrefetch elements of this thread are loaded before the
-  // shares are summed, so their latency overlaps the sums (p and s hold no
-  // values before iteration 0: selected away below, never scaled)
-  const int64_t stride = (int64_t)S.v_blocks * kBlock;
-  const int64_t i0 = (int64_t)lb * kBlock + threadIdx.x;
-  float rz[kBatchPrefetch], rp[kBatchPrefetch], rw[kBatchPrefetch], rs[kBatchPrefetch];
-  float rx[kBatchPrefetch], rv[kBatchPrefetch], rd[kBatchPrefetch];
-#pragma unroll
-  for (int j = 0; j < kBatchPrefetch; ++j) {
-    const int64_t i = i0 + j * stride;
-    if (i < S.n) {
-      rz[j] = z[i];
-      rp[j] = p[i];
-      rw[j] = w[i];
-      rs[j] = s[i];
-      rx[j] = x[i];
-      rv[j] = r[i];
-      rd[j] = dinv[i];
-    }
-  }
-  double gamma, rr, delta;
-  sum_partials3(q ? S.rz0 : S.rz1, S.v_blocks, q ? S.rr0 : S.rr1, S.v_blocks, S.pap, S.g_blocks,
-                gamma, rr, delta);
-  const bool first = iter == 0;
-  const double beta = first ? 0.0 : gamma / st->gamma[q ^ 1];
-  const double denom = first ? delta : delta - beta * gamma / st->alpha[q ^ 1];
-  const bool converged = rr <= st->tol2;
-  const bool spent = iter >= st->maxiter;
-  const bool bad = !(denom > 0.0) || !isfinite(denom) || !isfinite(gamma) || !isfinite(rr);
-  if (converged || spent || bad) {
-    if (lb == 0 && threadIdx.x == 0) {
-      st->done = 1;
-      st->rr = rr;
-      st->iter = iter;
-      st->status = converged ? TATVA_OK : spent ? TATVA_ENOTCONV : TATVA_EBREAKDOWN;
-    }
-    return;
-  }
-  const double alpha = gamma / denom;
-  if (lb == 0 && threadIdx.x == 0) {
-    st->alpha[q] = alpha;
-    st->gamma[q] = gamma;
-    st->it[q] = iter + 1;
-    st->iter = iter + 1;
-    st->rr = rr;
-  }
-  const float a = float(alpha), bt = float(beta);
-  double sg = 0.0, srr = 0.0;
-#pragma unroll
-  for (int j = 0; j < kBatchPrefetch; ++j) {
-    const int64_t i = i0 + j * stride;
-    if (i < S.n) {
-      const float pi = first ? rz[j] : rz[j] + bt * rp[j];
-      const float si = first ? rw[j] : rw[j] + bt * rs[j];
-      p[i] = pi;
-      s[i] = si;
-      x[i] = rx[j] + a * pi;
-      const float ri = rv[j] - a * si;
-      r[i] = ri;
-      const float zi = rd[j] * ri;
-      z[i] = zi;
-      sg += (double)ri * (double)zi;
-      srr += (double)ri * (double)ri;
-    }
-  }
-  for (int64_t i = i0 + kBatchPrefetch * stride; i < S.n; i += stride) {
-    const float pi = first ? z[i] : z[i] + bt * p[i];
-    const float si = first ? w[i] : w[i] + bt * s[i];
-    p[i] = pi;
-    s[i] = si;
-    x[i] += a * pi;
-    const float ri = r[i] - a * si;
-    r[i] = ri;
-    const float zi = dinv[i] * ri;
-    z[i] = zi;
-    sg += (double)ri * (double)zi;
-    srr += (double)ri * (double)ri;
-  }
-  block_sum2(sg, srr);
-  if (threadIdx.x == 0) {
-    (q ? S.rz1 : S.rz0)[lb] = sg;
-    (q ? S.rr1 : S.rr0)[lb] = srr;
-  }
+  const auto step = [&](auto ncc) {
+    node_step<decltype(ncc)::value, false>(
+        lb, S.v_blocks, S.n_nodes, S.n, S.tiles.slot_ptr, S.partial, S.dof_map, S.x, S.r, S.z, S.p,
+        S.s, S.dinv, S.pap, S.tiles.n_tiles, q ? S.rz0 : S.rz1, q ? S.rr0 : S.rr1, S.v_blocks,
+        q ? S.rz1 : S.rz0, q ? S.rr1 : S.rr0, q, st);
+  };
+  if (S.ncomp == 3) step(std::integral_constant<int, 3>{});
+  else if (S.ncomp == 2) step(std::integral_constant<int, 2>{});
+  else step(std::integral_constant<int, 1>{});
 }
 
 __global__ void k_batch_tick(int64_t *__restrict__ tick, int iters) {
@@ -222,8 +120,8 @@ __global__ void k_batch_tick(int64_t *__restrict__ tick, int iters) {
 }
 
 // Per-slot workspace: z, p, s, w, r, dinv (n floats each), tile partials
-// (n_slots * ncomp floats), the partial sums pap (gather blocks) and
-// rz0/rz1/rr0/rr1/bb (vector blocks).
+// (n_slots * ncomp floats), the partial sums pap (tiles) and
+// rz0/rz1/rr0/rr1/bb (step blocks).
 struct SlotLayout {
   size_t z, p, s, w, r, dinv, partial, pap, rz0, rz1, rr0, rr1, bb, total;
 };
@@ -245,8 +143,8 @@ static SlotLayout slot_layout(const tatva_mesh *m, int ncomp, int64_t n) {
   L.r = take(n * sizeof(float));
   L.dinv = take(n * sizeof(float));
   L.partial = take((size_t)std::max<int64_t>(1, m->n_slots) * ncomp * sizeof(float));
-  L.pap = take(gather_grid(m->n_nodes) * sizeof(double));
-  const size_t vb = step_grid(n, kBatchPrefetch) * sizeof(double);
+  L.pap = take((size_t)m->tiles.n_tiles * sizeof(double));
+  const size_t vb = step_grid(m->n_nodes, kStepNodes) * sizeof(double);
   L.rz0 = take(vb);
   L.rz1 = take(vb);
   L.rr0 = take(vb);
@@ -263,16 +161,16 @@ using namespace tatva;
 struct tatva_batch {
   struct Meta {
     bool active = false;
-    int kind = 0, dkind = 0, ncomp = 0, affine = 0;
+    int kind = 0, affine = 0;  // affine: the Hex8 geometry variant
     QuadRule quad{};
     size_t lds = 0;
     tatva_mesh *mesh = nullptr;
   };
   struct Launch {
-    int kind, dkind, ncomp, affine;
+    int kind, affine;
     QuadRule quad;
     size_t lds;
-    int a_off, a_n, g_off, g_n;
+    int a_off, a_n;
   };
   int device = 0;
   int capacity = 0;
@@ -320,6 +218,10 @@ bool same_quad(const QuadRule &a, const QuadRule &b) {
   return std::memcmp(&a, &b, sizeof(QuadRule)) == 0;
 }
 
+bool same_class(const tatva_batch::Launch &L, const tatva_batch::Meta &mi) {
+  return L.kind == mi.kind && L.affine == mi.affine && same_quad(L.quad, mi.quad);
+}
+
 // Re-plans the launches over the active slots and uploads the slot table and
 // the block map (pinned staging; the previous upload must have completed
 // before the staging is rewritten).
@@ -337,35 +239,20 @@ int batch_upload(tatva_batch *B, hipStream_t s) {
     if (!mi.active) continue;
     bool found = false;
     for (auto &L : B->launches)
-      if (L.kind == mi.kind && L.dkind == mi.dkind && L.affine == mi.affine &&
-          same_quad(L.quad, mi.quad))
-        found = true;
+      if (same_class(L, mi)) found = true;
     if (found) continue;
-    tatva_batch::Launch L{mi.kind, mi.dkind, mi.ncomp, mi.affine, mi.quad, 0, 0, 0, 0, 0};
-    B->launches.push_back(L);
+    B->launches.push_back(tatva_batch::Launch{mi.kind, mi.affine, mi.quad, 0, 0, 0});
   }
   for (auto &L : B->launches) {
     L.a_off = (int)bmap.size();
     for (int i = 0; i < B->capacity; ++i) {
       const auto &mi = B->meta[i];
-      if (!mi.active || mi.kind != L.kind || mi.dkind != L.dkind || mi.affine != L.affine ||
-          !same_quad(mi.quad, L.quad))
-        continue;
+      if (!mi.active || !same_class(L, mi)) continue;
       B->slots[i].a_blk0 = (int32_t)bmap.size() - L.a_off;
       bmap.insert(bmap.end(), B->slots[i].tiles.n_tiles, i);
       L.lds = std::max(L.lds, mi.lds);
     }
     L.a_n = (int)bmap.size() - L.a_off;
-    L.g_off = (int)bmap.size();
-    for (int i = 0; i < B->capacity; ++i) {
-      const auto &mi = B->meta[i];
-      if (!mi.active || mi.kind != L.kind || mi.dkind != L.dkind || mi.affine != L.affine ||
-          !same_quad(mi.quad, L.quad))
-        continue;
-      B->slots[i].g_blk0 = (int32_t)bmap.size() - L.g_off;
-      bmap.insert(bmap.end(), B->slots[i].g_blocks, i);
-    }
-    L.g_n = (int)bmap.size() - L.g_off;
   }
   B->v_off = (int)bmap.size();
   for (int i = 0; i < B->capacity; ++i) {
@@ -405,21 +292,11 @@ int batch_upload(tatva_batch *B, hipStream_t s) {
 }
 
 template <class F>
-int with_class(int kind, int dkind, F &&f) {
-  auto dens = [&](auto kc) -> int {
-    constexpr int K = decltype(kc)::value;
-    constexpr int D = Elem<K>::D;
-    switch (dkind) {
-      case TATVA_DENSITY_POISSON: return f(kc, Poisson<D, float>{0.0f});
-      case TATVA_DENSITY_LINEAR_ELASTIC: return f(kc, LinearElastic<D, float>{0.0f, 0.0f});
-      case TATVA_DENSITY_NEO_HOOKEAN: return f(kc, NeoHookean<D, float>{0.0f, 0.0f});
-      default: set_error("unknown density kind"); return TATVA_EINVAL;
-    }
-  };
+int with_kind(int kind, F &&f) {
   switch (kind) {
-    case TATVA_TRI3: return dens(std::integral_constant<int, TATVA_TRI3>{});
-    case TATVA_TET4: return dens(std::integral_constant<int, TATVA_TET4>{});
-    case TATVA_HEX8: return dens(std::integral_constant<int, TATVA_HEX8>{});
+    case TATVA_TRI3: return f(std::integral_constant<int, TATVA_TRI3>{});
+    case TATVA_TET4: return f(std::integral_constant<int, TATVA_TET4>{});
+    case TATVA_HEX8: return f(std::integral_constant<int, TATVA_HEX8>{});
     default: set_error("unknown element kind"); return TATVA_EINVAL;
   }
 }
@@ -540,8 +417,8 @@ extern "C" int tatva_batch_start(tatva_batch *B, int32_t slot, tatva_mesh *m,
   S.rr1 = (double *)(base + L.rr1);
   S.bb = (double *)(base + L.bb);
   S.st = B->d_states + slot;
-  S.g_blocks = gather_grid(m->n_nodes);
-  S.v_blocks = step_grid(n, kBatchPrefetch);
+  S.ncomp = ncomp;
+  S.v_blocks = step_grid(m->n_nodes, kStepNodes);
   S.start_tick = B->tick;
   // r = b - H x, z = D^-1 r, shares of r.z, r.r, b.b (w is scratch here)
   const int rc = matfree_pcg_setup(m, d, u, dof_map, n, diag, b, x, S.r, S.z, S.w, S.dinv, S.rz1,
@@ -551,8 +428,6 @@ extern "C" int tatva_batch_start(tatva_batch *B, int32_t slot, tatva_mesh *m,
   auto &mi = B->meta[slot];
   mi.active = true;
   mi.kind = m->kind;
-  mi.dkind = d->kind;
-  mi.ncomp = ncomp;
   mi.quad = m->quad;
   mi.affine = m->hex_box ? kGeomBox : m->hex_affine ? kGeomAffine : kGeomGeneral;
   mi.lds = lds;
@@ -601,24 +476,19 @@ int build_iterations(tatva_batch *B, int iters, hipGraph_t *out) {
   int rc = TATVA_OK;
   for (int it = 0; it < iters && err == hipSuccess && rc == TATVA_OK; ++it) {
     for (const auto &L : B->launches) {
-      rc = with_class(L.kind, L.dkind, [&](auto kc, auto dens_tag) -> int {
+      rc = with_kind(L.kind, [&](auto kc) -> int {
         constexpr int K = decltype(kc)::value;
-        using Dens = decltype(dens_tag);
         const int32_t *bm_a = B->d_bmap + L.a_off;
-        const int32_t *bm_g = B->d_bmap + L.g_off;
         QuadRule quad = L.quad;
         void *a_args[] = {(void *)&slots, (void *)&bm_a, (void *)&quad};
-        const void *fa = reinterpret_cast<const void *>(&k_batch_assemble<K, Dens, kGeomGeneral>);
+        const void *fa = reinterpret_cast<const void *>(&k_batch_assemble<K, kGeomGeneral>);
         if constexpr (K == TATVA_HEX8) {
           if (L.affine == kGeomBox)
-            fa = reinterpret_cast<const void *>(&k_batch_assemble<K, Dens, kGeomBox>);
+            fa = reinterpret_cast<const void *>(&k_batch_assemble<K, kGeomBox>);
           else if (L.affine == kGeomAffine)
-            fa = reinterpret_cast<const void *>(&k_batch_assemble<K, Dens, kGeomAffine>);
+            fa = reinterpret_cast<const void *>(&k_batch_assemble<K, kGeomAffine>);
         }
         err = add(fa, L.a_n, kTile, L.lds, a_args);
-        if (err != hipSuccess) return TATVA_OK;
-        void *g_args[] = {(void *)&slots, (void *)&bm_g};
-        err = add(reinterpret_cast<const void *>(&k_batch_gather<Dens::NC>), L.g_n, kBlock, 0, g_args);
         return TATVA_OK;
       });
       if (rc || err != hipSuccess) break;
@@ -649,8 +519,7 @@ std::vector<int64_t> launch_plan(const tatva_batch *B, int iters) {
   std::vector<int64_t> p{iters, B->v_off, B->v_n, (int64_t)(intptr_t)B->d_bmap,
                          (int64_t)(intptr_t)B->d_slots};
   for (const auto &L : B->launches) {
-    p.insert(p.end(), {L.kind, L.dkind, L.ncomp, L.affine, (int64_t)L.lds, L.a_off, L.a_n,
-                       L.g_off, L.g_n});
+    p.insert(p.end(), {L.kind, L.affine, (int64_t)L.lds, L.a_off, L.a_n});
     const int64_t *q = reinterpret_cast<const int64_t *>(&L.quad);
     p.insert(p.end(), q, q + sizeof(QuadRule) / sizeof(int64_t));
   }
