@@ -351,11 +351,6 @@ __device__ __forceinline__ void elem_diag(const double (&X)[Elem<KIND>::NNE][Ele
 // first makes them exactly zero there) has a constant Jacobian, inverted once
 // per element.  The results equal the nodal formulas up to rounding.
 
-// Hex8 local node -> sign index i + 2j + 4k (sx, sy, sz > 0 -> i, j, k = 1).
-__host__ __device__ constexpr int hex_bin(int a) {
-  return a ^ ((a >> 1) & 1);  // 2 <-> 3 and 6 <-> 7
-}
-
 // In-place sign-product transform v <- H v (unnormalised), stages x, y, z.
 template <class S>
 __device__ __forceinline__ void hadamard8(S (&v)[8]) {

@@ -158,7 +158,17 @@ __device__ __forceinline__ T block_sum_all(T v) {
 template <class T>
 __device__ __forceinline__ T sum_partials(const T *partials, int n) {
   T v = T(0);
-  for (int i = threadIdx.x; i < n; i += blockDim.x) v += partials[i];
+  // (eight loads together; a load at a time, the loop waits for each)
+  for (int i = threadIdx.x; i < n; i += 8 * kBlock) {
+    T w[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int j = i + k * kBlock;
+      w[k] = partials[j < n ? j : 0];
+      if (j >= n) w[k] = T(0);
+    }
+    v += ((w[0] + w[1]) + (w[2] + w[3])) + ((w[4] + w[5]) + (w[6] + w[7]));
+  }
   return block_sum_all(v);
 }
 

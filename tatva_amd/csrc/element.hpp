@@ -119,6 +119,61 @@ struct Elem<TATVA_HEX8> {
   }
 };
 
+// Hex8 node <-> sign index i + 2j + 4k (sx, sy, sz > 0 -> i, j, k = 1).
+__host__ __device__ constexpr int hex_bin(int a) {
+  return a ^ ((a >> 1) & 1);  // 2 <-> 3 and 6 <-> 7
+}
+
+// Natural derivatives and values of the trilinear shape functions at one point,
+// by sign index: a derivative is 1/8 times its sign times a product of two
+// factors (1 +- x), twelve products for the 24 derivatives.
+struct HexPoint {
+  double x, yz[4], xz[4], xy[4];
+  __device__ __forceinline__ HexPoint(double x_, double y, double z) : x(x_) {
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      const double a = (m & 1) ? 1.0 : -1.0, b = (m & 2) ? 1.0 : -1.0;
+      yz[m] = 0.125 * (1.0 + a * y) * (1.0 + b * z);
+      xz[m] = 0.125 * (1.0 + a * x) * (1.0 + b * z);
+      xy[m] = 0.125 * (1.0 + a * x) * (1.0 + b * y);
+    }
+  }
+  __device__ __forceinline__ void dN(int j, double (&d)[3]) const {
+    const double px = yz[(j >> 1) & 3], py = xz[(j & 1) | ((j >> 1) & 2)], pz = xy[j & 3];
+    d[0] = (j & 1) ? px : -px;
+    d[1] = (j & 2) ? py : -py;
+    d[2] = (j & 4) ? pz : -pz;
+  }
+  __device__ __forceinline__ double N(int j) const {
+    return ((j & 1) ? 1.0 + x : 1.0 - x) * yz[(j >> 1) & 3];
+  }
+};
+
+// Quadrature point q0 + s of the rule (the last one past its end) for lane s of
+// eight, by uniform reads of all eight: a kernel argument read at a lane's own
+// index is an uncached access to host memory.
+__device__ __forceinline__ void lane_point(const QuadRule &quad, int q0, int s, double &x, double &y,
+                                           double &z, double &w) {
+  x = y = z = w = 0.0;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int q = q0 + i < quad.nq ? q0 + i : quad.nq - 1;
+    if (s == i) {
+      x = quad.xi[q][0];
+      y = quad.xi[q][1];
+      z = quad.xi[q][2];
+      w = quad.w[q];
+    }
+  }
+}
+
+// Lanes of one wave writing and then reading the same LDS.
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // 1 / x: correctly rounded in FP64; in FP32 the hardware reciprocal (1 ulp),
 // which the FP32 tangent of the matrix-free product uses.
 template <class T>

@@ -36,13 +36,6 @@
 
 namespace tatva {
 
-// Lanes of one wave writing and then reading the same LDS.
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // Lanes per node and per element.  Hex8: eight lanes an element (lane s takes
 // quadrature points s, s + 8, ..., then one column block), 64 a node (the
 // eight elements of an inner node at once).  Simplices: one lane an element;
@@ -87,39 +80,17 @@ __device__ __forceinline__ void hex8_row_blocks(const double *__restrict__ xs, i
   for (int i = 0; i < NV; ++i) out[i] = 0.0;
   for (int q0 = 0; q0 < quad.nq; q0 += 8) {
     const bool on = q0 + s < quad.nq;
-    // this lane's point, by uniform reads of all eight (a kernel argument read
-    // at a lane's own index is an uncached access to host memory)
-    double x = 0.0, y = 0.0, z = 0.0, wq = 0.0;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int q = q0 + i < quad.nq ? q0 + i : quad.nq - 1;
-      if (s == i) {
-        x = t[0] * quad.xi[q][0];
-        y = t[1] * quad.xi[q][1];
-        z = t[2] * quad.xi[q][2];
-        wq = quad.w[q];
-      }
-    }
-    // dN of the node with signs (i, j, k): 1/8 times its sign times these products
-    double yz[4], xz[4], xy[4];
-#pragma unroll
-    for (int m = 0; m < 4; ++m) {
-      const double a = (m & 1) ? 1.0 : -1.0, b = (m & 2) ? 1.0 : -1.0;
-      yz[m] = 0.125 * (1.0 + a * y) * (1.0 + b * z);
-      xz[m] = 0.125 * (1.0 + a * x) * (1.0 + b * z);
-      xy[m] = 0.125 * (1.0 + a * x) * (1.0 + b * y);
-    }
-    const auto dn = [&](int j, double (&d)[3]) {
-      const double px = yz[(j >> 1) & 3], py = xz[(j & 1) | ((j >> 1) & 2)], pz = xy[j & 3];
-      d[0] = (j & 1) ? px : -px;
-      d[1] = (j & 2) ? py : -py;
-      d[2] = (j & 4) ? pz : -pz;
-    };
+    double x, y, z, wq;
+    lane_point(quad, q0, s, x, y, z, wq);
+    x *= t[0];
+    y *= t[1];
+    z *= t[2];
+    const HexPoint pt(x, y, z);
     double J[3][3] = {}, H[3][3] = {};
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       double d[3];
-      dn(j, d);
+      pt.dN(j, d);
       const double *nd = xs + (j ^ s) * 6;
 #pragma unroll
       for (int c = 0; c < 3; ++c) {
@@ -176,7 +147,7 @@ __device__ __forceinline__ void hex8_row_blocks(const double *__restrict__ xs, i
     }
     const auto block = [&](int j, double (&v)[NV]) {
       double d[3];
-      dn(j, d);
+      pt.dN(j, d);
       if constexpr (NC == 1) {
         v[0] = n[0] * d[0] + n[1] * d[1] + n[2] * d[2];
       } else {

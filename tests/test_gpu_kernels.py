@@ -207,3 +207,28 @@ def test_matfree_pcg_step_by_nodes(shape, density, full):
     assert out[0][0] == out[1][0] and torch.equal(out[0][1], out[1][1])
     r = b.double() - red.hvp_full_state(u.double(), out[0][1].double())
     assert float(r.norm() / b.double().norm()) < 2e-4
+
+
+@pytest.mark.parametrize("nc", [1, 2, 3, 4])
+@pytest.mark.parametrize("kind,points", [("tri3", 1), ("tri3", 3), ("tet4", 1), ("hex8", 1),
+                                         ("hex8", 2), ("hex8", 3)])
+@pytest.mark.parametrize("cells", [1, 2, 11])
+def test_point_fields(cells, kind, points, nc):
+    """Values and gradients at the points: elements that do not fill a wave and that
+    spill into the next block, 1, 8 and 27 points over eight lanes, the components
+    that are template parameters and one more."""
+    rule = (None, None)
+    if kind == "tri3":
+        mesh, el = ta.Mesh.unit_square(cells, 3), ta.Tri3
+        if points == 3:
+            rule = np.array([[1 / 6, 1 / 6], [2 / 3, 1 / 6], [1 / 6, 2 / 3]]), np.full(3, 1 / 6)
+    elif kind == "tet4":
+        mesh, el = ta.Mesh.box((cells, 3, 5), type="tetrahedron", jitter=0.1), ta.Tetrahedron4
+    else:
+        mesh, el, rule = ta.Mesh.box((cells, 3, 5), jitter=0.1), ta.Hexahedron8, gauss(points)
+    el = el(*rule)
+    op = ta.Operator(mesh, el)
+    oel = ORACLE_EL[type(el)](el.quad_points, el.quad_weights)
+    u = np.random.default_rng(1).standard_normal((mesh.n_nodes, nc))
+    assert rel_err(to_np(op.eval(u)), fem.op_eval(oel, mesh.coords, mesh.elements, u)) < RTOL
+    assert rel_err(to_np(op.grad(u)), fem.op_grad(oel, mesh.coords, mesh.elements, u)) < RTOL
