@@ -55,7 +55,11 @@ struct TileSet {
 // cache and writes no output; kModeHvpLin is kModeHvp reading that cache instead
 // of re-linearising at every call (same arithmetic, same result), for solvers
 // whose state is fixed over many products.
-enum { kModeResidual = 0, kModeHvp = 1, kModeDiag = 2, kModeLinearize = 3, kModeHvpLin = 4 };
+// kModeEnergy (Hex8) sums psi(G) w per element and writes the tile's share to dot.
+enum {
+  kModeResidual = 0, kModeHvp = 1, kModeDiag = 2, kModeLinearize = 3, kModeHvpLin = 4,
+  kModeEnergy = 5
+};
 
 // Cache layout: value k of quadrature point q of the element in tile slot t of
 // tile b at lin[((b * nq + q) * kLin + k) * kTile + t] (a tile's threads read
@@ -467,6 +471,7 @@ __device__ __forceinline__ double hex8_box_inverse(const double (&lo)[3], const 
 // Hessian-vector product (S = dP(G(u); G(v))): ye = sum_q w_q B_q^T S_q.
 // Geometry in FP64, physics in T.
 // MODE kModeLinearize / kModeHvpLin: as elem_hvp (cache at lin, stride kTile).
+// MODE kModeEnergy: ye[0][0] = sum_q w_q psi(G_q) (with the Poisson source).
 // GEOM: AFFINE for all but kGeomGeneral; the cached ones read J^-1 and det J
 // from geo (this element's geometry cache, stride kTile) instead of computing
 // them from X, the box ones hold the diagonal of J^-1 only (X: nodes 0 and 6).
@@ -564,6 +569,14 @@ __device__ __forceinline__ void hex8_element(const double (&X)[8][3], const T (&
           G[c][j] = BOX ? h[j] * iv[j][j] : h[0] * iv[j][0] + h[1] * iv[j][1] + h[2] * iv[j][2];
       }
     }
+    if constexpr (MODE == kModeEnergy) {
+      T uq = T(0);
+      if constexpr (Dens::kSource)
+        uq = UM[0][0] + UM[0][1] * xt + UM[0][2] * yt + UM[0][3] * xy + UM[0][4] * zt +
+             UM[0][5] * xz + UM[0][6] * yz + UM[0][7] * xyz;
+      A[0][0] += dens.psi(G, uq) * w;
+      continue;
+    }
     T *lq = (MODE == kModeLinearize || MODE == kModeHvpLin)
                 ? lin + (int64_t)q * Dens::kLin * kTile : nullptr;
     if constexpr (MODE == kModeLinearize) {
@@ -624,6 +637,10 @@ __device__ __forceinline__ void hex8_element(const double (&X)[8][3], const T (&
       A[0][7] -= s * xyz;
     }
   }
+  if constexpr (MODE == kModeEnergy) {
+    ye[0][0] = A[0][0];
+    return;
+  }
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
     T v[8];
@@ -659,29 +676,31 @@ inline int hex_affine_host(const double (&X)[8][3]) {
 
 // ------------------------------------------------------ tile assembly ------
 
-// LDS of one tile: per local node its coordinates (FP64), then the
+// LDS of one tile: per local node its coordinates (FP64), then (color sum) the
 // accumulator, the state and (HVP) the tangent in a T of tsize bytes.  With
 // the incidence-list sum the element vectors (kTile x nne x NC) reuse that
-// space, and the tile's incidence lists follow it.
+// space, and the tile's incidence lists follow it; an energy has neither.
 constexpr size_t align16(size_t x) { return (x + 15) & ~size_t(15); }
-constexpr size_t tile_stage_bytes(int max_local, int D, int NC, size_t tsize, int mode) {
-  return (size_t)max_local *
-         (D * sizeof(double) + ((mode == kModeHvp || mode == kModeHvpLin) ? 3 : 2) * NC * tsize);
+constexpr size_t tile_stage_bytes(bool gather, int max_local, int D, int NC, size_t tsize, int mode) {
+  const int vecs = 1 + (gather ? 0 : 1) + ((mode == kModeHvp || mode == kModeHvpLin) ? 1 : 0);
+  return (size_t)max_local * (D * sizeof(double) + vecs * NC * tsize);
 }
 // Values between two threads' element vectors in the incidence-list sum: nne*NC
 // rounded up to an odd count, so that the threads of a wave writing their
 // vectors hit distinct LDS banks (with 12 the lanes t and t + 8 share one).
 constexpr int tile_elem_stride(int nne, int NC) { return nne * NC + ((nne * NC) % 2 == 0 ? 1 : 0); }
 constexpr size_t tile_union_bytes(int max_local, int D, int nne, int NC, size_t tsize, int mode) {
-  const size_t staged = tile_stage_bytes(max_local, D, NC, tsize, mode);
-  const size_t elem = (size_t)kTile * tile_elem_stride(nne, NC) * tsize;
+  const size_t staged = tile_stage_bytes(true, max_local, D, NC, tsize, mode);
+  const size_t elem = mode == kModeEnergy ? 0 : (size_t)kTile * tile_elem_stride(nne, NC) * tsize;
   return align16(elem > staged ? elem : staged);
 }
 // the color sum's copy of the tile's color offsets, after the staged nodes
 constexpr size_t tile_offs_bytes() { return align16(sizeof(int16_t) * (kMaxTileColors + 1)); }
 constexpr size_t tile_lds_bytes(int kind, int max_local, int D, int nne, int NC, size_t tsize,
                                 int mode) {
-  if (!tile_gather_kind(kind)) return align16(tile_stage_bytes(max_local, D, NC, tsize, mode)) + tile_offs_bytes();
+  if (!tile_gather_kind(kind))
+    return align16(tile_stage_bytes(false, max_local, D, NC, tsize, mode)) + tile_offs_bytes();
+  if (mode == kModeEnergy) return tile_union_bytes(max_local, D, nne, NC, tsize, mode);
   return tile_union_bytes(max_local, D, nne, NC, tsize, mode) + (size_t)kTile * nne * sizeof(uint16_t) +
          align16((size_t)max_local * sizeof(uint16_t));
 }
@@ -752,7 +771,7 @@ __device__ __forceinline__ void tile_assemble(int tile, const double *__restrict
   const int nloc = ts.node_ptr[tile + 1] - nb;
   double *Xs = reinterpret_cast<double *>(lds);
   T *acc = reinterpret_cast<T *>(Xs + (size_t)ts.max_local * D);
-  T *us = acc + (size_t)ts.max_local * NC;
+  T *us = acc + (tile_gather<KIND>() ? 0 : (size_t)ts.max_local * NC);
   T *vs = us + (size_t)ts.max_local * NC;
   // Stage the local nodes, two per thread at a time (the second one is the
   // first again past the end: the same values stored twice).  Every load of
@@ -805,7 +824,7 @@ __device__ __forceinline__ void tile_assemble(int tile, const double *__restrict
         }
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
-          acc[j * NC + c] = T(0);
+          if constexpr (!tile_gather<KIND>()) acc[j * NC + c] = T(0);
           if constexpr (kUsesU) us[j * NC + c] = uv[h][c];
           if constexpr (kUsesV) vs[j * NC + c] = vv[h][c];
         }
@@ -831,7 +850,7 @@ __device__ __forceinline__ void tile_assemble(int tile, const double *__restrict
   const bool real = (int)threadIdx.x < (int)off[ts.max_colors];
   // the color sum reads the offsets from LDS (copied with the nodes)
   int16_t *offs = reinterpret_cast<int16_t *>(
-      lds + align16(tile_stage_bytes(ts.max_local, D, NC, sizeof(T), MODE)));
+      lds + align16(tile_stage_bytes(false, ts.max_local, D, NC, sizeof(T), MODE)));
   if constexpr (!tile_gather<KIND>() && MODE != kModeLinearize) {
     for (int c = threadIdx.x; c <= ts.max_colors; c += kTile) offs[c] = off[c];
   }
@@ -875,8 +894,8 @@ __device__ __forceinline__ void tile_assemble(int tile, const double *__restrict
     T *lp = lin ? lin + (int64_t)tile * quad.nq * Dens::kLin * kTile + threadIdx.x : nullptr;
     const T *gp =
         kGeo ? geo + (int64_t)tile * geo_floats(geom_box(GEOM)) * kTile + threadIdx.x : nullptr;
-    if constexpr (KIND == TATVA_HEX8 && MODE == kModeResidual) {
-      hex8_element<Dens, T, kModeResidual, GEOM>(X, ue, ue, quad, de, ye);
+    if constexpr (KIND == TATVA_HEX8 && (MODE == kModeResidual || MODE == kModeEnergy)) {
+      hex8_element<Dens, T, MODE, GEOM>(X, ue, ue, quad, de, ye);
     } else if constexpr (MODE == kModeResidual) {
       elem_residual<KIND, Dens>(X, ue, quad, de, ye);
     } else if constexpr (MODE == kModeHvp || MODE == kModeHvpLin || MODE == kModeLinearize) {
@@ -888,6 +907,10 @@ __device__ __forceinline__ void tile_assemble(int tile, const double *__restrict
     }
   }
   if constexpr (MODE == kModeLinearize) return;  // the cache is the output
+  if constexpr (MODE == kModeEnergy) {
+    tile_share((double)ye[0][0], lds, dot + tile);
+    return;
+  }
   if constexpr (tile_gather<KIND>()) {
     if constexpr (!kIncEarly) {
       inc_pk = reinterpret_cast<const IncVec *>(ts.inc_list + (int64_t)tile * kTile * NNE)[threadIdx.x];

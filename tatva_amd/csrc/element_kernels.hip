@@ -349,7 +349,9 @@ __global__ __launch_bounds__(kBlock) void k_density_eval(int64_t n_elem, int nq,
   psi[i] = dens.at(i / nq).psi(G, uq);
 }
 
-// Sum over elements of sum_q psi(G_q) detJ w_q (+ Poisson source via u_q).
+// Sum over elements of sum_q psi(G_q) detJ w_q (+ Poisson source via u_q):
+// simplices.  Hex8 energies run on the tiles (kModeEnergy): nodes staged in LDS and
+// modal derivatives, 80^3 distorted Neo-Hookean 65.8 -> 45.7 us.
 template <int KIND, class Dens>
 __global__ __launch_bounds__(kBlock) void k_energy(int64_t n_elem, const double *__restrict__ coords,
                                                    const int32_t *__restrict__ conn, QuadRule quad,
@@ -1194,7 +1196,8 @@ extern "C" int tatva_mesh_create(int device, int elem_kind, const double *coords
     return fail(err, "hipMalloc inv_list");
   if ((err = hipMalloc(&m->scratch, m->scratch_bytes)) != hipSuccess)
     return fail(err, "hipMalloc scratch");
-  if ((err = hipMalloc(&m->partials, kMaxReduceBlocks * 4 * sizeof(double))) != hipSuccess)
+  if ((err = hipMalloc(&m->partials, std::max<int64_t>(kMaxReduceBlocks * 4, m->tiles.n_tiles) *
+                                         sizeof(double))) != hipSuccess)
     return fail(err, "hipMalloc partials");
   if ((err = hipMemcpyAsync(m->coords, coords, n_nodes * dim * sizeof(double), hipMemcpyHostToDevice, up)) != hipSuccess)
     return fail(err, "copy coords");
@@ -1362,6 +1365,15 @@ extern "C" int tatva_density_eval(int dim, int64_t n_points, const tatva_density
   });
 }
 
+namespace tatva {
+template <class T, int MODE>
+static int launch_assembly(tatva_mesh *m, const tatva_density *d, const T *u, const T *v,
+                           const int32_t *dof_map, const double *f_ext, T *out, hipStream_t s,
+                           const int *skip, double *part_dot = nullptr, int gather_blocks = 0,
+                           int rev = 0, hipEvent_t between = nullptr, T *lin = nullptr,
+                           const T *geo = nullptr, const CgDefer &dx = CgDefer{});
+}  // namespace tatva
+
 extern "C" int tatva_energy(tatva_mesh *m, const tatva_density *d, const double *u,
                             const double *f_ext, double *out, void *stream) {
   MESH_PRELUDE(m);
@@ -1371,9 +1383,17 @@ extern "C" int tatva_energy(tatva_mesh *m, const tatva_density *d, const double 
     constexpr int K = decltype(kc)::value;
     return with_density<Elem<K>::D, double>(d, [&](auto dens) -> int {
       using Dens = decltype(dens);
-      const int g = reduce_grid(m->n_elements);
-      k_energy<K, Dens><<<g, kBlock, 0, s>>>(m->n_elements, m->coords, m->conn, m->quad, dens, u,
-                                             m->partials);
+      int g;
+      if constexpr (K == TATVA_HEX8) {
+        g = m->tiles.n_tiles;
+        const int e = launch_assembly<double, kModeEnergy>(m, d, u, nullptr, nullptr, nullptr,
+                                                           nullptr, s, nullptr, m->partials);
+        if (e) return e;
+      } else {
+        g = reduce_grid(m->n_elements);
+        k_energy<K, Dens><<<g, kBlock, 0, s>>>(m->n_elements, m->coords, m->conn, m->quad, dens, u,
+                                               m->partials);
+      }
       k_finalize_sum<double><<<1, kBlock, 0, s>>>(m->partials, g, out, 0);
       TATVA_CHECK_LAUNCH();
       return TATVA_OK;
@@ -1399,9 +1419,8 @@ namespace tatva {
 template <class T, int MODE>
 static int launch_assembly(tatva_mesh *m, const tatva_density *d, const T *u, const T *v,
                            const int32_t *dof_map, const double *f_ext, T *out, hipStream_t s,
-                           const int *skip, double *part_dot = nullptr, int gather_blocks = 0,
-                           int rev = 0, hipEvent_t between = nullptr, T *lin = nullptr,
-                           const T *geo = nullptr, const CgDefer &dx = CgDefer{}) {
+                           const int *skip, double *part_dot, int gather_blocks, int rev,
+                           hipEvent_t between, T *lin, const T *geo, const CgDefer &dx) {
   T *partial = (T *)m->scratch;
   return with_kind(m->kind, [&](auto kc) -> int {
     constexpr int K = decltype(kc)::value;
@@ -1410,6 +1429,9 @@ static int launch_assembly(tatva_mesh *m, const tatva_density *d, const T *u, co
       constexpr int NC = Dens::NC;
       if constexpr ((MODE == kModeLinearize || MODE == kModeHvpLin) && Dens::kLin == 0) {
         set_error("this density has no linearisation to cache");
+        return TATVA_EINVAL;
+      } else if constexpr (MODE == kModeEnergy && K != TATVA_HEX8) {
+        set_error("the tiled energy is for Hex8");
         return TATVA_EINVAL;
       } else {
       const size_t lds = tile_lds_bytes(K, m->tiles.max_local, Elem<K>::D, Elem<K>::NNE, NC, sizeof(T), MODE);
@@ -1457,6 +1479,10 @@ static int launch_assembly(tatva_mesh *m, const tatva_density *d, const T *u, co
       if constexpr (MODE == kModeLinearize) {
         TATVA_CHECK_LAUNCH();
         return TATVA_OK;  // the cache is the output: no gather
+      }
+      if constexpr (MODE == kModeEnergy) {
+        TATVA_CHECK_LAUNCH();
+        return TATVA_OK;  // the tiles' shares are the output
       }
       // optional event between the tile kernel and the gather (kernel timing)
       if (between) TATVA_TRY_HIP(hipEventRecord(between, s));

@@ -25,7 +25,7 @@ struct tatva_mesh {
   int32_t *inv_list;     // packed (element << 3 | local node), sorted by element per node
   void *scratch;         // tile partial sums: n_slots * dim doubles
   int64_t scratch_bytes;
-  double *partials;      // reduction partials, kMaxReduceBlocks * 4
+  double *partials;      // reduction partials: the larger of kMaxReduceBlocks * 4 and a tile each
   int max_incident;      // largest number of elements sharing a node
   int hex_affine;        // Hex8 mesh of parallelepipeds only (constant Jacobian per element)
   int hex_box;           // ... of boxes along the coordinate axes (diagonal Jacobian)

@@ -232,3 +232,22 @@ def test_point_fields(cells, kind, points, nc):
     u = np.random.default_rng(1).standard_normal((mesh.n_nodes, nc))
     assert rel_err(to_np(op.eval(u)), fem.op_eval(oel, mesh.coords, mesh.elements, u)) < RTOL
     assert rel_err(to_np(op.grad(u)), fem.op_grad(oel, mesh.coords, mesh.elements, u)) < RTOL
+
+
+@pytest.mark.parametrize("density", [LE, NH, PO], ids=["le", "nh", "poisson"])
+@pytest.mark.parametrize("points", [1, 2, 3])
+@pytest.mark.parametrize("shape,jitter", [((1, 1, 1), 0.0), ((8, 4, 4), 0.0), ((43, 3, 1), 0.1),
+                                          ((9, 7, 5), 0.1)])
+def test_hex8_energy_by_tiles(shape, jitter, points, density):
+    """One element, exactly a tile (128), one element more and a part-filled last
+    tile; affine and general elements, other rules, the Poisson source.  Neo-Hookean
+    energies are differences of terms of mu/2 (I1, 3, 2 ln J) over the unit volume, so
+    rounding is relative to those; gradients stay near 0.1, short of inverted elements."""
+    el = ta.Hexahedron8(*gauss(points))
+    mesh = ta.Mesh.box(shape, jitter=jitter, seed=4)
+    prob = fem.Problem(fem.Hex8(el.quad_points, el.quad_weights), mesh.coords, mesh.elements,
+                       ORACLE[density])
+    E = ta.Operator(mesh, el).energy(density)
+    u = 0.05 / max(shape) * np.random.default_rng(2).uniform(-1, 1, E.size)
+    ref = prob.energy(u)
+    assert abs(float(E(u)) - ref) < RTOL * (abs(ref) + 1.5 * 0.7)
