@@ -291,7 +291,7 @@ __device__ __forceinline__ void elem_hvp(const double (&X)[Elem<KIND>::NNE][Elem
   }
 }
 
-// diag of K_e: d_e[a][c] = sum_q w (dP(G; e_c B_a) B)_ac
+// diag of K_e: d_e[a][c] = sum_q w (dP(G; e_c B_a) B)_ac (simplices)
 template <int KIND, class Dens, class T>
 __device__ __forceinline__ void elem_diag(const double (&X)[Elem<KIND>::NNE][Elem<KIND>::D],
                                           const T (&ue)[Elem<KIND>::NNE][Dens::NC],
@@ -323,20 +323,14 @@ __device__ __forceinline__ void elem_diag(const double (&X)[Elem<KIND>::NNE][Ele
       }
     const auto L = dens.linearize(G);
 #pragma unroll
-    for (int a = 0; a < NNE; ++a)
+    for (int a = 0; a < NNE; ++a) {
+      T Ba[D], d[NC];
 #pragma unroll
-      for (int c = 0; c < NC; ++c) {
-        T dG[NC][D], dP[NC][D];
+      for (int j = 0; j < D; ++j) Ba[j] = B[j][a];
+      dens.diag(L, Ba, d);
 #pragma unroll
-        for (int cc = 0; cc < NC; ++cc)
-#pragma unroll
-          for (int j = 0; j < D; ++j) dG[cc][j] = (cc == c) ? B[j][a] : T(0);
-        dens.dP(L, dG, dP);
-        T s = T(0);
-#pragma unroll
-        for (int j = 0; j < D; ++j) s += dP[c][j] * B[j][a];
-        de[a][c] += w * s;
-      }
+      for (int c = 0; c < NC; ++c) de[a][c] += w * d[c];
+    }
   }
 }
 
@@ -472,6 +466,10 @@ __device__ __forceinline__ double hex8_box_inverse(const double (&lo)[3], const 
 // Geometry in FP64, physics in T.
 // MODE kModeLinearize / kModeHvpLin: as elem_hvp (cache at lin, stride kTile).
 // MODE kModeEnergy: ye[0][0] = sum_q w_q psi(G_q) (with the Poisson source).
+// MODE kModeDiag: ye += the diagonal of the element stiffness, from the density's
+// closed form at each node's shape gradient (24 directional derivatives per point
+// and the nodal FP64 geometry took 1575 us at 160^3 boxes in FP32, now 252; 29 -> 16
+// at 40^3); the gradients are rounded from FP64 as they were.
 // GEOM: AFFINE for all but kGeomGeneral; the cached ones read J^-1 and det J
 // from geo (this element's geometry cache, stride kTile) instead of computing
 // them from X, the box ones hold the diagonal of J^-1 only (X: nodes 0 and 6).
@@ -524,6 +522,15 @@ __device__ __forceinline__ void hex8_element(const double (&X)[8][3], const T (&
   } else if constexpr (AFFINE) {
     det0 = hex8_affine_inverse<T>(X, iv0);
   }
+  double inv[3][3];
+  if constexpr (MODE == kModeDiag && BOX) {
+    double iv[3];
+    hex8_box_inverse<double>(X[0], X[6], iv);
+#pragma unroll
+    for (int j = 0; j < 3; ++j) inv[j][j] = iv[j];
+  } else if constexpr (MODE == kModeDiag && AFFINE) {
+    hex8_affine_inverse<double>(X, inv);
+  }
   for (int q = 0; q < quad.nq; ++q) {
     const double x = quad.xi[q][0], y = quad.xi[q][1], z = quad.xi[q][2];
     // the point in T and its products: uniform values (FP32: from the kernel
@@ -536,7 +543,7 @@ __device__ __forceinline__ void hex8_element(const double (&X)[8][3], const T (&
       xt = T(x), yt = T(y), zt = T(z);
       yz = yt * zt, xz = xt * zt, xy = xt * yt, xyz = xt * yt * zt;
     }
-    double inv[3][3], det;
+    double det;
     if constexpr (AFFINE) {
       det = det0;
     } else {
@@ -575,6 +582,28 @@ __device__ __forceinline__ void hex8_element(const double (&X)[8][3], const T (&
         uq = UM[0][0] + UM[0][1] * xt + UM[0][2] * yt + UM[0][3] * xy + UM[0][4] * zt +
              UM[0][5] * xz + UM[0][6] * yz + UM[0][7] * xyz;
       A[0][0] += dens.psi(G, uq) * w;
+      continue;
+    }
+    if constexpr (MODE == kModeDiag) {
+      const auto L = dens.linearize(G);
+      // the nodes' shape gradients, rounded to T once
+      const double px[2] = {0.5 - 0.5 * x, 0.5 + 0.5 * x};
+      const double py[2] = {0.5 - 0.5 * y, 0.5 + 0.5 * y};
+      const double pz[2] = {0.5 - 0.5 * z, 0.5 + 0.5 * z};
+#pragma unroll
+      for (int a = 0; a < 8; ++a) {
+        const int i = hex_bin(a) & 1, j = (hex_bin(a) >> 1) & 1, k = hex_bin(a) >> 2;
+        const double n[3] = {(i - 0.5) * (py[j] * pz[k]), (j - 0.5) * (px[i] * pz[k]),
+                             (k - 0.5) * (px[i] * py[j])};
+        T B[3], d[NC];
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+          B[j] = T(BOX ? n[j] * inv[j][j]
+                       : n[0] * inv[j][0] + n[1] * inv[j][1] + n[2] * inv[j][2]);
+        dens.diag(L, B, d);
+#pragma unroll
+        for (int c = 0; c < NC; ++c) ye[a][c] += w * d[c];
+      }
       continue;
     }
     T *lq = (MODE == kModeLinearize || MODE == kModeHvpLin)
@@ -637,6 +666,7 @@ __device__ __forceinline__ void hex8_element(const double (&X)[8][3], const T (&
       A[0][7] -= s * xyz;
     }
   }
+  if constexpr (MODE == kModeDiag) return;
   if constexpr (MODE == kModeEnergy) {
     ye[0][0] = A[0][0];
     return;
@@ -894,7 +924,8 @@ __device__ __forceinline__ void tile_assemble(int tile, const double *__restrict
     T *lp = lin ? lin + (int64_t)tile * quad.nq * Dens::kLin * kTile + threadIdx.x : nullptr;
     const T *gp =
         kGeo ? geo + (int64_t)tile * geo_floats(geom_box(GEOM)) * kTile + threadIdx.x : nullptr;
-    if constexpr (KIND == TATVA_HEX8 && (MODE == kModeResidual || MODE == kModeEnergy)) {
+    if constexpr (KIND == TATVA_HEX8 && (MODE == kModeResidual || MODE == kModeEnergy ||
+                                        MODE == kModeDiag)) {
       hex8_element<Dens, T, MODE, GEOM>(X, ue, ue, quad, de, ye);
     } else if constexpr (MODE == kModeResidual) {
       elem_residual<KIND, Dens>(X, ue, quad, de, ye);

@@ -55,6 +55,12 @@ struct Poisson {
 #pragma unroll
     for (int j = 0; j < D; ++j) out[0][j] = w * dG[0][j];
   }
+  // d[c] = e_c . dP(e_c B) B: the diagonal of the tangent of a shape gradient B
+  __device__ __forceinline__ void diag(const Lin &, const T (&B)[D], T (&d)[NC]) const {
+    d[0] = T(0);
+#pragma unroll
+    for (int j = 0; j < D; ++j) d[0] += B[j] * B[j];
+  }
 };
 
 template <int D, class T>
@@ -124,6 +130,14 @@ struct LinearElastic {
   // w dP (the quadrature weight folded into the moduli)
   __device__ __forceinline__ void dPw(const Lin &, const T dG[NC][D], T w, T out[NC][D]) const {
     stress_with(w * mu, w * lam, dG, out);
+  }
+  // d[c] = mu |B|^2 + (mu + lambda) B_c^2
+  __device__ __forceinline__ void diag(const Lin &, const T (&B)[D], T (&d)[NC]) const {
+    T bb = T(0);
+#pragma unroll
+    for (int j = 0; j < D; ++j) bb += B[j] * B[j];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) d[c] = mu * bb + (mu + lam) * (B[c] * B[c]);
   }
 };
 
@@ -227,6 +241,22 @@ struct NeoHookean {
   // w dP (the quadrature weight folded into mu, mu - lambda ln J and lambda)
   __device__ __forceinline__ void dPw(const Lin &L, const T dG[NC][D], T w, T out[NC][D]) const {
     dP_with(w * mu, w * L.c1, w * lam, L, dG, out);
+  }
+  // d[c] = mu |B|^2 + (mu - lambda ln J + lambda) (F^-T B)_c^2: with dG = e_c B,
+  // tr(W) = (F^-T B)_c and e_c . Z^T B = (F^-T B)_c^2
+  __device__ __forceinline__ void diag(const Lin &L, const T (&B)[D], T (&d)[NC]) const {
+    T bb = T(0);
+#pragma unroll
+    for (int j = 0; j < D; ++j) bb += B[j] * B[j];
+    bb *= mu;
+    const T k = L.c1 + lam;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      T g = T(0);
+#pragma unroll
+      for (int j = 0; j < D; ++j) g += L.Fi[j][c] * B[j];
+      d[c] = bb + k * (g * g);
+    }
   }
   // m dG + c Z^T + l tr(W) F^-T with W = F^-1 dG, Z = W F^-1
   // ((F^-T dG^T F^-T)_ij = Z_ji, tr(F^-1 dG) = tr W)

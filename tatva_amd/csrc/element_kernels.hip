@@ -1460,7 +1460,7 @@ static int launch_assembly(tatva_mesh *m, const tatva_density *d, const T *u, co
             gather_blocks ? nullptr : part_dot);
       };
       using std::integral_constant;
-      if constexpr (K == TATVA_HEX8 && MODE != kModeDiag) {  // (the diagonal works nodal)
+      if constexpr (K == TATVA_HEX8) {
         if (geo) {
           if constexpr (kCacheable) {
             if (m->hex_box) launch(integral_constant<int, kGeomBoxCache>{});

@@ -251,3 +251,23 @@ def test_hex8_energy_by_tiles(shape, jitter, points, density):
     u = 0.05 / max(shape) * np.random.default_rng(2).uniform(-1, 1, E.size)
     ref = prob.energy(u)
     assert abs(float(E(u)) - ref) < RTOL * (abs(ref) + 1.5 * 0.7)
+
+
+@pytest.mark.parametrize("density", [LE, NH, PO], ids=["le", "nh", "poisson"])
+@pytest.mark.parametrize("form", ["box", "turned", "sheared", "general", "tet4"])
+def test_stiffness_diagonal(form, density):
+    """The closed forms against the oracle: FP64 to 1e-12, FP32 to 2e-6 of the largest
+    entry (some tens of roundings of 6e-8, as the product)."""
+    import torch
+
+    if form == "tet4":
+        mesh, el = ta.Mesh.box((5, 4, 7), type="tetrahedron", jitter=0.1), ta.Tetrahedron4
+    else:
+        mesh, el = hex_variant(form), ta.Hexahedron8
+    E = ta.Operator(mesh, el()).energy(density)
+    prob = fem.Problem(ORACLE_EL[el](), mesh.coords, mesh.elements, ORACLE[density])
+    u = 0.005 * np.random.default_rng(5).standard_normal(E.size)
+    assert rel_err(to_np(E.hessian_diag(u)), prob.hessian_diag(u)) < RTOL
+    u32 = torch.as_tensor(u, dtype=torch.float32, device="cuda")
+    ref = prob.hessian_diag(to_np(u32).astype(float))
+    assert rel_err(to_np(E.hessian_diag(u32, dtype=torch.float32)), ref) < 2e-6
