@@ -471,7 +471,7 @@ __device__ __forceinline__ double hex8_box_inverse(const double (&lo)[3], const 
 // and the nodal FP64 geometry took 1575 us at 160^3 boxes in FP32, now 252; 29 -> 16
 // at 40^3); the gradients are rounded from FP64 as they were.
 // GEOM: AFFINE for all but kGeomGeneral; the cached ones read J^-1 and det J
-// from geo (this element's geometry cache, stride kTile) instead of computing
+// from geo (this element's geo_floats values of the cache) instead of computing
 // them from X, the box ones hold the diagonal of J^-1 only (X: nodes 0 and 6).
 template <class Dens, class T, int MODE, int GEOM>
 __device__ __forceinline__ void hex8_element(const double (&X)[8][3], const T (&ue)[8][Dens::NC],
@@ -502,9 +502,9 @@ __device__ __forceinline__ void hex8_element(const double (&X)[8][3], const T (&
   double det0 = 0.0;
   if constexpr (GEO && BOX) {
 #pragma unroll
-    for (int j = 0; j < 3; ++j) iv0[j][j] = geo[j * kTile];
-    const uint32_t lo = __float_as_uint(float(geo[3 * kTile]));
-    const uint32_t hi = __float_as_uint(float(geo[4 * kTile]));
+    for (int j = 0; j < 3; ++j) iv0[j][j] = geo[j];
+    const uint32_t lo = __float_as_uint(float(geo[3]));
+    const uint32_t hi = __float_as_uint(float(geo[4]));
     det0 = __hiloint2double((int)hi, (int)lo);
   } else if constexpr (BOX) {
     T iv[3];
@@ -515,9 +515,9 @@ __device__ __forceinline__ void hex8_element(const double (&X)[8][3], const T (&
 #pragma unroll
     for (int i = 0; i < 3; ++i)
 #pragma unroll
-      for (int j = 0; j < 3; ++j) iv0[i][j] = geo[(i * 3 + j) * kTile];
-    const uint32_t lo = __float_as_uint(float(geo[9 * kTile]));
-    const uint32_t hi = __float_as_uint(float(geo[10 * kTile]));
+      for (int j = 0; j < 3; ++j) iv0[i][j] = geo[i * 3 + j];
+    const uint32_t lo = __float_as_uint(float(geo[9]));
+    const uint32_t hi = __float_as_uint(float(geo[10]));
     det0 = __hiloint2double((int)hi, (int)lo);
   } else if constexpr (AFFINE) {
     det0 = hex8_affine_inverse<T>(X, iv0);
@@ -784,7 +784,8 @@ __device__ __forceinline__ void tile_assemble(int tile, const double *__restrict
                                               unsigned char *__restrict__ lds,
                                               T *__restrict__ lin = nullptr,
                                               const T *__restrict__ geo = nullptr,
-                                              double *__restrict__ dot = nullptr) {
+                                              double *__restrict__ dot = nullptr,
+                                              const int *__restrict__ skip = nullptr) {
   constexpr bool kUsesU = MODE != kModeHvpLin;
   constexpr bool kUsesV = MODE == kModeHvp || MODE == kModeHvpLin;
   using El = Elem<KIND>;
@@ -797,12 +798,43 @@ __device__ __forceinline__ void tile_assemble(int tile, const double *__restrict
                                              MODE == kModeLinearize)),
                 "a geometry cache serves the FP32 product");
   constexpr bool uses_x = !kGeo;
-  const int32_t nb = ts.node_ptr[tile];
-  const int nloc = ts.node_ptr[tile + 1] - nb;
+  // the stop flag together with the tile's node range, not one wait after the other
+  const int32_t *flag = skip ? skip : ts.node_ptr;
+  const int32_t nb = ts.node_ptr[tile], ne = ts.node_ptr[tile + 1], stop = *flag;
+  asm volatile("" ::"s"(nb), "s"(ne), "s"(stop));
+  if (skip && stop) return;
+  const int nloc = ne - nb;
   double *Xs = reinterpret_cast<double *>(lds);
   T *acc = reinterpret_cast<T *>(Xs + (size_t)ts.max_local * D);
   T *us = acc + (tile_gather<KIND>() ? 0 : (size_t)ts.max_local * NC);
   T *vs = us + (size_t)ts.max_local * NC;
+  // Loads that depend on the tile alone, before the staging's chain (node ids, then
+  // values) so that their latency overlaps it: the element's local node numbers
+  // (padding slots hold valid entries too) and its incidence entries, one 16- / 8-byte
+  // load each for Hex8 / Tet4, and its geometry cache.  The lists wait in LDS of their own.
+  // Loaded where they are used (the cache, the lists and the sums' places behind a
+  // barrier each, a sum's entries one by one), they cost the FP32 Neo-Hookean product
+  // of boxes 261 us at 160^3, now 234, and 13.3 at 40^3 (one tile a CU), now 12.4.
+  const int64_t slot = (int64_t)tile * kTile + threadIdx.x;
+  using PackedNodes = std::conditional_t<NNE == 8, uint4, uint2>;  // NNE uint16 entries
+  constexpr bool kLists = tile_gather<KIND>() && MODE != kModeLinearize && MODE != kModeEnergy;
+  PackedNodes ln_pk{}, inc_pk{};
+  if constexpr (NNE == 8 || NNE == 4) ln_pk = reinterpret_cast<const PackedNodes *>(ts.lnodes)[slot];
+  T gv[kGeo ? geo_floats(geom_box(GEOM)) : 1];
+  if constexpr (kGeo) {
+#pragma unroll
+    for (int k = 0; k < geo_floats(geom_box(GEOM)); ++k)
+      gv[k] = geo[((int64_t)tile * geo_floats(geom_box(GEOM)) + k) * kTile + threadIdx.x];
+  }
+  uint32_t inc_e[2] = {};
+  if constexpr (kLists) {
+    inc_pk = reinterpret_cast<const PackedNodes *>(ts.inc_list)[slot];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int j = (int)threadIdx.x + h * kTile;
+      inc_e[h] = ts.inc_end[nb + (j < nloc ? j : 0)];
+    }
+  }
   // Stage the local nodes, two per thread at a time (the second one is the
   // first again past the end: the same values stored twice).  Every load of
   // the pair is issued before the first wait: the global node ids, then the
@@ -863,18 +895,17 @@ __device__ __forceinline__ void tile_assemble(int tile, const double *__restrict
   };
   if (kUsesV && dof_map) stage(std::true_type{});
   else stage(std::false_type{});
-  // Tet4: the tile's incidence lists are loaded here and stored to LDS after
-  // the element work, so their latency overlaps it (Hex8: loaded after the
-  // element work, whose registers are all in use)
-  using IncVec = std::conditional_t<NNE == 8, uint4, uint2>;  // NNE uint16 entries
-  constexpr bool kIncEarly = NNE == 4;
-  IncVec inc_pk{};
-  uint32_t inc_e = 0;
-  if constexpr (tile_gather<KIND>() && kIncEarly) {
-    inc_pk = reinterpret_cast<const IncVec *>(ts.inc_list + (int64_t)tile * kTile * NNE)[threadIdx.x];
-    if ((int)threadIdx.x < nloc) inc_e = ts.inc_end[nb + threadIdx.x];
+  uint16_t *il = nullptr, *ie = nullptr;
+  if constexpr (kLists) {
+    il = reinterpret_cast<uint16_t *>(lds +
+                                      tile_union_bytes(ts.max_local, D, NNE, NC, sizeof(T), MODE));
+    ie = il + kTile * NNE;
+    reinterpret_cast<PackedNodes *>(il)[threadIdx.x] = inc_pk;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      if ((int)threadIdx.x + h * kTile < nloc) ie[threadIdx.x + h * kTile] = (uint16_t)inc_e[h];
+    for (int j = threadIdx.x + 2 * kTile; j < nloc; j += kTile) ie[j] = ts.inc_end[nb + j];
   }
-  const int64_t slot = (int64_t)tile * kTile + threadIdx.x;
   const int16_t *off = ts.color_off + (int64_t)tile * (ts.max_colors + 1);
   // the tile's elements fill its first off[max_colors] slots (the rest is padding)
   const bool real = (int)threadIdx.x < (int)off[ts.max_colors];
@@ -884,14 +915,10 @@ __device__ __forceinline__ void tile_assemble(int tile, const double *__restrict
   if constexpr (!tile_gather<KIND>() && MODE != kModeLinearize) {
     for (int c = threadIdx.x; c <= ts.max_colors; c += kTile) offs[c] = off[c];
   }
-  // the element's local node numbers (padding slots hold valid entries too):
-  // one 16- / 8-byte load for Hex8 / Tet4
   int l[NNE];
   if constexpr (NNE == 8 || NNE == 4) {
-    using Vec = std::conditional_t<NNE == 8, uint4, uint2>;
-    const Vec pk = reinterpret_cast<const Vec *>(ts.lnodes)[slot];
-    const uint32_t w[4] = {pk.x, pk.y, NNE == 8 ? ((const uint32_t *)&pk)[2] : 0u,
-                           NNE == 8 ? ((const uint32_t *)&pk)[3] : 0u};
+    uint32_t w[NNE / 2];
+    __builtin_memcpy(w, &ln_pk, sizeof(ln_pk));
 #pragma unroll
     for (int a = 0; a < NNE; ++a) l[a] = real ? (int)((w[a >> 1] >> (16 * (a & 1))) & 0xffffu) : 0;
   } else {
@@ -922,8 +949,6 @@ __device__ __forceinline__ void tile_assemble(int tile, const double *__restrict
     }
     // this thread's cached linearisation (kModeLinearize / kModeHvpLin)
     T *lp = lin ? lin + (int64_t)tile * quad.nq * Dens::kLin * kTile + threadIdx.x : nullptr;
-    const T *gp =
-        kGeo ? geo + (int64_t)tile * geo_floats(geom_box(GEOM)) * kTile + threadIdx.x : nullptr;
     if constexpr (KIND == TATVA_HEX8 && (MODE == kModeResidual || MODE == kModeEnergy ||
                                         MODE == kModeDiag)) {
       hex8_element<Dens, T, MODE, GEOM>(X, ue, ue, quad, de, ye);
@@ -931,7 +956,7 @@ __device__ __forceinline__ void tile_assemble(int tile, const double *__restrict
       elem_residual<KIND, Dens>(X, ue, quad, de, ye);
     } else if constexpr (MODE == kModeHvp || MODE == kModeHvpLin || MODE == kModeLinearize) {
       if constexpr (KIND == TATVA_HEX8)
-        hex8_element<Dens, T, MODE, GEOM>(X, ue, ve, quad, de, ye, lp, gp);
+        hex8_element<Dens, T, MODE, GEOM>(X, ue, ve, quad, de, ye, lp, gv);
       else elem_hvp<KIND, Dens, T, MODE>(X, ue, ve, quad, de, ye, lp);
     } else {
       elem_diag<KIND, Dens, T>(X, ue, quad, de, ye);
@@ -942,24 +967,22 @@ __device__ __forceinline__ void tile_assemble(int tile, const double *__restrict
     tile_share((double)ye[0][0], lds, dot + tile);
     return;
   }
-  if constexpr (tile_gather<KIND>()) {
-    if constexpr (!kIncEarly) {
-      inc_pk = reinterpret_cast<const IncVec *>(ts.inc_list + (int64_t)tile * kTile * NNE)[threadIdx.x];
-      if ((int)threadIdx.x < nloc) inc_e = ts.inc_end[nb + threadIdx.x];
+  if constexpr (kLists) {
+    // where this thread's first two sums go, loaded while the tile's are computed
+    int32_t slot01[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int j = (int)threadIdx.x + h * kTile;
+      slot01[h] = ts.slot_pos[nb + (j < nloc ? j : 0)];
     }
     __syncthreads();  // every element has read its nodes: the LDS is free
     T *ys = reinterpret_cast<T *>(lds);
-    uint16_t *il = reinterpret_cast<uint16_t *>(
-        lds + tile_union_bytes(ts.max_local, D, NNE, NC, sizeof(T), MODE));
-    uint16_t *ie = il + kTile * NNE;
     constexpr int kYS = tile_elem_stride(NNE, NC);
+    constexpr int kSumChunk = 4;
 #pragma unroll
     for (int a = 0; a < NNE; ++a)
 #pragma unroll
       for (int c = 0; c < NC; ++c) ys[(int)threadIdx.x * kYS + a * NC + c] = ye[a][c];
-    reinterpret_cast<IncVec *>(il)[threadIdx.x] = inc_pk;
-    if ((int)threadIdx.x < nloc) ie[threadIdx.x] = (uint16_t)inc_e;
-    for (int j = threadIdx.x + kTile; j < nloc; j += kTile) ie[j] = ts.inc_end[nb + j];
     __syncthreads();
     // one local node per thread, its components together: one read of each
     // incidence entry serves all NC sums (each still in ascending entry order)
@@ -979,13 +1002,25 @@ __device__ __forceinline__ void tile_assemble(int tile, const double *__restrict
       T sum[NC];
 #pragma unroll
       for (int c = 0; c < NC; ++c) sum[c] = T(0);
-      for (int q = q0; q < q1; ++q) {
-        const int e = il[q];  // entry slot * NNE + a
-        const int base = (e / NNE) * kYS + (e % NNE) * NC;
+      for (int q = q0; q < q1; q += kSumChunk) {
+        int base[kSumChunk];
+        T part[kSumChunk][NC];
 #pragma unroll
-        for (int c = 0; c < NC; ++c) sum[c] += ys[base + c];
+        for (int k = 0; k < kSumChunk; ++k) {
+          const int e = il[q + k < q1 ? q + k : q];  // entry slot * NNE + a
+          base[k] = (e / NNE) * kYS + (e % NNE) * NC;
+        }
+#pragma unroll
+        for (int k = 0; k < kSumChunk; ++k)
+#pragma unroll
+          for (int c = 0; c < NC; ++c) part[k][c] = ys[base[k] + c];
+#pragma unroll
+        for (int k = 0; k < kSumChunk; ++k)
+#pragma unroll
+          for (int c = 0; c < NC; ++c) sum[c] += q + k < q1 ? part[k][c] : T(0);
       }
-      const int64_t pos = (int64_t)ts.slot_pos[nb + j] * NC;
+      const int32_t to = j < kTile ? slot01[0] : j < 2 * kTile ? slot01[1] : ts.slot_pos[nb + j];
+      const int64_t pos = (int64_t)to * NC;
 #pragma unroll
       for (int c = 0; c < NC; ++c) partial[pos + c] = sum[c];
       if constexpr (kDot) {
@@ -1035,7 +1070,6 @@ __global__ __launch_bounds__(kTile) void k_tile_assemble(const double *__restric
                                                          T *__restrict__ lin,
                                                          const T *__restrict__ geo, CgDefer dx,
                                                          double *__restrict__ dot) {
-  if (skip && *skip) return;
   extern __shared__ unsigned char lds_raw[];
   // dx (FP32 HVP): a CG step's p and x streams, run by the launch's streaming
   // workgroups on the memory bandwidth the tiles leave idle (grid of tile_grid)
@@ -1045,6 +1079,7 @@ __global__ __launch_bounds__(kTile) void k_tile_assemble(const double *__restric
       constexpr int per = kNumXcd * kDeferRows;
       const int grp = b / (per + kNumXcd), j = b - grp * (per + kNumXcd);
       if (j >= per) {
+        if (skip && *skip) return;
         cg_defer_stream(dx, (int64_t)grp * kNumXcd + (j - per),
                         (int64_t)(gridDim.x / (per + kNumXcd)) * kNumXcd);
         return;
@@ -1060,7 +1095,7 @@ __global__ __launch_bounds__(kTile) void k_tile_assemble(const double *__restric
   if (rev) tile = ts.n_tiles - 1 - tile;
   constexpr bool kDot = KIND == TATVA_HEX8 && sizeof(T) == 4;
   tile_assemble<KIND, Dens, T, MODE, GEOM, kDot>(tile, coords, quad, dens, u, v, dof_map, ts,
-                                                 partial, lds_raw, lin, geo, dot);
+                                                 partial, lds_raw, lin, geo, dot, skip);
 }
 
 // Sum of node i's tile slots (ascending tile): the tiles wrote them to the
