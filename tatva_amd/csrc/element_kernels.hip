@@ -1691,13 +1691,15 @@ extern "C" int tatva_colored_hessian(tatva_mesh *m, const tatva_density *d, cons
       constexpr int NNE = Elem<K>::NNE, NC = Dens::NC;
       using Sh = RowsShape<K, NC>;
       // node rows: as many nodes per block as its LDS holds, in whole waves
-      const size_t wave_lds = (kWave / Sh::LG) * Sh::lds_bytes(n_colors);
-      const int waves = (int)std::min<size_t>(kBlock / kWave, kTileLdsMax / wave_lds);
+      const bool affine_rows = K == TATVA_HEX8 && Dens::kLinear && m->hex_affine;
+      const size_t node_lds = Sh::lds_bytes(n_colors, !affine_rows);
+      const int waves = (int)std::min<size_t>(kBlock / kWave,
+                                              kTileLdsMax / ((kWave / Sh::LG) * node_lds));
       if (waves >= 1) {
         const int threads = waves * kWave, per = threads / Sh::LG;
         const auto launch = [&](auto affine, auto mapped) {
           k_node_rows<K, Dens, decltype(affine)::value, decltype(mapped)::value>
-              <<<grid_for(m->n_nodes, per), threads, per * Sh::lds_bytes(n_colors), s>>>(
+              <<<grid_for(m->n_nodes, per), threads, per * node_lds, s>>>(
                   m->n_nodes, n_rows, m->coords, m->conn, m->quad, m->hex_ref, dens, u, dof_map,
                   colors, n_colors, indptr, indices, m->inv_ptr, m->inv_list, data);
         };
@@ -1706,7 +1708,7 @@ extern "C" int tatva_colored_hessian(tatva_mesh *m, const tatva_density *d, cons
           else launch(affine, std::false_type{});
         };
         if constexpr (K == TATVA_HEX8 && Dens::kLinear) {
-          if (m->hex_affine) with_map(std::true_type{});
+          if (affine_rows) with_map(std::true_type{});
           else with_map(std::false_type{});
         } else {
           with_map(std::false_type{});

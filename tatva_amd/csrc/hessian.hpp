@@ -15,11 +15,12 @@
 // Hex8 element, one wave per matrix row gathering it): 64^3 Hex8 linear
 // elasticity moved 2.4 GB through that buffer and took 633 + 1735 us; here
 // each element's geometry is recomputed for each of its nodes and only the
-// matrix is written: 477 us (836 MB, 1.75 TB/s).  48^3 Hex8 Neo-Hookean 1346
-// -> 820 us, distorted linear elastic 1036 -> 373 us; 24^3 x 6 Tet4
-// Neo-Hookean 193 -> 52 us; 200^2 Tri3 linear elastic 97 -> 16 us.  Bound by
-// latency: about half of a wave's time waits on its chain of loads and LDS
-// sums, and the Hex8 kernel of a general element holds 230-300 registers (two
+// matrix is written: 433 us (656 MB, 1.5 TB/s).  48^3 Hex8 Neo-Hookean 1346
+// -> 733 us, distorted linear elastic 1036 -> 353 us; 24^3 x 6 Tet4
+// Neo-Hookean 193 -> 45 us; 200^2 Tri3 linear elastic 97 -> 15 us.  The sums are
+// LDS adds one element after another: read, added and stored, each waiting for the
+// element before, the same cases took 473, 820, 373, 52 and 16 us.  Bound by
+// latency: 60% of a wave's time waits on its chain of loads, and the Hex8 kernel of a general element holds 230-300 registers (two
 // waves a SIMD, one for Neo-Hookean; forced to three it spills and runs twice
 // as long).
 #pragma once
@@ -49,13 +50,14 @@ struct RowsShape {
   // entries per lane looked up ahead (an inner node's 27 / 15 / 7 neighbours);
   // elements whose blocks are read ahead of their sums
   static constexpr int kPre = (NC * NC * (KIND == TATVA_HEX8 ? 27 : KIND == TATVA_TET4 ? 15 : 7) + LG - 1) / LG;
-  static constexpr int kAhead = KIND == TATVA_HEX8 ? 8 : KIND == TATVA_TET4 ? 6 : 3;
-  // Hex8 stages the nodes' coordinates and state in the block buffer
-  static constexpr int kStage = KIND == TATVA_HEX8 ? 64 * 6 : 0;
-  static constexpr int kBlk = P * NC * ND > kStage ? P * NC * ND : kStage;  // doubles
-  static __host__ __device__ size_t lds_bytes(int n_colors) {
-    return ((size_t)NC * (n_colors + 1) + kBlk) * sizeof(double) +
-           (((size_t)P * ND * sizeof(int32_t) + 7) & ~size_t(7));
+  static constexpr int kAhead = KIND == TATVA_TET4 ? 6 : 3;
+  // Hex8 stages the nodes' coordinates and state (general elements), simplices
+  // their blocks and the blocks' colors
+  static constexpr int kBlk = KIND == TATVA_HEX8 ? 64 * 6 : P * NC * ND;  // doubles
+  static constexpr int kTab = KIND == TATVA_HEX8 ? 0 : P * ND;            // int32
+  static __host__ __device__ size_t lds_bytes(int n_colors, bool staged) {
+    return ((size_t)NC * (n_colors + 1) + (staged ? kBlk : 0)) * sizeof(double) +
+           (((size_t)kTab * sizeof(int32_t) + 7) & ~size_t(7));
   }
 };
 
@@ -323,11 +325,18 @@ __device__ __forceinline__ void hex8_affine_row_blocks(const double (&X)[3], int
   }
 }
 
+// p[0] += v on LDS.  A wave's LDS operations run in their order, so sums added one
+// instruction after another have one order without a wait between them.
+__device__ __forceinline__ void lds_add(double *p, double v) {
+  __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+}
+
 // One group of LG lanes per node.  The group's compressed Jacobian rows
 // J[c][color] live in LDS (the last slot takes constrained columns); the
-// node's elements are taken P at a time in ascending order, their blocks
-// written to LDS and added to J one element after another (inside an element
-// every column has its own color), so the sums have one order.  Then
+// node's elements are taken P at a time in ascending order, their blocks added to
+// J one element after another (inside an element every column has its own color;
+// a simplex's block goes through LDS to all lanes of the group first), so the
+// sums have one order.  Then
 // data[k] = J[c][colors[indices[k]]] (sparse/base.py:173).
 // The loads are issued level by level (the node's rows and elements, their row
 // ranges and element nodes, column indices and node data, colors), none behind
@@ -354,7 +363,7 @@ __global__ __launch_bounds__(kBlock) void k_node_rows(
   const int64_t node =
       xcd_block(blockIdx.x, gridDim.x) * (blockDim.x / LG) + threadIdx.x / LG;
   if (node >= n_nodes) return;
-  unsigned char *mine = lds_raw + (size_t)(threadIdx.x / LG) * Sh::lds_bytes(n_colors);
+  unsigned char *mine = lds_raw + (size_t)(threadIdx.x / LG) * Sh::lds_bytes(n_colors, !AFFINE);
   const int ncol = n_colors + 1;
   double *Jr = reinterpret_cast<double *>(mine);
   double *blk = Jr + (size_t)NC * ncol;
@@ -450,7 +459,6 @@ __global__ __launch_bounds__(kBlock) void k_node_rows(
       packed = element_of(p0 + P);
       nodes_of(packed);
     }
-    wave_lds_sync();  // the blocks of the chunk before have been read
     if constexpr (kHex) {
       double v[NC * NC];
       if constexpr (AFFINE) {
@@ -466,46 +474,48 @@ __global__ __launch_bounds__(kBlock) void k_node_rows(
         hex8_row_blocks<Dens>(blk + pl * 48, hex_bin(a), quad, de, s, v);
         wave_lds_sync();  // the staged nodes have been read
       }
+      // element after element, its eight lanes adding their blocks
+      for (int p = 0; p < cnt; ++p)
+        if (pl == p) {
 #pragma unroll
-      for (int k = 0; k < NC; ++k) ctab[pl * ND + s * NC + k] = col[k];
+          for (int c = 0; c < NC; ++c)
 #pragma unroll
-      for (int c = 0; c < NC; ++c)
-#pragma unroll
-        for (int k = 0; k < NC; ++k) blk[(pl * NC + c) * ND + s * NC + k] = v[c * NC + k];
+            for (int k = 0; k < NC; ++k) lds_add(Jr + c * ncol + col[k], v[c * NC + k]);
+        }
     } else {
       double v[NC][ND];
       simplex_row_blocks<KIND, Dens>(X, ue, a, quad, de, v);
+      wave_lds_sync();  // the blocks of the chunk before have been read
 #pragma unroll
       for (int i = 0; i < ND; ++i) ctab[pl * ND + i] = col[i];
 #pragma unroll
       for (int c = 0; c < NC; ++c)
 #pragma unroll
         for (int i = 0; i < ND; ++i) blk[(pl * NC + c) * ND + i] = v[c][i];
-    }
-    wave_lds_sync();
-    // one element after another; its values are read ahead of the sums
-    constexpr int R = (NC * ND + LG - 1) / LG, W = Sh::kAhead;
-    for (int pb = 0; pb < cnt; pb += W) {
-      double val[W][R];
-      int32_t dst[W][R];
-#pragma unroll
-      for (int pi = 0; pi < W; ++pi)
-#pragma unroll
-        for (int rr = 0; rr < R; ++rr) {
-          const int p = pb + pi < cnt ? pb + pi : 0;
-          const int i = rr * LG + lane < NC * ND ? rr * LG + lane : 0;
-          const int c = i / ND, j = i - c * ND;
-          val[pi][rr] = blk[p * NC * ND + i];
-          dst[pi][rr] = c * ncol + ctab[p * ND + j];
-        }
       wave_lds_sync();
+      // element after element, its values taken by the group's lanes; those of
+      // some elements are read ahead of their sums
+      constexpr int R = (NC * ND + LG - 1) / LG, W = Sh::kAhead;
+      for (int pb = 0; pb < cnt; pb += W) {
+        double val[W][R];
+        int32_t dst[W][R];
 #pragma unroll
-      for (int pi = 0; pi < W; ++pi) {
-        if (pb + pi >= cnt) break;
+        for (int pi = 0; pi < W; ++pi)
 #pragma unroll
-        for (int rr = 0; rr < R; ++rr)
-          if (rr * LG + lane < NC * ND) Jr[dst[pi][rr]] += val[pi][rr];
-        wave_lds_sync();
+          for (int rr = 0; rr < R; ++rr) {
+            const int p = pb + pi < cnt ? pb + pi : 0;
+            const int i = rr * LG + lane < NC * ND ? rr * LG + lane : 0;
+            const int c = i / ND, j = i - c * ND;
+            val[pi][rr] = blk[p * NC * ND + i];
+            dst[pi][rr] = c * ncol + ctab[p * ND + j];
+          }
+#pragma unroll
+        for (int pi = 0; pi < W; ++pi) {
+          if (pb + pi >= cnt) break;
+#pragma unroll
+          for (int rr = 0; rr < R; ++rr)
+            if (rr * LG + lane < NC * ND) lds_add(Jr + dst[pi][rr], val[pi][rr]);
+        }
       }
     }
   }
