@@ -1697,21 +1697,23 @@ extern "C" int tatva_colored_hessian(tatva_mesh *m, const tatva_density *d, cons
                                               kTileLdsMax / ((kWave / Sh::LG) * node_lds));
       if (waves >= 1) {
         const int threads = waves * kWave, per = threads / Sh::LG;
-        const auto launch = [&](auto affine, auto mapped) {
-          k_node_rows<K, Dens, decltype(affine)::value, decltype(mapped)::value>
+        const auto launch = [&](auto geom, auto mapped) {
+          k_node_rows<K, Dens, decltype(geom)::value, decltype(mapped)::value>
               <<<grid_for(m->n_nodes, per), threads, per * node_lds, s>>>(
                   m->n_nodes, n_rows, m->coords, m->conn, m->quad, m->hex_ref, dens, u, dof_map,
                   colors, n_colors, indptr, indices, m->inv_ptr, m->inv_list, data);
         };
-        const auto with_map = [&](auto affine) {
-          if (dof_map) launch(affine, std::true_type{});
-          else launch(affine, std::false_type{});
+        const auto with_map = [&](auto geom) {
+          if (dof_map) launch(geom, std::true_type{});
+          else launch(geom, std::false_type{});
         };
+        using std::integral_constant;
         if constexpr (K == TATVA_HEX8 && Dens::kLinear) {
-          if (affine_rows) with_map(std::true_type{});
-          else with_map(std::false_type{});
+          if (m->hex_box) with_map(integral_constant<int, kGeomBox>{});
+          else if (affine_rows) with_map(integral_constant<int, kGeomAffine>{});
+          else with_map(integral_constant<int, kGeomGeneral>{});
         } else {
-          with_map(std::false_type{});
+          with_map(integral_constant<int, kGeomGeneral>{});
         }
         TATVA_CHECK_LAUNCH();
         return TATVA_OK;

@@ -15,12 +15,15 @@
 // Hex8 element, one wave per matrix row gathering it): 64^3 Hex8 linear
 // elasticity moved 2.4 GB through that buffer and took 633 + 1735 us; here
 // each element's geometry is recomputed for each of its nodes and only the
-// matrix is written: 433 us (656 MB, 1.5 TB/s).  48^3 Hex8 Neo-Hookean 1346
-// -> 733 us, distorted linear elastic 1036 -> 353 us; 24^3 x 6 Tet4
-// Neo-Hookean 193 -> 45 us; 200^2 Tri3 linear elastic 97 -> 15 us.  The sums are
+// matrix is written: 396 us (656 MB, 1.7 TB/s).  48^3 Hex8 Neo-Hookean 1346
+// -> 733 us, distorted linear elastic 1036 -> 344 us; 24^3 x 6 Tet4
+// Neo-Hookean 193 -> 43 us; 200^2 Tri3 linear elastic 97 -> 15 us.  The sums are
 // LDS adds one element after another: read, added and stored, each waiting for the
-// element before, the same cases took 473, 820, 373, 52 and 16 us.  Bound by
-// latency: 60% of a wave's time waits on its chain of loads, and the Hex8 kernel of a general element holds 230-300 registers (two
+// element before, the same cases took 473, 820, 373, 52 and 16 us.  The rows of
+// boxes are bound by their ~500 vector instructions a wave (half of the time) and
+// 72 LDS adds (40%); a wave waits 60% of its life on its chain of loads, so six
+// waves a SIMD matter (loading the next node's data under this one's work cost
+// half of them: 505 us; forced to eight waves it spills: 628).  The Hex8 kernel of a general element holds 230-300 registers (two
 // waves a SIMD, one for Neo-Hookean; forced to three it spills and runs twice
 // as long).
 #pragma once
@@ -325,6 +328,39 @@ __device__ __forceinline__ void hex8_affine_row_blocks(const double (&X)[3], int
   }
 }
 
+// The same for a box along the axes: the Jacobian is the diagonal of half the
+// edges, so the block is det J M_ab[k][l] / (J_k J_l): fewer registers than the
+// general parallelepiped's (six waves a SIMD instead of five, 64^3 linear elastic
+// 433 -> 396 us).
+template <class Dens>
+__device__ __forceinline__ void hex8_box_row_blocks(const double (&X)[3], int ja,
+                                                    const double *__restrict__ ref,
+                                                    const Dens &dens, int s,
+                                                    double (&out)[Dens::NC * Dens::NC]) {
+  constexpr int NC = Dens::NC;
+  double m[9];
+#pragma unroll
+  for (int i = 0; i < 9; ++i)
+    if (NC > 1 || i % 4 == 0) m[i] = ref[i * 64 + ja * 8 + s];
+  // (lane s ^ 7 is across the edge along z: its x and y are not looked at)
+  const double o[3] = {dpp_move<kDppXor1>(X[0]), dpp_move<kDppXor2>(X[1]),
+                       dpp_move<kDppHalfMirror>(X[2])};
+  double J[3];
+#pragma unroll
+  for (int c = 0; c < 3; ++c) J[c] = 0.5 * ((s >> c & 1) ? X[c] - o[c] : o[c] - X[c]);
+  const double det = J[0] * J[1] * J[2], r = 1.0 / det;
+  const double h[3] = {J[1] * J[2] * r, J[0] * J[2] * r, J[0] * J[1] * r};
+  if constexpr (NC == 1) {
+    out[0] = det * (h[0] * h[0] * m[0] + h[1] * h[1] * m[4] + h[2] * h[2] * m[8]);
+  } else {
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+#pragma unroll
+      for (int k = 0; k < 3; ++k) out[c * 3 + k] = det * h[c] * h[k] * m[c * 3 + k];
+    dens.row_block(out);
+  }
+}
+
 // p[0] += v on LDS.  A wave's LDS operations run in their order, so sums added one
 // instruction after another have one order without a wait between them.
 __device__ __forceinline__ void lds_add(double *p, double v) {
@@ -343,7 +379,7 @@ __device__ __forceinline__ void lds_add(double *p, double v) {
 // a branch: a lane without work reads a valid address and drops the value.
 // Behind branches each load waited for the one before (64^3 Hex8 linear
 // elasticity, general geometry: 1540 us against 1130 us).
-template <int KIND, class Dens, bool AFFINE, bool MAPPED>
+template <int KIND, class Dens, int GEOM, bool MAPPED>
 __global__ __launch_bounds__(kBlock) void k_node_rows(
     int64_t n_nodes, int64_t n_rows, const double *__restrict__ coords,
     const int32_t *__restrict__ conn, QuadRule quad, const double *__restrict__ ref, Dens dens,
@@ -356,6 +392,7 @@ __global__ __launch_bounds__(kBlock) void k_node_rows(
                 P = Sh::P;
   constexpr bool kHex = KIND == TATVA_HEX8;
   constexpr int NL = kHex ? 1 : NNE;  // nodes a lane loads
+  constexpr bool AFFINE = GEOM != kGeomGeneral;
   static_assert(!AFFINE || (kHex && Dens::kLinear), "constant blocks");
   extern __shared__ unsigned char lds_raw[];
   const int lane = threadIdx.x % LG;
@@ -369,9 +406,9 @@ __global__ __launch_bounds__(kBlock) void k_node_rows(
   double *blk = Jr + (size_t)NC * ncol;
   int32_t *ctab = reinterpret_cast<int32_t *>(blk + Sh::kBlk);
   // level 1: the node's rows and element range
-  int64_t row[NC];
+  int32_t row[NC];
 #pragma unroll
-  for (int c = 0; c < NC; ++c) row[c] = MAPPED ? (int64_t)dof_map[node * NC + c] : node * NC + c;
+  for (int c = 0; c < NC; ++c) row[c] = MAPPED ? dof_map[node * NC + c] : (int32_t)(node * NC + c);
   const int32_t b0 = inv_ptr[node], b1 = inv_ptr[node + 1];
   // level 2: row ranges, this lane's element.  The rows' entries are flattened:
   // entry t of the group is data[at + t] of row c, off <= t < the next off.
@@ -383,7 +420,7 @@ __global__ __launch_bounds__(kBlock) void k_node_rows(
   int32_t packed = element_of(b0);
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
-    const int64_t r = row[c] >= 0 && row[c] < n_rows ? row[c] : 0;
+    const int32_t r = row[c] >= 0 && row[c] < n_rows ? row[c] : 0;
     k0[c] = indptr[r];
     off1[c] = indptr[r + 1];
   }
@@ -436,14 +473,13 @@ __global__ __launch_bounds__(kBlock) void k_node_rows(
     const Dens de = dens.at(packed >> 3);
     // level 4: node data
     double X[NL][D], ue[NL][NC];
-    int64_t sd[NL * NC];
-    int32_t col[NL * NC];
+    int32_t sd[NL * NC], col[NL * NC];
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
 #pragma unroll
       for (int k = 0; k < NC; ++k) {
         const int64_t dof = (int64_t)g[i] * NC + k;
-        sd[i * NC + k] = MAPPED ? (int64_t)dof_map[dof] : dof;
+        sd[i * NC + k] = MAPPED ? dof_map[dof] : (int32_t)dof;
         ue[i][k] = Dens::kLinear ? 0.0 : u[dof];
       }
 #pragma unroll
@@ -461,7 +497,9 @@ __global__ __launch_bounds__(kBlock) void k_node_rows(
     }
     if constexpr (kHex) {
       double v[NC * NC];
-      if constexpr (AFFINE) {
+      if constexpr (GEOM == kGeomBox) {
+        hex8_box_row_blocks<Dens>(X[0], hex_bin(a), ref, de, s, v);
+      } else if constexpr (AFFINE) {
         hex8_affine_row_blocks<Dens>(X[0], hex_bin(a), ref, de, s, v);
       } else {
 #pragma unroll
