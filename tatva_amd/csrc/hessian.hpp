@@ -23,9 +23,9 @@
 // boxes are bound by their ~500 vector instructions a wave (half of the time) and
 // 72 LDS adds (40%); a wave waits 60% of its life on its chain of loads, so six
 // waves a SIMD matter (loading the next node's data under this one's work cost
-// half of them: 505 us; forced to eight waves it spills: 628).  The Hex8 kernel of a general element holds 230-300 registers (two
-// waves a SIMD, one for Neo-Hookean; forced to three it spills and runs twice
-// as long).
+// half of them: 505 us; forced to eight waves it spills: 628).  The Hex8 kernel
+// of a general element holds 230-300 registers (two waves a SIMD, one for
+// Neo-Hookean; forced to three it spills and runs twice as long).
 #pragma once
 
 #include <hip/hip_runtime.h>

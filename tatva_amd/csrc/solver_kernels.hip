@@ -1052,6 +1052,173 @@ static PcgParts parts_at(char *w, const WsLayout &L) {
                   b + 4 * kMaxReduceBlocks, b + 5 * kMaxReduceBlocks};
 }
 
+// ------------------------------------------------------- small systems ----
+//
+// A sliced-ELL system of at most kSmallRows rows runs its iterations in one
+// workgroup: a launch and two kernel boundaries per iteration cost more than the
+// work of such a system (64^2 Poisson, 3969 rows of 7: 8.2 us per iteration as two
+// kernels, 2.7 us here).  Lane l of wave w holds the rows of slices w, w + 16, ...:
+// their first kSmallLen entries, s and D^-1 in registers (longer rows read the rest
+// from the last-level caches), u, p, x and 1 / D^-1 in LDS.  What bounds it: the FP64
+// instructions of eight waves on one CU and two barriers an iteration.  Seven entries
+// are a node's neighbours and itself in a triangulation; eight spill (3.9 us), with
+// six the seventh comes from memory (3.2).  Eight waves of 256 registers, not sixteen
+// of 128 (3.9 us: spills, and every wave repeats the scalars).  The host takes it for
+// up to kSmallRows rows (128 KB of LDS) when the slices' longest rows are kSmallMean
+// on average, so that an iteration streams little.  The same recurrences
+// and tests as k_sell_spmv and k_cg_step<double>, with one sum over the workgroup per
+// iteration; r.u and r.r of the last step pass from launch to launch in the parts.
+constexpr int kSmallThreads = 512, kSmallWaves = kSmallThreads / kWave;
+constexpr int kSmallRows = 4096, kSmallSlices = kSmallRows / kSmallThreads, kSmallLen = 7;
+constexpr int kSmallMean = 8;
+constexpr int kSmallIters = 256;  // iterations per launch, at least
+static_assert(kSellRows == kWave, "a row per lane");
+
+__global__ __launch_bounds__(kSmallThreads) void k_pcg_small(
+    int n, int nsl, const int64_t *__restrict__ soff, const int32_t *__restrict__ cols,
+    const double *__restrict__ vals, double *__restrict__ x, double *__restrict__ u,
+    double *__restrict__ p, double *__restrict__ s, const double *__restrict__ dinv,
+    double *__restrict__ part_g, double *__restrict__ part_rr, int n_part, int iters,
+    PcgState *__restrict__ st) {
+  if (st->done) return;
+  __shared__ double us[kSmallRows], ps[kSmallRows], xs[kSmallRows], rd[kSmallRows];
+  __shared__ double red[2][3][kSmallWaves];
+  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+  const bool begun = st->it[1] > 0;  // before iteration 0, p and s hold no values
+  double v[kSmallSlices][kSmallLen], sr[kSmallSlices], di[kSmallSlices];
+  uint32_t c[kSmallSlices][(kSmallLen + 1) / 2];  // two columns each, as bytes into us
+  int at[kSmallSlices], len[kSmallSlices];  // uniform
+#pragma unroll
+  for (int k = 0; k < kSmallSlices; ++k) {
+    const int sl = wave + k * kSmallWaves, row = sl * kWave + lane;
+    const int64_t o = soff[sl < nsl ? sl : 0], e = soff[sl < nsl ? sl + 1 : 0];
+    at[k] = __builtin_amdgcn_readfirstlane((int)o) * kSellRows;
+    const int J = len[k] = __builtin_amdgcn_readfirstlane((int)(e - o));
+#pragma unroll
+    for (int j = 0; j < kSmallLen; ++j) {
+      const int pos = J > 0 ? at[k] + (j < J ? j : J - 1) * kSellRows : 0;
+      const double val = vals[pos + lane];
+      const uint32_t col = 8u * (uint32_t)(j < J ? cols[pos + lane] : row);
+      v[k][j] = j < J ? val : 0.0;
+      c[k][j / 2] = j & 1 ? c[k][j / 2] | col << 16 : col;
+    }
+    const bool on = row < n;
+    const int g = on ? row : 0;
+    const double gu = u[g], gp = p[g], gx = x[g], gs = s[g], gd = dinv[g];
+    us[row] = on ? gu : 0.0;
+    ps[row] = on && begun ? gp : 0.0;
+    xs[row] = on ? gx : 0.0;
+    sr[k] = on && begun ? gs : 0.0;
+    di[k] = on ? gd : 0.0;
+    rd[row] = on && gd != 0.0 ? 1.0 / gd : 0.0;
+  }
+  double sg = (int)threadIdx.x < n_part ? part_g[threadIdx.x] : 0.0;
+  double srr = (int)threadIdx.x < n_part ? part_rr[threadIdx.x] : 0.0;
+  int iter = st->it[1];
+  // beta gamma / alpha_old = beta^2 denom_old: a division less
+  double gamma_old = st->gamma[1], denom_old = begun ? gamma_old / st->alpha[1] : 0.0;
+  double rr_last = st->rr;
+  const double tol2 = st->tol2;
+  const int maxiter = st->maxiter;
+  int flip = 0;
+  // the workgroup's sums of three values, in every thread (one barrier: the buffers
+  // alternate, and a buffer is read before the barrier that its next writes follow).
+  // Second stage: the waves' shares of value g sit in eight lanes.
+  static_assert(kSmallWaves == 8, "a wave's share per lane of half a row");
+  const auto sum3 = [&](double &a, double &b, double &d) {
+    a = wave_sum(a);
+    b = wave_sum(b);
+    d = wave_sum(d);
+    if (lane < 3) red[flip][lane][wave] = lane == 0 ? a : lane == 1 ? b : d;
+    __syncthreads();
+    double t = red[flip][lane < 24 ? lane / 8 : 0][lane % 8];
+    t += dpp_move<kDppXor1>(t);
+    t += dpp_move<kDppXor2>(t);
+    t += dpp_move<kDppHalfMirror>(t);
+    a = read_lane(t, 0);
+    b = read_lane(t, 8);
+    d = read_lane(t, 16);
+    flip ^= 1;
+  };
+  int status = -1;
+  __syncthreads();
+  for (int i = 0; i < iters; ++i) {
+    double w[kSmallSlices], delta = 0.0;
+#pragma unroll
+    for (int k = 0; k < kSmallSlices; ++k) {
+      const int row = (wave + k * kSmallWaves) * kWave + lane;
+      double a = 0.0;
+#pragma unroll
+      for (int j = 0; j < kSmallLen; ++j)
+        a += v[k][j] * *reinterpret_cast<const double *>(
+                           reinterpret_cast<const char *>(us) +
+                           (j & 1 ? c[k][j / 2] >> 16 : c[k][j / 2] & 0xffffu));
+      for (int j = kSmallLen; j < len[k]; ++j) {
+        const int pos = at[k] + j * kSellRows + lane;
+        a += vals[pos] * us[cols[pos]];
+      }
+      w[k] = a;
+      delta += a * us[row];
+    }
+    double gamma = sg, rr = srr;
+    sum3(gamma, rr, delta);
+    const bool first = iter == 0;
+    const double beta = first ? 0.0 : gamma / gamma_old;
+    const double denom = delta - beta * beta * denom_old;
+    const bool converged = rr <= tol2, spent = iter >= maxiter;
+    const bool bad = !(denom > 0.0) || !isfinite(denom) || !isfinite(gamma) || !isfinite(rr);
+    rr_last = rr;
+    if (converged || spent || bad) {
+      status = converged ? TATVA_OK : spent ? TATVA_ENOTCONV : TATVA_EBREAKDOWN;
+      break;
+    }
+    const double alpha = gamma / denom;
+    sg = 0.0;
+    srr = 0.0;
+#pragma unroll
+    for (int k = 0; k < kSmallSlices; ++k) {
+      const int row = (wave + k * kSmallWaves) * kWave + lane;
+      const double pn = us[row] + beta * ps[row];
+      sr[k] = w[k] + beta * sr[k];
+      const double un = us[row] - alpha * (di[k] * sr[k]), ri = un * rd[row];
+      ps[row] = pn;
+      xs[row] += alpha * pn;
+      us[row] = un;
+      sg += ri * un;
+      srr += ri * ri;
+    }
+    gamma_old = gamma;
+    denom_old = denom;
+    ++iter;
+    __syncthreads();
+  }
+#pragma unroll
+  for (int k = 0; k < kSmallSlices; ++k) {
+    const int row = (wave + k * kSmallWaves) * kWave + lane;
+    if (row < n) {
+      x[row] = xs[row];
+      u[row] = us[row];
+      p[row] = ps[row];
+      s[row] = sr[k];
+    }
+  }
+  double unused = 0.0;
+  sum3(sg, srr, unused);
+  if ((int)threadIdx.x < n_part) {
+    part_g[threadIdx.x] = threadIdx.x == 0 ? sg : 0.0;
+    part_rr[threadIdx.x] = threadIdx.x == 0 ? srr : 0.0;
+  }
+  if (threadIdx.x == 0) {
+    st->alpha[1] = gamma_old / denom_old;
+    st->gamma[1] = gamma_old;
+    st->it[1] = iter;
+    st->iter = iter;
+    st->rr = rr_last;
+    if (status >= 0) st->status = status;
+    if (status >= 0) st->done = 1;
+  }
+}
+
 // Runs captured chunks until the device state reports done; fills stats.
 // With profiling, the graph holds the chunk minus its first operator
 // application, which `sampled_op` launches eagerly on the same stream between
@@ -1377,6 +1544,14 @@ extern "C" int tatva_pcg_csr(int64_t n, int64_t nnz, const int32_t *indptr,
                                             P.rz(q ^ 1), P.rr(q ^ 1), P.rz(q), P.rr(q), q, st);
     return TATVA_OK;
   };
+  const bool small = nblk == 1 && !profiling && n <= kSmallRows && gv <= kSmallThreads &&
+                     sv_ell.steps <= kSmallMean * sv_ell.nsl;
+  const std::function<int(int, bool)> run_small = [&](int, bool) -> int {
+    k_pcg_small<<<1, kSmallThreads, 0, s>>>((int)n, (int)sv_ell.nsl, sv_ell.soff, sv_ell.cols,
+                                            sv_ell.vals, x, u, p, sv, dinv, P.rz(1), P.rr(1), gv,
+                                            std::max(chunk, kSmallIters), st);
+    return TATVA_OK;
+  };
   GraphKey key{};
   key.ws = workspace;
   key.a = indptr;
@@ -1390,7 +1565,8 @@ extern "C" int tatva_pcg_csr(int64_t n, int64_t nnz, const int32_t *indptr,
   key.i0 = nblk;
   key.i1 = chunk;
   key.i2 = profiling ? 1 : 0;
-  rc = chunk_graph(s, chunk, step, profiling, key, res->csr);
+  key.i3 = small ? 1 : 0;
+  rc = chunk_graph(s, small ? 1 : chunk, small ? run_small : step, profiling, key, res->csr);
   if (rc == TATVA_OK)
     rc = run_chunks(res, res->csr.exec, st, maxiter, chunk, profiling, sampled_spmv, stats,
                     sum_shares);

@@ -271,3 +271,38 @@ def test_stiffness_diagonal(form, density):
     u32 = torch.as_tensor(u, dtype=torch.float32, device="cuda")
     ref = prob.hessian_diag(to_np(u32).astype(float))
     assert rel_err(to_np(E.hessian_diag(u32, dtype=torch.float32)), ref) < 2e-6
+
+
+@pytest.mark.parametrize("longer", [False, True], ids=["short-rows", "a-longer-row"])
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 1023, 1025, 4033, 4096, 4097])
+def test_small_csr_pcg(n, longer):
+    """Systems solved in one workgroup (at most 4096 rows of 8 entries on average), a
+    row longer than the registers hold, and the first size past the limit; stopped by
+    the tolerance (on a recurrence residual of 1e-12 of b; FP64 rounding over a few
+    hundred iterations of a matrix of condition 1e3 stays far below 1e-9) and, more
+    launches than one, by the iteration limit."""
+    from tatva_amd import solvers
+
+    rng = np.random.default_rng(n)
+    A = sps.lil_matrix((n, n))
+    for value, off in ((-1.0, 1), (-0.5, 2), (-0.25, 60)):
+        if off < n:
+            A += sps.diags([value], [off], shape=(n, n))
+    A = A.tolil()
+    if longer and n > 40:
+        A[7, 12:38:2] = -0.03
+    A = (A + A.T).tocsr()
+    A = (A + sps.diags(np.asarray(-A.sum(axis=1)).ravel() + 0.003)).tocsr()
+    A.sort_indices()
+    K = sparse.ColoredMatrix.from_csr(A)
+    b = rng.standard_normal(n)
+    x, info = solvers.pcg(K, b, tol=1e-12)
+    assert info.converged
+    assert np.linalg.norm(b - A @ to_np(x)) < 1e-9 * np.linalg.norm(b)
+    x0 = rng.standard_normal(n)
+    x, info = solvers.pcg(K, A @ x0, x0=x0, tol=1e-12)
+    assert info.iterations <= 1 and rel_err(to_np(x), x0) < 1e-9
+    if n > 1000:
+        x, info = solvers.pcg(K, b, tol=0.0, maxiter=300)
+        assert not info.converged and info.iterations == 300
+        assert np.isfinite(to_np(x)).all()
