@@ -74,7 +74,7 @@ enum {
 // Jacobian is diagonal, so a gradient takes three products instead of nine of
 // three terms, and the geometry is three edge lengths (against kGeomAffine /
 // kGeomCache: 160^3 Neo-Hookean FP32 product 341 -> 287 us, in the PCG 299 -> 268
-// us; 64^3 linear elastic in the PCG 18.8 -> 17.0 us; 64^3 Neo-Hookean FP64
+// us, 234 with the tile's loads before its staging; 64^3 linear elastic in the PCG 18.8 -> 17.0 us; 64^3 Neo-Hookean FP64
 // 47.5 -> 42.8 us).
 enum { kGeomGeneral = 0, kGeomAffine = 1, kGeomCache = 2, kGeomBox = 3, kGeomBoxCache = 4 };
 constexpr bool geom_cached(int geom) { return geom == kGeomCache || geom == kGeomBoxCache; }

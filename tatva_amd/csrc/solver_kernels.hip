@@ -340,94 +340,6 @@ static int sell_grid(int64_t n) {
 
 // ------------------------------------------------------------ PCG steps ----
 
-// K1 for a matrix-free operator: the block's share of p.Ap.
-template <class T>
-__global__ __launch_bounds__(kBlock) void k_pcg_dot(int64_t n, const T *__restrict__ p,
-                                                    const T *__restrict__ Ap,
-                                                    double *__restrict__ part_pap,
-                                                    const PcgState *__restrict__ st) {
-  if (st->done) return;
-  double dot = 0.0;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x)
-    dot += (double)p[i] * (double)Ap[i];
-  dot = block_sum(dot);
-  if (threadIdx.x == 0) part_pap[blockIdx.x] = dot;
-}
-
-// K2: alpha, x and r updates, shares of r.z and r.r for parity q.
-template <class T>
-__global__ __launch_bounds__(kBlock) void k_pcg_update(int64_t n, T *__restrict__ x, T *__restrict__ r,
-                                                       const T *__restrict__ p,
-                                                       const T *__restrict__ Ap,
-                                                       const T *__restrict__ dinv,
-                                                       const double *__restrict__ part_pap, int n_pap,
-                                                       const double *__restrict__ part_rz_old,
-                                                       double *__restrict__ part_rz_new,
-                                                       double *__restrict__ part_rr_new,
-                                                       PcgState *__restrict__ st) {
-  if (st->done) return;
-  const int iter = st->iter;
-  const double pap = sum_partials(part_pap, n_pap);
-  const double rz = sum_partials(part_rz_old, gridDim.x);
-  if (!(pap > 0.0) || !isfinite(pap) || iter >= st->maxiter) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-      st->done = 1;
-      st->status = (iter >= st->maxiter) ? TATVA_ENOTCONV : TATVA_EBREAKDOWN;
-    }
-    return;
-  }
-  const T alpha = T(rz / pap);
-  double srz = 0.0, srr = 0.0;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    x[i] += alpha * p[i];
-    const T ri = r[i] - alpha * Ap[i];
-    r[i] = ri;
-    srz += (double)ri * (double)(dinv[i] * ri);
-    srr += (double)ri * (double)ri;
-  }
-  srz = block_sum(srz);
-  srr = block_sum(srr);
-  if (threadIdx.x == 0) {
-    part_rz_new[blockIdx.x] = srz;
-    part_rr_new[blockIdx.x] = srr;
-  }
-}
-
-// K3: convergence test and p = D^-1 r + beta p.
-template <class T>
-__global__ __launch_bounds__(kBlock) void k_pcg_pupdate(int64_t n, T *__restrict__ p,
-                                                        const T *__restrict__ r,
-                                                        const T *__restrict__ dinv,
-                                                        const double *__restrict__ part_rz_old,
-                                                        const double *__restrict__ part_rz_new,
-                                                        const double *__restrict__ part_rr_new,
-                                                        PcgState *__restrict__ st) {
-  if (st->done) return;
-  const double rz_old = sum_partials(part_rz_old, gridDim.x);
-  const double rz_new = sum_partials(part_rz_new, gridDim.x);
-  const double rr = sum_partials(part_rr_new, gridDim.x);
-  const bool converged = rr <= st->tol2;
-  const bool bad = !isfinite(rr) || !isfinite(rz_new);
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    st->iter += 1;
-    st->rr = rr;
-    if (converged) {
-      st->done = 1;
-      st->status = TATVA_OK;
-    } else if (bad) {
-      st->done = 1;
-      st->status = TATVA_EBREAKDOWN;
-    }
-  }
-  if (converged || bad) return;
-  const T beta = T(rz_new / rz_old);
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x)
-    p[i] = dinv[i] * r[i] + beta * p[i];
-}
-
 // Vectors of the CG step: FP32 in 16-byte vectors of 4 (a clang vector type,
 // which the non-temporal store builtin takes: 115 -> 94 us per step at n =
 // 12.4 M), FP64 one element at a time (in 16-byte vectors of 2 it measured
@@ -1695,8 +1607,8 @@ extern "C" int tatva_pcg_matfree_f32(tatva_mesh *m, const tatva_density *d, cons
   float *lin = lin_bytes ? reinterpret_cast<float *>(wsb + matfree_lin_offset(m, nv)) : nullptr;
   // affine Hex8: the elements' J^-1 and det J are written once per solve and
   // read by every product instead of the coordinates (option, on by default: the
-  // 64^3 linear elasticity product 22.1 -> 19.9 us, the 160^3 Neo-Hookean one
-  // unchanged at 334 us)
+  // 64^3 linear elasticity product of parallelepipeds 22.1 -> 19.9 us when it came;
+  // loaded before the staging, the 160^3 Neo-Hookean one of boxes 244 -> 234 us)
   float *geo = matfree_geo_bytes(m)
                    ? reinterpret_cast<float *>(wsb + matfree_lin_offset(m, nv) + lin_bytes)
                    : nullptr;

@@ -341,15 +341,25 @@ class Lifter:
         """``lift`` starting from zeros (base.py:223-229)."""
         self._require_device_kernels()
         t = nat.torch()
-        out = t.zeros(self.size, dtype=t.float64, device=nat.device())
-        self._scatter(u_reduced, out)
+        ur = self._reduced_vec(u_reduced)
+        out = t.empty(self.size, dtype=t.float64, device=ur.device)
+        # zeros and free dofs in one pass (a fill and a scatter are two launches)
+        if self.size_reduced:
+            nat.check(nat.lib().tatva_lift_map(self.size, nat.dptr(self.dof_map_device()),
+                                               nat.dptr(ur), nat.dptr(out), nat.stream()))
+        else:
+            out.zero_()
         self.apply_constraints(out)
         return out
 
-    def _scatter(self, u_reduced, out):
+    def _reduced_vec(self, u_reduced):
         ur = nat.to_device(u_reduced).reshape(-1).contiguous()
         if ur.shape[0] != self.size_reduced:
             raise LifterError(f"u_reduced must have {self.size_reduced} entries, got {ur.shape[0]}")
+        return ur
+
+    def _scatter(self, u_reduced, out):
+        ur = self._reduced_vec(u_reduced)
         nat.check(nat.lib().tatva_scatter_free(self.size_reduced, nat.dptr(self.free_device()),
                                                nat.dptr(ur), nat.dptr(out), nat.stream()))
 

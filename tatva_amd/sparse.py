@@ -347,6 +347,11 @@ def linearized_jacfwd(fn, colored_matrix: ColoredMatrix, *, color_batch_size: in
     asm = _HessianAssembler(fn, colored_matrix)
 
     def _wrapped(u):
+        if asm.reduced:
+            en = fn.energy
+            uf = en.lift(u)  # once for both
+            return (en.residual_full_state(uf),
+                    replace(colored_matrix, data=asm.assemble_full_state(uf, en.lifter)))
         return fn(u), replace(colored_matrix, data=asm(u))
 
     _wrapped.assembler = asm

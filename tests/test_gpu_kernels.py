@@ -306,3 +306,35 @@ def test_small_csr_pcg(n, longer):
         x, info = solvers.pcg(K, b, tol=0.0, maxiter=300)
         assert not info.converged and info.iterations == 300
         assert np.isfinite(to_np(x)).all()
+
+
+@pytest.mark.parametrize("case", ["none", "fixed", "values", "all", "periodic"])
+def test_lift_in_one_pass_and_once_per_jvp(case):
+    """lift_from_zeros against its definition (exact), with no, some and only
+    constrained dofs; jvp and linearized_jacfwd, which lift once, against the separate
+    calls (the same kernels on the same state: exact)."""
+    mesh = ta.Mesh.unit_square(4, 3)
+    n, rng = mesh.n_nodes, np.random.default_rng(0)
+    left, right = (np.where(mesh.coords[:, 0] == x)[0] for x in (0.0, 1.0))
+    ref = np.zeros(n)
+    cons = {"none": [], "fixed": [lifter.Fixed(left, 0.5)],
+            "values": [lifter.Fixed(left, np.arange(left.size) + 1.0)],
+            "all": [lifter.Fixed(np.arange(n), 2.0)],
+            "periodic": [lifter.Periodic(right, left)]}[case]
+    L = lifter.Lifter(n, *cons)
+    u = rng.standard_normal(L.size_reduced)
+    ref[L.free_dofs] = u
+    for c in cons:
+        ref[c.dofs] = ref[left] if case == "periodic" else c.values
+    assert np.array_equal(to_np(L.lift_from_zeros(u)), ref)
+    if case in ("all", "periodic"):
+        return
+    red = ta.Operator(mesh, ta.Tri3()).energy(PO).reduced(L)
+    v = rng.standard_normal(red.size)
+    r, hv = ta.jvp(red.grad, (u,), (v,))
+    assert np.array_equal(to_np(r), to_np(red.residual(u)))
+    assert np.array_equal(to_np(hv), to_np(red.hvp(u, v)))
+    cm = sparse.ColoredMatrix.from_csr(L.adapt_sparsity(sparse.pattern_from_mesh(mesh, 1)))
+    r, K = sparse.linearized_jacfwd(red.grad, cm)(u)
+    assert np.array_equal(to_np(r), to_np(red.residual(u)))
+    assert np.array_equal(to_np(K.data), to_np(sparse.jacfwd(red.grad, cm)(u).data))
