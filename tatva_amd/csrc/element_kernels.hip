@@ -271,7 +271,10 @@ __global__ __launch_bounds__(kBlock) void k_integrate_elem(int64_t n_elem, const
 }
 
 // partials[block] = block share of sum_e sum_q vals[e, q, c] * detJ * w_q for
-// one component c (grid-stride over elements; no per-element buffer).
+// one component c (grid-stride over elements; no per-element buffer).  The values of
+// eight points are loaded together, and Hex8 takes det J from the coordinate modes:
+// a point at a time, with the gradients of all eight nodes, a field on 64 x 61 x 67
+// Hex8 took 14.6 us, now 10.0.
 template <int KIND>
 __global__ __launch_bounds__(kBlock) void k_integrate_comp(int64_t n_elem, const double *__restrict__ coords,
                                                            const int32_t *__restrict__ conn,
@@ -279,26 +282,52 @@ __global__ __launch_bounds__(kBlock) void k_integrate_comp(int64_t n_elem, const
                                                            const double *__restrict__ vals,
                                                            double *__restrict__ partials) {
   using El = Elem<KIND>;
-  constexpr int D = El::D, NNE = El::NNE;
+  constexpr int D = El::D, NNE = El::NNE, kChunk = KIND == TATVA_HEX8 ? 8 : 1;
   double s = 0.0;
   for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < n_elem;
        e += (int64_t)gridDim.x * blockDim.x) {
     int32_t nodes[NNE];
     double X[NNE][D];
     load_element<KIND>(e, conn, coords, nodes, X);
-    for (int q = 0; q < quad.nq; ++q) {
-      const double w = qp_detJ<KIND>(X, quad.xi[q]) * quad.w[q];
-      double v;
-      if (nodal) {
-        double N[NNE];
-        El::N(quad.xi[q], N);
-        v = 0.0;
+    double XM[D][8];  // (Hex8)
+    if constexpr (KIND == TATVA_HEX8) hex_modes<double, 3>(X, XM);
+    for (int q0 = 0; q0 < quad.nq; q0 += kChunk) {
+      double v[kChunk];
+      if (!nodal) {
 #pragma unroll
-        for (int a = 0; a < NNE; ++a) v += N[a] * vals[(int64_t)nodes[a] * nc + c];
-      } else {
-        v = vals[(e * quad.nq + q) * nc + c];
+        for (int k = 0; k < kChunk; ++k) {
+          const int q = q0 + k < quad.nq ? q0 + k : q0;
+          v[k] = vals[(e * quad.nq + q) * nc + c];
+        }
       }
-      s += v * w;
+#pragma unroll
+      for (int k = 0; k < kChunk; ++k) {
+        const int q = q0 + k;
+        if (q >= quad.nq) break;
+        double w;
+        if constexpr (KIND == TATVA_HEX8) {
+          double J[3][3];
+#pragma unroll
+          for (int j = 0; j < 3; ++j) {
+            double d[3];
+            hex_dmodes<double>(XM[j], quad.xi[q][0], quad.xi[q][1], quad.xi[q][2], d);
+            J[0][j] = d[0];
+            J[1][j] = d[1];
+            J[2][j] = d[2];
+          }
+          w = det_only(J) * quad.w[q];
+        } else {
+          w = qp_detJ<KIND>(X, quad.xi[q]) * quad.w[q];
+        }
+        if (nodal) {
+          double N[NNE];
+          El::N(quad.xi[q], N);
+          v[k] = 0.0;
+#pragma unroll
+          for (int a = 0; a < NNE; ++a) v[k] += N[a] * vals[(int64_t)nodes[a] * nc + c];
+        }
+        s += v[k] * w;
+      }
     }
   }
   s = block_sum(s);

@@ -338,3 +338,22 @@ def test_lift_in_one_pass_and_once_per_jvp(case):
     r, K = sparse.linearized_jacfwd(red.grad, cm)(u)
     assert np.array_equal(to_np(r), to_np(red.residual(u)))
     assert np.array_equal(to_np(K.data), to_np(sparse.jacfwd(red.grad, cm)(u).data))
+
+
+@pytest.mark.parametrize("points", [1, 2, 3])
+@pytest.mark.parametrize("shape", [(1, 1, 1), (7, 5, 9)])
+def test_hex8_integrals(shape, points):
+    """1, 8 and 27 points in chunks of eight: fields at the points and at the nodes,
+    one component and three; sums of values of one sign, so relative to the result."""
+    el = ta.Hexahedron8(*gauss(points))
+    mesh = ta.Mesh.box(shape, jitter=0.1, seed=6)
+    oel = fem.Hex8(el.quad_points, el.quad_weights)
+    op = ta.Operator(mesh, el)
+    rng = np.random.default_rng(3)
+    for field in (rng.uniform(1, 2, (mesh.n_elements, points**3)),
+                  rng.uniform(1, 2, (mesh.n_elements, points**3, 3)),
+                  rng.uniform(1, 2, mesh.n_nodes), rng.uniform(1, 2, (mesh.n_nodes, 3))):
+        if field.shape[0] == mesh.n_nodes and mesh.n_nodes == mesh.n_elements:
+            continue
+        ref = fem.integrate(oel, mesh.coords, mesh.elements, field)
+        assert rel_err(to_np(op.integrate(field)), ref) < RTOL
