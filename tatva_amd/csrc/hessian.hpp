@@ -370,9 +370,11 @@ __device__ __forceinline__ void lds_add(double *p, double v) {
 // One group of LG lanes per node.  The group's compressed Jacobian rows
 // J[c][color] live in LDS (the last slot takes constrained columns); the
 // node's elements are taken P at a time in ascending order, their blocks added to
-// J one element after another (inside an element every column has its own color;
-// a simplex's block goes through LDS to all lanes of the group first), so the
-// sums have one order.  Then
+// J one element after another (a simplex's block goes through LDS to all lanes of
+// the group first), so the sums have one order where the columns of an element
+// have colors of their own: a distance-2 coloring of a pattern that couples an
+// element's dofs.  Only the last slot, which is never read, takes several
+// columns of an element at once.  Then
 // data[k] = J[c][colors[indices[k]]] (sparse/base.py:173).
 // The loads are issued level by level (the node's rows and elements, their row
 // ranges and element nodes, column indices and node data, colors), none behind
@@ -467,6 +469,7 @@ __global__ __launch_bounds__(kBlock) void k_node_rows(
 #pragma unroll
   for (int i = 0; i < Sh::kPre; ++i) pre[i] = colors[pre[i]];
   for (int i = lane; i < NC * ncol; i += LG) Jr[i] = 0.0;
+  wave_lds_sync();  // the lanes add to entries that others have zeroed
   for (int32_t p0 = b0; p0 < b1; p0 += P) {
     const int cnt = b1 - p0 < P ? b1 - p0 : P;
     const int a = packed & 7;

@@ -357,3 +357,28 @@ def test_hex8_integrals(shape, points):
             continue
         ref = fem.integrate(oel, mesh.coords, mesh.elements, field)
         assert rel_err(to_np(op.integrate(field)), ref) < RTOL
+
+
+@pytest.mark.parametrize("density", [LE, PO], ids=["le", "poisson"])
+@pytest.mark.parametrize("form", ["box", "turned", "general"])
+def test_hessian_rows_after_lds_of_nan(form, density):
+    """A node's rows are zeroed in LDS by other lanes than those that add to them: on
+    every geometry variant, right after kernels that leave NaN in the LDS, the rows
+    equal the oracle's, and those of a second assembly bit for bit."""
+    import torch
+
+    mesh = hex_variant(form, (11, 9, 8))
+    op = ta.Operator(mesh, ta.Hexahedron8())
+    E = op.energy(density)
+    cm = sparse.ColoredMatrix.from_csr(sparse.pattern_from_mesh(mesh, E.ncomp))
+    J = sparse.jacfwd(E.grad, cm)
+    nan = torch.full((E.size,), float("nan"), dtype=torch.float64, device="cuda")
+    u = torch.zeros(E.size, dtype=torch.float64, device="cuda")
+    data = []
+    for _ in range(2):
+        E.residual(nan)
+        op.grad(nan.reshape(mesh.n_nodes, -1))
+        data.append(to_np(J(u).data))
+    assert np.array_equal(data[0], data[1])
+    ref = hessian_pair(mesh, ta.Hexahedron8(), density, ORACLE[density])[1]
+    assert rel_err(data[0], ref) < RTOL
