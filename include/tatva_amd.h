@@ -133,7 +133,8 @@ int tatva_mesh_destroy(tatva_mesh *mesh);
 /* Sizes of a mesh handle's device layout (no counterpart in the reference; for
  * byte counts of the kernels): out[0..n) of {n_nodes, n_elements, n_tiles,
  * n_slots (tile, local node) pairs, largest local node count of a tile, largest
- * element color count of a tile, affine Hex8 flag, quadrature points}. */
+ * element color count of a tile, affine Hex8 flag, quadrature points, flag of a
+ * Hex8 mesh of boxes along the axes}. */
 int tatva_mesh_info(const tatva_mesh *mesh, int64_t *out, int32_t n);
 
 /* Integration weights detJ*w_q, out (E, Q).

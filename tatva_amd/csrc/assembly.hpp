@@ -683,8 +683,10 @@ __device__ __forceinline__ void hex8_element(const double (&X)[8][3], const T (&
 }
 
 // 1 when the element's bilinear coordinate modes are all exactly zero (computed
-// with the same butterfly as hex_modes), 2 when its Jacobian is diagonal too
-// (a box along the axes, whose edges along an axis are then equal), else 0.
+// with the same butterfly as hex_modes), 2 when it is a box along the axes too: each
+// coordinate takes one value at the nodes on either side, so any edge gives the
+// diagonal of the Jacobian (zero linear modes would not say so: their sums round,
+// and hide shears of the coordinates' last place), else 0.
 inline int hex_affine_host(const double (&X)[8][3]) {
   int kind = 2;
   for (int j = 0; j < 3; ++j) {
@@ -698,8 +700,8 @@ inline int hex_affine_host(const double (&X)[8][3]) {
           v[b | h] = hi - lo;
         }
     if (v[3] != 0.0 || v[5] != 0.0 || v[6] != 0.0 || v[7] != 0.0) return 0;
-    for (int k = 0; k < 3; ++k)
-      if (k != j && v[1 << k] != 0.0) kind = 1;
+    for (int a = 0; a < 8; ++a)
+      if (X[a][j] != ((hex_bin(a) >> j) & 1 ? X[6][j] : X[0][j])) kind = 1;
   }
   return kind;
 }

@@ -1269,9 +1269,10 @@ extern "C" int tatva_mesh_destroy(tatva_mesh *m) {
 
 extern "C" int tatva_mesh_info(const tatva_mesh *m, int64_t *out, int32_t n) {
   TATVA_REQUIRE(m && out && n >= 0, "invalid arguments");
-  const int64_t v[8] = {m->n_nodes,       m->n_elements,           m->tiles.n_tiles, m->n_slots,
-                        m->tiles.max_local, m->tiles.max_colors, m->hex_affine,    m->quad.nq};
-  for (int32_t i = 0; i < n && i < 8; ++i) out[i] = v[i];
+  const int64_t v[9] = {m->n_nodes,         m->n_elements,       m->tiles.n_tiles,
+                        m->n_slots,         m->tiles.max_local,  m->tiles.max_colors,
+                        m->hex_affine,      m->quad.nq,          m->hex_box};
+  for (int32_t i = 0; i < n && i < 9; ++i) out[i] = v[i];
   return TATVA_OK;
 }
 

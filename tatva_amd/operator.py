@@ -105,10 +105,10 @@ class Operator:
     def device_layout(self) -> dict:
         """Sizes of the mesh's device layout (tiles of elements and their
         (tile, local node) slots), for the kernels' byte counts."""
-        out = (ctypes.c_int64 * 8)()
-        nat.check(nat.lib().tatva_mesh_info(self.handle, out, 8))
+        out = (ctypes.c_int64 * 9)()
+        nat.check(nat.lib().tatva_mesh_info(self.handle, out, 9))
         keys = ("n_nodes", "n_elements", "n_tiles", "n_slots", "max_local", "max_colors",
-                "hex_affine", "n_quad")
+                "hex_affine", "n_quad", "hex_box")
         return {k: int(v) for k, v in zip(keys, out)}
 
     @property

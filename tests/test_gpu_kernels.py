@@ -382,3 +382,27 @@ def test_hessian_rows_after_lds_of_nan(form, density):
     assert np.array_equal(data[0], data[1])
     ref = hessian_pair(mesh, ta.Hexahedron8(), density, ORACLE[density])[1]
     assert rel_err(data[0], ref) < RTOL
+
+
+def test_boxes_are_told_by_their_coordinates():
+    """A Hex8 of equal edges whose corner line is one last place off has no linear or
+    bilinear mode that is not rounded to zero, and is no box: two of its nodes across
+    the body do not give its edge lengths.  One element, the corner line along x at
+    y = z = 1 shifted; and meshes that are boxes, turned, sheared and general."""
+    def hex_box(mesh):
+        return ta.Operator(mesh, ta.Hexahedron8()).device_layout()["hex_box"]
+
+    # lo + hi is an odd number of last places, a tie in the coarser sum: one place less
+    # at both rounds to the same
+    place = np.spacing(0.875)
+    m = ta.Mesh.box((1, 1, 1), lengths=(0.0625, 1.0, 1.0), origin=(0.875, 0.0, 0.0))
+    X = m.coords.copy()
+    X[X[:, 0] > 0.9, 0] += place
+    assert hex_box(m.set_coords(X)) == 1
+    X[(X[:, 1] == 1.0) & (X[:, 2] == 1.0), 0] -= place
+    v = X[:, 0][m.elements[0]][[0, 1, 3, 2, 4, 5, 7, 6]].reshape(2, 2, 2)  # z, y, x
+    for axis in (2, 1, 0):
+        v = np.stack([v.take(1, axis) + v.take(0, axis), v.take(1, axis) - v.take(0, axis)], axis)
+    assert np.count_nonzero(v) == 2  # the sum and the x mode
+    assert hex_box(m.set_coords(X)) == 0
+    assert [hex_box(hex_variant(f)) for f in ("box", "turned", "sheared", "general")] == [1, 0, 0, 0]
