@@ -379,8 +379,9 @@ __global__ __launch_bounds__(kBlock) void k_density_eval(int64_t n_elem, int nq,
 }
 
 // Sum over elements of sum_q psi(G_q) detJ w_q (+ Poisson source via u_q):
-// simplices.  Hex8 energies run on the tiles (kModeEnergy): nodes staged in LDS and
-// modal derivatives, 80^3 distorted Neo-Hookean 65.8 -> 45.7 us.
+// simplices, and Hex8 meshes whose tiles do not fit the LDS.  Other Hex8 energies run
+// on the tiles (kModeEnergy): nodes staged in LDS and modal derivatives, 80^3 distorted
+// Neo-Hookean 65.8 -> 45.7 us.
 template <int KIND, class Dens>
 __global__ __launch_bounds__(kBlock) void k_energy(int64_t n_elem, const double *__restrict__ coords,
                                                    const int32_t *__restrict__ conn, QuadRule quad,
@@ -1413,14 +1414,17 @@ extern "C" int tatva_energy(tatva_mesh *m, const tatva_density *d, const double 
     constexpr int K = decltype(kc)::value;
     return with_density<Elem<K>::D, double>(d, [&](auto dens) -> int {
       using Dens = decltype(dens);
-      int g;
-      if constexpr (K == TATVA_HEX8) {
-        g = m->tiles.n_tiles;
+      // Hex8: on the tiles where their nodes fit the LDS (up to 1365 of three
+      // components; 256 elements that share few nodes have up to 2048)
+      const bool tiled = K == TATVA_HEX8 &&
+                         tile_lds_bytes(K, m->tiles.max_local, Elem<K>::D, Elem<K>::NNE, Dens::NC,
+                                        sizeof(double), kModeEnergy) <= kTileLdsMax;
+      const int g = tiled ? m->tiles.n_tiles : reduce_grid(m->n_elements);
+      if (tiled) {
         const int e = launch_assembly<double, kModeEnergy>(m, d, u, nullptr, nullptr, nullptr,
                                                            nullptr, s, nullptr, m->partials);
         if (e) return e;
       } else {
-        g = reduce_grid(m->n_elements);
         k_energy<K, Dens><<<g, kBlock, 0, s>>>(m->n_elements, m->coords, m->conn, m->quad, dens, u,
                                                m->partials);
       }

@@ -406,3 +406,19 @@ def test_boxes_are_told_by_their_coordinates():
     assert np.count_nonzero(v) == 2  # the sum and the x mode
     assert hex_box(m.set_coords(X)) == 0
     assert [hex_box(hex_variant(f)) for f in ("box", "turned", "sheared", "general")] == [1, 0, 0, 0]
+
+
+@pytest.mark.parametrize("density", [LE, NH, PO], ids=["le", "nh", "poisson"])
+@pytest.mark.parametrize("joined,elements", [(1, 255), (1, 256), (1, 700), (2, 512)])
+def test_hex8_energy_of_separate_bodies(joined, elements, density):
+    """Bodies of one or two elements: a tile of 256 elements has up to 2048 nodes, more
+    than its LDS holds (1365 of three components).  Tolerance as test_hex8_energy_by_tiles."""
+    body = ta.Mesh.box((joined, 1, 1), jitter=0.1, seed=7)
+    k = elements // joined
+    X = (body.coords + 3.0 * np.arange(k)[:, None, None] * [0, 0, 1]).reshape(-1, 3)
+    conn = (body.elements + body.n_nodes * np.arange(k)[:, None, None]).reshape(-1, 8)
+    mesh = ta.Mesh(X, conn)
+    E = ta.Operator(mesh, ta.Hexahedron8()).energy(density)
+    u = 0.02 * np.random.default_rng(3).uniform(-1, 1, E.size)
+    ref = fem.Problem(fem.Hex8(), mesh.coords, mesh.elements, ORACLE[density]).energy(u)
+    assert abs(float(E(u)) - ref) < RTOL * (abs(ref) + 1.5 * 0.7 * k)
