@@ -197,7 +197,7 @@ class Residual:
 
     def jvp(self, u, v):
         """(r(u), H(u) v), as ``jax.jvp(jax.grad(E), (u,), (v,))``."""
-        if isinstance(self.energy, ReducedEnergy):
+        if type(self.energy) is ReducedEnergy:  # (a subclass may have its own residual or product)
             uf = self.energy.lift(u)  # once for both
             return self.energy.residual_full_state(uf), self.energy.hvp_full_state(uf, v)
         return self.energy.residual(u), self.energy.hvp(u, v)

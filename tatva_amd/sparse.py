@@ -347,8 +347,8 @@ def linearized_jacfwd(fn, colored_matrix: ColoredMatrix, *, color_batch_size: in
     asm = _HessianAssembler(fn, colored_matrix)
 
     def _wrapped(u):
-        if asm.reduced:
-            en = fn.energy
+        en = fn.energy
+        if type(fn) is Residual and type(en) is ReducedEnergy:  # (a subclass may have its own residual)
             uf = en.lift(u)  # once for both
             return (en.residual_full_state(uf),
                     replace(colored_matrix, data=asm.assemble_full_state(uf, en.lifter)))

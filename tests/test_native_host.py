@@ -461,3 +461,57 @@ def test_hvp_tile_bytes_counts_every_array_once():
     # Tri3, two components: every color offset, 2-D coordinates
     tri3 = (2 * 3 * E + S * (4 + 8 * 2 + 8 + 8 + 8 + 8 + 4) + T * (2 * (C + 1) + 8))
     assert bench.hvp_tile_bytes(Op(0, lay), dens_ncomp=2, mapped=True)[0] == tri3
+
+
+def test_subclasses_keep_their_own_residual_and_product():
+    """jvp and linearized_jacfwd lift once and pass by residual() and hvp() of the built-in
+    reduced energy only: those of a subclass are called."""
+    from tatva_amd import energies
+
+    class OwnEnergy(energies.ReducedEnergy):
+        size = 1
+
+        def __init__(self):
+            pass
+
+        def lift(self, u):
+            return ("lifted", u)
+
+        def residual_full_state(self, uf):
+            return ("built-in residual", uf)
+
+        def hvp_full_state(self, uf, v):
+            return ("built-in product", uf, v)
+
+        def residual(self, u):
+            return ("own residual", u)
+
+        def hvp(self, u, v):
+            return ("own product", u, v)
+
+    class OwnResidual(energies.Residual):
+        def __call__(self, u):
+            return ("own call", u)
+
+    class Assembler:
+        def __init__(self, fn, cm):
+            self.reduced = True
+
+        def __call__(self, u, data=None):
+            return np.zeros(1)
+
+        def assemble_full_state(self, uf, lifter=None, data=None):
+            return np.zeros(1)
+
+    assert ta.jvp(energies.Residual(OwnEnergy()), (1,), (2,)) == (("own residual", 1),
+                                                                 ("own product", 1, 2))
+    cm = sparse.ColoredMatrix(np.zeros(1), np.zeros(2, np.int32), np.zeros(1, np.int32), (1, 1),
+                              np.zeros(1, np.int32), 1)
+    own = object.__new__(energies.ReducedEnergy)
+    own.lift = own.residual_full_state = own.residual = lambda u: u
+    own.lifter = None
+    with pytest.MonkeyPatch.context() as mp:
+        mp.setattr(sparse, "_HessianAssembler", Assembler)
+        assert sparse.linearized_jacfwd(energies.Residual(OwnEnergy()), cm)(1)[0] == ("own residual", 1)
+        assert sparse.linearized_jacfwd(OwnResidual(own), cm)(1)[0] == ("own call", 1)
+        assert sparse.linearized_jacfwd(energies.Residual(own), cm)(1)[0] == 1
