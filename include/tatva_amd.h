@@ -193,8 +193,15 @@ int tatva_hessian_diag_f32(tatva_mesh *mesh, const tatva_density *density, const
 
 /* ------------------------------------------------------ colored Hessian ---- */
 
-/* Workspace bytes for tatva_colored_hessian on this mesh with ncomp components. */
+/* Workspace bytes that serve every call below on this mesh with ncomp components
+ * (the stiffness of every element). */
 int64_t tatva_colored_hessian_workspace(tatva_mesh *mesh, int ncomp);
+
+/* Workspace bytes that tatva_colored_hessian asks for with this density and
+ * n_colors: 0 (NULL is taken) where the rows come straight from the mesh, all but
+ * patterns of very many colors; -1 for invalid arguments. */
+int64_t tatva_colored_hessian_need(tatva_mesh *mesh, const tatva_density *density,
+                                   int32_t n_colors);
 
 /* Colored sparse Hessian decompressed into CSR data.  Replaces sparse.jacfwd /
  * colored_jacobian_batch (tatva/sparse/base.py:139-176,230-270): one JVP per

@@ -63,6 +63,7 @@ _SIGS = {
     "tatva_hessian_diag_f32": (c_int, [c_void, ctypes.POINTER(Density), c_void, c_void, c_void,
                                        c_void]),
     "tatva_colored_hessian_workspace": (c_i64, [c_void, c_int]),
+    "tatva_colored_hessian_need": (c_i64, [c_void, ctypes.POINTER(Density), c_i32]),
     "tatva_colored_hessian": (c_int, [c_void, ctypes.POINTER(Density), c_void, c_void, c_void, c_i64,
                                       c_void, c_i32, c_void, c_void, c_i64, c_void, c_void, c_i64,
                                       c_void]),

@@ -1700,6 +1700,32 @@ extern "C" int64_t tatva_colored_hessian_workspace(tatva_mesh *m, int nc) {
 
 static constexpr int kMaxColors = 2048;
 
+// Waves per block of k_node_rows for n_colors, as many as its LDS holds; 0: one
+// wave's rows do not fit, and the rows come from the element stiffness.
+template <int K, class Dens>
+static int node_rows_waves(const tatva_mesh *m, int32_t n_colors) {
+  using Sh = RowsShape<K, Dens::NC>;
+  const bool affine = K == TATVA_HEX8 && Dens::kLinear && m->hex_affine;
+  const size_t wave_lds = (kWave / Sh::LG) * Sh::lds_bytes(n_colors, !affine);
+  return (int)std::min<size_t>(kBlock / kWave, kTileLdsMax / wave_lds);
+}
+
+extern "C" int64_t tatva_colored_hessian_need(tatva_mesh *m, const tatva_density *d,
+                                              int32_t n_colors) {
+  if (!m || !d || n_colors < 1 || n_colors > kMaxColors) return -1;
+  int64_t need = -1;
+  const int rc = with_kind(m->kind, [&](auto kc) -> int {
+    constexpr int K = decltype(kc)::value;
+    return with_density<Elem<K>::D, double>(d, [&](auto dens) -> int {
+      using Dens = decltype(dens);
+      need = node_rows_waves<K, Dens>(m, n_colors) >= 1
+                 ? 0 : tatva_colored_hessian_workspace(m, Dens::NC);
+      return TATVA_OK;
+    });
+  });
+  return rc == TATVA_OK ? need : -1;
+}
+
 extern "C" int tatva_colored_hessian(tatva_mesh *m, const tatva_density *d, const double *u,
                                      const int32_t *dof_map, const int32_t *red_to_full,
                                      int64_t n_rows, const int32_t *colors, int32_t n_colors,
@@ -1714,8 +1740,6 @@ extern "C" int tatva_colored_hessian(tatva_mesh *m, const tatva_density *d, cons
   TATVA_REQUIRE(n_rows > 0, "the pattern has no rows");
   const int nc = density_ncomp(m, d);
   if (!dof_map) TATVA_REQUIRE(n_rows == m->n_nodes * nc, "pattern size does not match the mesh dofs");
-  const int64_t need = tatva_colored_hessian_workspace(m, nc);
-  TATVA_REQUIRE(workspace && ws_bytes >= need, "colored Hessian workspace too small");
   (void)nnz;
   hipStream_t s = (hipStream_t)stream;
   return with_kind(m->kind, [&](auto kc) -> int {
@@ -1724,12 +1748,10 @@ extern "C" int tatva_colored_hessian(tatva_mesh *m, const tatva_density *d, cons
       using Dens = decltype(dens);
       constexpr int NNE = Elem<K>::NNE, NC = Dens::NC;
       using Sh = RowsShape<K, NC>;
-      // node rows: as many nodes per block as its LDS holds, in whole waves
-      const bool affine_rows = K == TATVA_HEX8 && Dens::kLinear && m->hex_affine;
-      const size_t node_lds = Sh::lds_bytes(n_colors, !affine_rows);
-      const int waves = (int)std::min<size_t>(kBlock / kWave,
-                                              kTileLdsMax / ((kWave / Sh::LG) * node_lds));
+      const int waves = node_rows_waves<K, Dens>(m, n_colors);
       if (waves >= 1) {
+        const bool affine_rows = K == TATVA_HEX8 && Dens::kLinear && m->hex_affine;
+        const size_t node_lds = Sh::lds_bytes(n_colors, !affine_rows);
         const int threads = waves * kWave, per = threads / Sh::LG;
         const auto launch = [&](auto geom, auto mapped) {
           k_node_rows<K, Dens, decltype(geom)::value, decltype(mapped)::value>
@@ -1754,6 +1776,8 @@ extern "C" int tatva_colored_hessian(tatva_mesh *m, const tatva_density *d, cons
       }
       // so many colors that a wave's rows do not fit: one row per wave, from
       // the element stiffness
+      TATVA_REQUIRE(workspace && ws_bytes >= tatva_colored_hessian_workspace(m, NC),
+                    "colored Hessian workspace too small");
       double *Ke = (double *)workspace;
       const int rows_per_block = kBlock / kWave;
       const size_t lds = (size_t)rows_per_block * n_colors * sizeof(double);

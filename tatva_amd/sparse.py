@@ -267,13 +267,21 @@ class _HessianAssembler:
         if cm.n_colors > 2048:
             raise ValueError("more than 2048 colors are not supported")
         self._ws = None
+        self._need = {}
         self._serial = {}
 
-    def workspace(self):
-        if self._ws is None:
-            t = nat.torch()
-            nbytes = nat.lib().tatva_colored_hessian_workspace(self.full.op.handle, self.full.ncomp)
-            self._ws = t.empty(int(nbytes), dtype=t.uint8, device=nat.device())
+    def workspace(self, mapped: bool = True):
+        """The element stiffness, for the calls that go through it (``mapped``: a lifter with
+        Periodic constraints; else patterns of very many colors); empty for the others."""
+        if mapped not in self._need:
+            L, handle = nat.lib(), self.full.op.handle
+            self._need[mapped] = int(
+                L.tatva_colored_hessian_workspace(handle, self.full.ncomp) if mapped else
+                L.tatva_colored_hessian_need(handle, ctypes.byref(self.full._desc),
+                                             self.cm.n_colors))
+        nbytes = max(self._need[mapped], 0)  # (invalid arguments: the call itself says which)
+        if self._ws is None or self._ws.numel() < nbytes:
+            self._ws = nat.torch().empty(nbytes, dtype=nat.torch().uint8, device=nat.device())
         return self._ws
 
     def __call__(self, u, data=None):
@@ -302,10 +310,11 @@ class _HessianAssembler:
         cm = self.cm
         if data is None:
             data = t.empty(cm.nnz, dtype=t.float64, device=u_full.device)
-        ws = self.workspace()
+        mapped = lifter is not None and lifter.has_periodic
+        ws = self.workspace(mapped)
         desc = self.full._desc
         L = nat.lib()
-        if lifter is not None and lifter.has_periodic:
+        if mapped:
             ptr, lst = lifter.reduce_rows_device()
             nat.check(L.tatva_colored_hessian_mapped(
                 self.full.op.handle, ctypes.byref(desc), nat.dptr(u_full),

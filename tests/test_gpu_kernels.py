@@ -422,3 +422,53 @@ def test_hex8_energy_of_separate_bodies(joined, elements, density):
     u = 0.02 * np.random.default_rng(3).uniform(-1, 1, E.size)
     ref = fem.Problem(fem.Hex8(), mesh.coords, mesh.elements, ORACLE[density]).energy(u)
     assert abs(float(E(u)) - ref) < RTOL * (abs(ref) + 1.5 * 0.7 * k)
+
+
+@pytest.mark.parametrize("kind", ["hex8", "hex8-general", "tet4", "tri3"])
+@pytest.mark.parametrize("density", [LE, NH, PO], ids=["le", "nh", "poisson"])
+def test_hessian_takes_no_memory_that_it_does_not_use(kind, density):
+    """No element-stiffness buffer where the rows come from the mesh; the stiffness of
+    every element where the colors are too many (refused with a byte less) and in a
+    Periodic call of the same assembler."""
+    import ctypes
+
+    import torch
+
+    from tatva_amd import _native as nat
+
+    if kind == "tri3":
+        mesh, el = ta.Mesh.unit_square(9, 8), ta.Tri3()
+    elif kind == "tet4":
+        mesh, el = ta.Mesh.box((5, 4, 3), type="tetrahedron"), ta.Tetrahedron4()
+    else:
+        mesh, el = ta.Mesh.box((5, 4, 3), jitter=0.1 if kind == "hex8-general" else 0.0), ta.Hexahedron8()
+    op = ta.Operator(mesh, el)
+    E = op.energy(density)
+    L, h, desc = nat.lib(), op.handle, E._desc
+    full = L.tatva_colored_hessian_workspace(h, E.ncomp)
+    assert full == mesh.n_elements * (mesh.elements.shape[1] * E.ncomp) ** 2 * 8
+    needs = [L.tatva_colored_hessian_need(h, ctypes.byref(desc), c) for c in (1, 150, 2048)]
+    assert needs[:2] == [0, 0] and needs[2] in (0, full)
+    assert L.tatva_colored_hessian_need(h, ctypes.byref(desc), 0) == -1
+    assert L.tatva_colored_hessian_need(h, ctypes.byref(desc), 2049) == -1
+
+    cm = sparse.ColoredMatrix.from_csr(sparse.pattern_from_mesh(mesh, E.ncomp))
+    u = torch.zeros(E.size, dtype=torch.float64, device="cuda")
+    J = sparse.jacfwd(E.grad, cm)
+    K = J(u)
+    assert J.assembler.workspace(False).numel() == 0
+    n_colors = 2048
+    data = torch.empty(cm.nnz, dtype=torch.float64, device="cuda")
+    ws = torch.empty(max(full, 1), dtype=torch.uint8, device="cuda")
+
+    def call(nbytes):
+        return L.tatva_colored_hessian(h, ctypes.byref(desc), u.data_ptr(), None, None, E.size,
+                                       cm.colors.data_ptr(), n_colors, cm.indptr.data_ptr(),
+                                       cm.indices.data_ptr(), cm.nnz, data.data_ptr(),
+                                       ws.data_ptr() if nbytes else None, nbytes, nat.stream())
+
+    assert call(needs[2]) == nat.OK
+    assert rel_err(to_np(data), to_np(K.data)) < RTOL
+    if needs[2]:
+        assert call(needs[2] - 1) != nat.OK and call(0) != nat.OK
+    assert J.assembler.workspace().numel() == full
