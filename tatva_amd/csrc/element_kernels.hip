@@ -185,7 +185,8 @@ __global__ __launch_bounds__(kBlock) void k_point_field(int64_t n_elem, const do
   }
 }
 
-// The same for a number of components that is not a template parameter.
+// The same for a number of components that is not a template parameter, and for Hex8
+// rules of few points (kPointFieldMin).
 template <int KIND>
 __global__ __launch_bounds__(kBlock) void k_eval(int64_t n_elem, const int32_t *__restrict__ conn,
                                                  QuadRule quad, int nc, const double *__restrict__ u,
@@ -1297,13 +1298,26 @@ extern "C" int tatva_weights(tatva_mesh *m, double *out, void *stream) {
   });
 }
 
-// k_point_field for one, two or three components (else false).
+// Points from which k_point_field is the faster kernel on Hex8: its eight lanes of an
+// element take a point each, and with few points most of them wait for the nodes and
+// write nothing, where k_eval / k_grad give an element to a thread.  Gradients of one
+// component at 96^3: 4 points 64 us (k_grad) against 93, 5 points 88 and 94, 6 points
+// 115 and 97; of three: 1 point 42 and 131, 3 points 153 and 154, 4 points 208 and 171.
+// Values of one component: 3 points 21 and 30, 4 points 29 and 30, 5 points 32 and 31;
+// of two: 2 points 25 and 32, 3 points 37 and 33; of three: 1 point 20 and 36, 2 points
+// 39 and 38.
+template <bool GRAD, int NC>
+constexpr int kPointFieldMin = GRAD ? (NC == 1 ? 6 : 4) : (NC == 1 ? 5 : NC == 2 ? 3 : 2);
+
+// k_point_field for one, two or three components where it is the faster kernel (else false).
 template <int K, bool GRAD>
 static bool launch_point_field(const tatva_mesh *m, int nc, const double *u, double *out,
                                hipStream_t s) {
   constexpr int kElems = kBlock / (K == TATVA_HEX8 ? 8 : 1);
   const auto go = [&](auto ncc) {
-    k_point_field<K, decltype(ncc)::value, GRAD><<<grid_for(m->n_elements, kElems), kBlock, 0, s>>>(
+    constexpr int NC = decltype(ncc)::value;
+    if (K == TATVA_HEX8 && m->quad.nq < kPointFieldMin<GRAD, NC>) return false;
+    k_point_field<K, NC, GRAD><<<grid_for(m->n_elements, kElems), kBlock, 0, s>>>(
         m->n_elements, m->coords, m->conn, m->quad, u, out);
     return true;
   };
