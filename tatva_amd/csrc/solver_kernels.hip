@@ -805,8 +805,12 @@ static int get_res(int device, DeviceRes **out) {
   return TATVA_OK;
 }
 
+// Systems of at most kSmallRows rows may run in one workgroup (k_pcg_small).
+constexpr int kSmallRows = 4096;
+
 struct SellView {
   int64_t nsl = 0, steps = 0;
+  int64_t host_soff[kSmallRows / kSellRows + 1] = {};  // soff, of at most kSmallRows rows
   const int64_t *soff = nullptr;
   const int32_t *cols = nullptr;
   const double *vals = nullptr;
@@ -816,7 +820,7 @@ static size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
 // Lays the CSR matrix out as sliced ELL in the caller's workspace from byte
 // offset `at` (slice offsets, values, columns); one host synchronisation reads
-// the padded size, which must fit the workspace.
+// the padded size, which must fit the workspace (of small systems every offset).
 static int build_sell(int64_t n, const int32_t *indptr, const int32_t *indices,
                       const double *data, char *ws, size_t at, size_t ws_bytes, hipStream_t s,
                       SellView &V) {
@@ -827,8 +831,11 @@ static int build_sell(int64_t n, const int32_t *indptr, const int32_t *indices,
   k_sell_len<<<grid_for(V.nsl), kBlock, 0, s>>>(n, V.nsl, indptr, soff);
   k_scan_inplace<<<1, kBlock, 0, s>>>(soff, V.nsl + 1);
   TATVA_CHECK_LAUNCH();
-  TATVA_TRY_HIP(hipMemcpyAsync(&V.steps, soff + V.nsl, sizeof(int64_t), hipMemcpyDeviceToHost, s));
+  const int64_t first = n <= kSmallRows ? 0 : V.nsl;
+  TATVA_TRY_HIP(hipMemcpyAsync(V.host_soff, soff + first, (size_t)(V.nsl - first + 1) * sizeof(int64_t),
+                               hipMemcpyDeviceToHost, s));
   TATVA_TRY_HIP(hipStreamSynchronize(s));
+  V.steps = V.host_soff[V.nsl - first];
   const size_t entries = (size_t)V.steps * kSellRows;
   TATVA_REQUIRE(vals_at + entries * (sizeof(double) + sizeof(int32_t)) <= ws_bytes,
                 "PCG workspace too small for the sliced ELL copy");
@@ -969,7 +976,7 @@ static PcgParts parts_at(char *w, const WsLayout &L) {
 // A sliced-ELL system of at most kSmallRows rows runs its iterations in one
 // workgroup: a launch and two kernel boundaries per iteration cost more than the
 // work of such a system (64^2 Poisson, 3969 rows of 7: 8.2 us per iteration as two
-// kernels, 2.7 us here).  Lane l of wave w holds the rows of slices w, w + 16, ...:
+// kernels, 2.7 us here).  Lane l of wave w holds the rows of slices w, w + 8, ...:
 // their first kSmallLen entries, s and D^-1 in registers (longer rows read the rest
 // from the last-level caches), u, p, x and 1 / D^-1 in LDS.  What bounds it: the FP64
 // instructions of eight waves on one CU and two barriers an iteration.  Seven entries
@@ -977,12 +984,15 @@ static PcgParts parts_at(char *w, const WsLayout &L) {
 // six the seventh comes from memory (3.2).  Eight waves of 256 registers, not sixteen
 // of 128 (3.9 us: spills, and every wave repeats the scalars).  The host takes it for
 // up to kSmallRows rows (128 KB of LDS) when the slices' longest rows are kSmallMean
-// on average, so that an iteration streams little.  The same recurrences
+// on average, so that an iteration streams little, and no wave reads more than
+// kSmallExtra entries a lane past its registers: they come one after another, 0.175 us
+// each, so that an iteration of 4096 rows takes 5.1 us with 16 of them in one wave, 7.5
+// with 28 and 10.3 with 44, against 8.1 to 8.8 us as two kernels.  The same recurrences
 // and tests as k_sell_spmv and k_cg_step<double>, with one sum over the workgroup per
 // iteration; r.u and r.r of the last step pass from launch to launch in the parts.
 constexpr int kSmallThreads = 512, kSmallWaves = kSmallThreads / kWave;
-constexpr int kSmallRows = 4096, kSmallSlices = kSmallRows / kSmallThreads, kSmallLen = 7;
-constexpr int kSmallMean = 8;
+constexpr int kSmallSlices = kSmallRows / kSmallThreads, kSmallLen = 7;
+constexpr int kSmallMean = 8, kSmallExtra = 24;
 constexpr int kSmallIters = 256;  // iterations per launch, at least
 static_assert(kSellRows == kWave, "a row per lane");
 
@@ -1129,6 +1139,18 @@ __global__ __launch_bounds__(kSmallThreads) void k_pcg_small(
     if (status >= 0) st->status = status;
     if (status >= 0) st->done = 1;
   }
+}
+
+// Entries a lane that the wave with most of them reads past its registers.
+static int64_t small_extra(const SellView &V) {
+  int64_t most = 0;
+  for (int w = 0; w < kSmallWaves; ++w) {
+    int64_t extra = 0;
+    for (int64_t sl = w; sl < V.nsl; sl += kSmallWaves)
+      extra += std::max<int64_t>(0, V.host_soff[sl + 1] - V.host_soff[sl] - kSmallLen);
+    most = std::max(most, extra);
+  }
+  return most;
 }
 
 // Runs captured chunks until the device state reports done; fills stats.
@@ -1457,7 +1479,7 @@ extern "C" int tatva_pcg_csr(int64_t n, int64_t nnz, const int32_t *indptr,
     return TATVA_OK;
   };
   const bool small = nblk == 1 && !profiling && n <= kSmallRows && gv <= kSmallThreads &&
-                     sv_ell.steps <= kSmallMean * sv_ell.nsl;
+                     sv_ell.steps <= kSmallMean * sv_ell.nsl && small_extra(sv_ell) <= kSmallExtra;
   const std::function<int(int, bool)> run_small = [&](int, bool) -> int {
     k_pcg_small<<<1, kSmallThreads, 0, s>>>((int)n, (int)sv_ell.nsl, sv_ell.soff, sv_ell.cols,
                                             sv_ell.vals, x, u, p, sv, dinv, P.rz(1), P.rr(1), gv,

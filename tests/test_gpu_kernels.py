@@ -511,3 +511,56 @@ def test_gradients_at_one_point_cost_less_than_at_eight():
         times.append(np.median(runs))
         op.close()
     assert times[0] < 0.39 * times[1]
+
+
+def system_with_long_rows(n, entries, rows):
+    """A diagonally dominant tridiagonal system with `entries` more in each of some rows
+    (and columns)."""
+    A = sps.diags([-1.0, 2.01, -1.0], [-1, 0, 1], shape=(n, n)).tolil()
+    for row in rows:
+        for col in row + 5 + np.arange(entries):
+            A[row, col % n] = A[col % n, row] = -0.001
+        A[row, row] += 0.001 * entries
+    A = A.tocsr()
+    A.sort_indices()
+    return A
+
+
+@pytest.mark.parametrize("entries,rows", [(28, [3]), (29, [3]), (300, [3]), (16, [3, 515]),
+                                          (17, [3, 515]), (40, range(3, 4096, 512))],
+                         ids=["24", "25", "296", "24-in-two", "26-in-two", "288-in-eight"])
+def test_small_csr_pcg_of_long_rows(entries, rows):
+    """At most, and more than, 24 entries past the registers in one wave of the
+    one-workgroup solve (rows of entries + 3, 7 in registers); tolerances as
+    test_small_csr_pcg."""
+    from tatva_amd import solvers
+
+    A = system_with_long_rows(4096, entries, rows)
+    b = np.random.default_rng(1).standard_normal(4096)
+    x, info = solvers.pcg(sparse.ColoredMatrix.from_csr(A), b, tol=1e-12)
+    assert info.converged
+    assert np.linalg.norm(b - A @ to_np(x)) < 1e-9 * np.linalg.norm(b)
+
+
+def test_small_csr_pcg_of_long_rows_is_no_slower_than_a_larger_one():
+    """Eight rows of 43 entries that one wave would read one after another: 128 iterations
+    of 4096 rows took 5.6 times those of 4097 (which never run in one workgroup); the
+    same kernels now, so half as much again is the limit.  Medians of five."""
+    import time
+
+    import torch
+
+    from tatva_amd import solvers
+
+    times = []
+    for n in (4096, 4097):
+        K = sparse.ColoredMatrix.from_csr(system_with_long_rows(n, 40, range(3, 4096, 512)))
+        b, ws = torch.ones(n, dtype=torch.float64, device="cuda"), solvers._Workspace()
+        runs = []
+        for maxiter in (16, 144) * 6:
+            start = time.perf_counter()
+            solvers.pcg(K, b, tol=0.0, maxiter=maxiter, workspace=ws)
+            torch.cuda.synchronize()
+            runs.append(time.perf_counter() - start)
+        times.append(np.median(runs[3::2]) - np.median(runs[2::2]))
+    assert times[0] < 1.5 * times[1]
