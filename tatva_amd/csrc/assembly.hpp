@@ -844,7 +844,12 @@ __device__ __forceinline__ void tile_assemble(int tile, const double *__restrict
   // (a constrained dof, r < 0, reads a valid dummy address and stores 0, so
   // that no load sits behind a branch).
   const T *dummy = reinterpret_cast<const T *>(coords);
-  // the tangent at this thread's first two local nodes, for the dot
+  // the tangent at this thread's first two local nodes, for the dot.  Hex8 keeps it from
+  // the staging; Tet4 reads it from the LDS after the element work, through which it
+  // would take registers (77 instead of 61: six waves a SIMD, not eight; 100^3 x 6 linear
+  // elasticity in a batch 187 us an iteration instead of 175, where Hex8 so read took
+  // 397 at 160^3, not 388).
+  constexpr bool kDotKept = kDot && NNE == 8;
   T v01[2][NC];
   const auto stage = [&](auto mapped) {
     constexpr bool kMapped = decltype(mapped)::value;
@@ -876,7 +881,7 @@ __device__ __forceinline__ void tile_assemble(int tile, const double *__restrict
           for (int c = 0; c < NC; ++c) {
             const T val = *(r[h][c] >= 0 ? v + r[h][c] : dummy);
             vv[h][c] = r[h][c] >= 0 ? val : T(0);
-            if (kDot && j0 == (int)threadIdx.x) v01[h][c] = vv[h][c];
+            if (kDotKept && j0 == (int)threadIdx.x) v01[h][c] = vv[h][c];
           }
       }
 #pragma unroll
@@ -976,6 +981,14 @@ __device__ __forceinline__ void tile_assemble(int tile, const double *__restrict
     for (int h = 0; h < 2; ++h) {
       const int j = (int)threadIdx.x + h * kTile;
       slot01[h] = ts.slot_pos[nb + (j < nloc ? j : 0)];
+    }
+    if constexpr (kDot && !kDotKept) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int j = (int)threadIdx.x + h * kTile;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) v01[h][c] = vs[(j < nloc ? j : 0) * NC + c];
+      }
     }
     __syncthreads();  // every element has read its nodes: the LDS is free
     T *ys = reinterpret_cast<T *>(lds);

@@ -515,3 +515,26 @@ def test_subclasses_keep_their_own_residual_and_product():
         assert sparse.linearized_jacfwd(energies.Residual(OwnEnergy()), cm)(1)[0] == ("own residual", 1)
         assert sparse.linearized_jacfwd(OwnResidual(own), cm)(1)[0] == ("own call", 1)
         assert sparse.linearized_jacfwd(energies.Residual(own), cm)(1)[0] == 1
+
+
+def kernel_registers():
+    """Vector registers of the built kernels by symbol, from the library's own metadata
+    (a kernel's map lists .symbol and, after it, .vgpr_count as a MessagePack integer)."""
+    data = open(nat.lib()._name, "rb").read()
+    out = {}
+    for m in re.finditer(rb"\.symbol(?:[\xa0-\xbf]|\xd9.|\xda..)(\w+)\.kd", data, re.S):
+        at = data.index(b".vgpr_count", m.end()) + len(b".vgpr_count")
+        out[m.group(1).decode()] = (data[at] if data[at] < 0x80 else data[at + 1] if data[at] == 0xcc
+                                    else int.from_bytes(data[at + 1:at + 3], "big"))
+    return out
+
+
+def test_simplex_batch_tiles_keep_eight_waves():
+    """The batch's Tet4 and Tri3 tile kernels are bound by latency and traffic: at most 64
+    registers, so that a SIMD holds eight waves (the dot's tangent kept through the element
+    work made it 77 and six, and 100^3 x 6 elements 6 % slower)."""
+    regs = {s: n for s, n in kernel_registers().items() if "k_batch_assemble" in s}
+    assert len(regs) == 5
+    for kind in (0, 1):
+        (n,) = [n for s, n in regs.items() if f"k_batch_assembleILi{kind}E" in s]
+        assert 0 < n <= 64
