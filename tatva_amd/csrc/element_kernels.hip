@@ -1778,9 +1778,16 @@ extern "C" int tatva_colored_hessian(tatva_mesh *m, const tatva_density *d, cons
           else launch(geom, std::false_type{});
         };
         using std::integral_constant;
-        if constexpr (K == TATVA_HEX8 && Dens::kLinear) {
-          if (m->hex_box) with_map(integral_constant<int, kGeomBox>{});
-          else if (affine_rows) with_map(integral_constant<int, kGeomAffine>{});
+        if constexpr (K == TATVA_HEX8) {
+          if constexpr (Dens::kLinear) {
+            if (affine_rows) {
+              if (m->hex_box) with_map(integral_constant<int, kGeomBox>{});
+              else with_map(integral_constant<int, kGeomAffine>{});
+              TATVA_CHECK_LAUNCH();
+              return TATVA_OK;
+            }
+          }
+          if (m->quad.nq == 1) with_map(integral_constant<int, kGeomOnePoint>{});
           else with_map(integral_constant<int, kGeomGeneral>{});
         } else {
           with_map(integral_constant<int, kGeomGeneral>{});

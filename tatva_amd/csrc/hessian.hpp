@@ -72,8 +72,11 @@ struct RowsShape {
 // of the row's node.  Columns are taken in the order j ^ s: lane s then keeps
 // slots 0..3 and sends 4..7 to lane s ^ 7, whose slots 3..0 they are, and so
 // on, with no selects; seen from lane s the element is mirrored in the
-// directions of s's bits, which the signs t fold in.
-template <class Dens>
+// directions of s's bits, which the signs t fold in.  ONE (a rule of one point): all
+// eight lanes take it, each for its own column, with no exchange (32^3 Neo-Hookean,
+// element order shuffled: 92 us, 212 with seven lanes' points left out by their weight;
+// from the element stiffness, a buffer that the last-level cache holds, 186).
+template <class Dens, bool ONE>
 __device__ __forceinline__ void hex8_row_blocks(const double *__restrict__ xs, int ja,
                                                 const QuadRule &quad, const Dens &dens, int s,
                                                 double (&out)[Dens::NC * Dens::NC]) {
@@ -84,9 +87,16 @@ __device__ __forceinline__ void hex8_row_blocks(const double *__restrict__ xs, i
 #pragma unroll
   for (int i = 0; i < NV; ++i) out[i] = 0.0;
   for (int q0 = 0; q0 < quad.nq; q0 += 8) {
-    const bool on = q0 + s < quad.nq;
+    const bool on = ONE || q0 + s < quad.nq;
     double x, y, z, wq;
-    lane_point(quad, q0, s, x, y, z, wq);
+    if constexpr (ONE) {
+      x = quad.xi[0][0];
+      y = quad.xi[0][1];
+      z = quad.xi[0][2];
+      wq = quad.w[0];
+    } else {
+      lane_point(quad, q0, s, x, y, z, wq);
+    }
     x *= t[0];
     y *= t[1];
     z *= t[2];
@@ -173,6 +183,10 @@ __device__ __forceinline__ void hex8_row_blocks(const double *__restrict__ xs, i
         }
       }
     };
+    if constexpr (ONE) {  // (slot 0 is the lane's own column)
+      block(0, out);
+      break;
+    }
     // slot j + what the partner sends to it, over the three exchanges
     const auto half = [&](int j, double (&v)[NV]) {
       double send[NV];
@@ -361,6 +375,9 @@ __device__ __forceinline__ void hex8_box_row_blocks(const double (&X)[3], int ja
   }
 }
 
+// k_node_rows on general Hex8 elements of a one-point rule.
+constexpr int kGeomOnePoint = -1;
+
 // p[0] += v on LDS.  A wave's LDS operations run in their order, so sums added one
 // instruction after another have one order without a wait between them.
 __device__ __forceinline__ void lds_add(double *p, double v) {
@@ -394,8 +411,10 @@ __global__ __launch_bounds__(kBlock) void k_node_rows(
                 P = Sh::P;
   constexpr bool kHex = KIND == TATVA_HEX8;
   constexpr int NL = kHex ? 1 : NNE;  // nodes a lane loads
-  constexpr bool AFFINE = GEOM != kGeomGeneral;
+  constexpr bool ONE = GEOM == kGeomOnePoint;
+  constexpr bool AFFINE = GEOM != kGeomGeneral && !ONE;
   static_assert(!AFFINE || (kHex && Dens::kLinear), "constant blocks");
+  static_assert(!ONE || kHex, "simplices take one lane an element");
   extern __shared__ unsigned char lds_raw[];
   const int lane = threadIdx.x % LG;
   const int pl = lane / S, s = lane % S;
@@ -512,7 +531,7 @@ __global__ __launch_bounds__(kBlock) void k_node_rows(
           for (int j = 0; j < 3; ++j) blk[lane * 6 + 3 + j] = ue[0][j];
         }
         wave_lds_sync();
-        hex8_row_blocks<Dens>(blk + pl * 48, hex_bin(a), quad, de, s, v);
+        hex8_row_blocks<Dens, ONE>(blk + pl * 48, hex_bin(a), quad, de, s, v);
         wave_lds_sync();  // the staged nodes have been read
       }
       // element after element, its eight lanes adding their blocks

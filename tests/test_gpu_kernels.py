@@ -487,6 +487,22 @@ def test_point_fields_of_rules_of_few_points(points, nc):
     assert rel_err(to_np(op.grad(u)), fem.op_grad(oel, mesh.coords, mesh.elements, u)) < RTOL
 
 
+def median_ms(call, runs=5, calls=20):
+    import torch
+
+    call()
+    times = []
+    for _ in range(runs):
+        start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        start.record()
+        for _ in range(calls):
+            call()
+        end.record()
+        end.synchronize()
+        times.append(start.elapsed_time(end))
+    return np.median(times)
+
+
 def test_gradients_at_one_point_cost_less_than_at_eight():
     """One point an element (an eighth of the output) took 0.59 of the time of eight on
     96^3 Hex8 when eight lanes shared an element whatever its rule; a thread an element
@@ -498,17 +514,7 @@ def test_gradients_at_one_point_cost_less_than_at_eight():
     times = []
     for points in (1, 2):
         op = ta.Operator(mesh, ta.Hexahedron8(*gauss(points)))
-        op.grad(u)
-        runs = []
-        for _ in range(5):
-            start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
-            start.record()
-            for _ in range(20):
-                op.grad(u)
-            end.record()
-            end.synchronize()
-            runs.append(start.elapsed_time(end))
-        times.append(np.median(runs))
+        times.append(median_ms(lambda op=op: op.grad(u)))
         op.close()
     assert times[0] < 0.39 * times[1]
 
@@ -564,3 +570,27 @@ def test_small_csr_pcg_of_long_rows_is_no_slower_than_a_larger_one():
             runs.append(time.perf_counter() - start)
         times.append(np.median(runs[3::2]) - np.median(runs[2::2]))
     assert times[0] < 1.5 * times[1]
+
+
+@pytest.mark.parametrize("density", [LE, NH, PO], ids=["le", "nh", "poisson"])
+@pytest.mark.parametrize("k", [3, 4, 9])
+def test_hessian_rows_at_one_point(k, density):
+    """General Hex8 elements of a one-point rule, whose lanes all take that point: nodes
+    in fewer, as many and more elements than are held at a time."""
+    got, ref = hessian_pair(fan("hex8", k), ta.Hexahedron8(*gauss(1)), density, ORACLE[density])
+    assert rel_err(got, ref) < RTOL
+
+
+def test_hessian_rows_at_one_point_cost_less_than_at_eight():
+    """32^3 Neo-Hookean: 212 us for one point and for eight when the lanes without a point
+    computed theirs for a weight of zero; 92 and 210 now, so 0.7 is between."""
+    import torch
+
+    mesh = ta.Mesh.box((32, 32, 32), jitter=0.1)
+    times = []
+    for points in (1, 2):
+        E = ta.Operator(mesh, ta.Hexahedron8(*gauss(points))).energy(NH)
+        u = torch.zeros(E.size, dtype=torch.float64, device="cuda")
+        J = sparse.jacfwd(E.grad, sparse.ColoredMatrix.from_csr(sparse.pattern_from_mesh(mesh, 3)))
+        times.append(median_ms(lambda J=J, u=u: J(u)))
+    assert times[0] < 0.7 * times[1]
