@@ -1429,8 +1429,13 @@ extern "C" int tatva_energy(tatva_mesh *m, const tatva_density *d, const double 
     return with_density<Elem<K>::D, double>(d, [&](auto dens) -> int {
       using Dens = decltype(dens);
       // Hex8: on the tiles where their nodes fit the LDS (up to 1365 of three
-      // components; 256 elements that share few nodes have up to 2048)
-      const bool tiled = K == TATVA_HEX8 &&
+      // components; 256 elements that share few nodes have up to 2048).  Not for one
+      // point on general elements of three components, where staging and modes cost
+      // more than one point's nodal gradients: linear elasticity 41 us by elements
+      // against 47 at 112^3, 59 and 68 at 128^3, the same at 96^3 and 160^3; two points
+      // are faster on the tiles at every size.
+      const bool one = m->quad.nq == 1 && !m->hex_affine && Dens::NC == 3;
+      const bool tiled = K == TATVA_HEX8 && !one &&
                          tile_lds_bytes(K, m->tiles.max_local, Elem<K>::D, Elem<K>::NNE, Dens::NC,
                                         sizeof(double), kModeEnergy) <= kTileLdsMax;
       const int g = tiled ? m->tiles.n_tiles : reduce_grid(m->n_elements);
