@@ -594,3 +594,172 @@ def test_hessian_rows_at_one_point_cost_less_than_at_eight():
         J = sparse.jacfwd(E.grad, sparse.ColoredMatrix.from_csr(sparse.pattern_from_mesh(mesh, 3)))
         times.append(median_ms(lambda J=J, u=u: J(u)))
     assert times[0] < 0.7 * times[1]
+
+
+def parallelepipeds(shape):
+    """Hex8 parallelepipeds that are no boxes: node numbers over 8 times a matrix of
+    multiples of 1/8, so that every sum of coordinates is exact."""
+    m = ta.Mesh.box(shape)
+    X = np.round(m.coords * shape) / 8.0
+    m = m.set_coords(X @ np.array([[1.0, 0.25, 0.0], [0.5, 1.0, 0.125], [0.0, -0.25, 1.0]]))
+    lay = ta.Operator(m, ta.Hexahedron8()).device_layout()
+    assert (lay["hex_affine"], lay["hex_box"]) == (1, 0)
+    return m
+
+
+@pytest.mark.parametrize("density", [LE, NH, PO], ids=["le", "nh", "poisson"])
+@pytest.mark.parametrize("points", [1, 2, 3])
+def test_parallelepipeds(points, density):
+    """Energy, residual, product, diagonal and Hessian rows (with and without constrained
+    dofs) against the oracle; tolerances as the tests of each above."""
+    import torch
+
+    mesh, el = parallelepipeds((5, 7, 9)), ta.Hexahedron8(*gauss(points))
+    E = ta.Operator(mesh, el).energy(density)
+    prob = fem.Problem(fem.Hex8(el.quad_points, el.quad_weights), mesh.coords, mesh.elements,
+                       ORACLE[density])
+    rng = np.random.default_rng(5)
+    u, v = 0.005 * rng.standard_normal(E.size), rng.standard_normal(E.size)
+    volume = 0.90625 * 315 / 512
+    assert abs(float(E(u)) - prob.energy(u)) < RTOL * (abs(prob.energy(u)) + 1.5 * 0.7 * volume)
+    assert rel_err(to_np(E.grad(u)), prob.residual(u)) < RTOL
+    assert rel_err(to_np(E.hvp(u, v)), prob.hvp(u, v)) < RTOL
+    assert rel_err(to_np(E.hessian_diag(u)), prob.hessian_diag(u)) < RTOL
+    u32, v32 = (torch.as_tensor(a, dtype=torch.float32, device="cuda") for a in (u, v))
+    u_, v_ = to_np(u32).astype(float), to_np(v32).astype(float)
+    assert rel_err(to_np(E.hvp(u32, v32)), prob.hvp(u_, v_)) < 2e-6
+    assert rel_err(to_np(E.hessian_diag(u32, dtype=torch.float32)), prob.hessian_diag(u_)) < 2e-6
+    nc = E.ncomp
+    for fixed in (None, np.r_[0:4 * nc, [11 * nc, 30 * nc + nc - 1]]):
+        got, ref = hessian_pair(parallelepipeds((4, 3, 5)), el, density, ORACLE[density], fixed=fixed)
+        assert rel_err(got, ref) < RTOL
+
+
+@pytest.mark.parametrize("density", [LE, NH, PO], ids=["le", "nh", "poisson"])
+def test_parallelepipeds_matfree_pcg(density):
+    """The FP32 PCG reads the geometry of parallelepipeds (44 bytes an element) or computes
+    it: the same bits, also where the linearisation is written through it.  Residual as
+    test_matfree_pcg_step_by_nodes."""
+    import torch
+
+    from tatva_amd import solvers
+
+    mesh = parallelepipeds((9, 7, 10))
+    E = ta.Operator(mesh, ta.Hexahedron8()).energy(density)
+    nc = E.ncomp
+    low = np.where(mesh.coords[:, 2] <= mesh.coords[:, 1] * 0.125)[0]
+    L = lifter.Lifter(E.size, lifter.Fixed((low[:, None] * nc + np.arange(nc)).ravel(), 0.0))
+    red = E.reduced(L)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    u = 1e-3 * torch.randn(E.size, dtype=torch.float32, device="cuda", generator=g)
+    b = torch.randn(red.size, dtype=torch.float32, device="cuda", generator=g)
+    try:
+        for lin in ("never", "always"):
+            solvers.set_linearization_cache(lin)
+            out = []
+            for geo in (True, False):
+                solvers.set_geometry_cache(geo)
+                x, info = solvers.pcg_matfree(red, u, b, tol=1e-4)
+                assert info.converged
+                out.append((info.iterations, x))
+            assert out[0][0] == out[1][0] and torch.equal(out[0][1], out[1][1])
+            r = b.double() - red.hvp_full_state(u.double(), out[0][1].double())
+            assert float(r.norm() / b.double().norm()) < 2e-4
+    finally:
+        solvers.set_geometry_cache(True)   # the defaults
+        solvers.set_linearization_cache("never")
+
+
+def batch_solve(problems, tol=1e-4):
+    """x of H(u) x = b of each (reduced energy, u, b) as slots of one batch, and its
+    iterations."""
+    import ctypes
+
+    import torch
+
+    from tatva_amd import _native as nat
+
+    L, s, B = nat.lib(), nat.stream(), ctypes.c_void_p()
+    nat.check(L.tatva_batch_create(0, len(problems), ctypes.byref(B)))
+    keep, xs = [], []
+    for k, (red, u, b) in enumerate(problems):
+        E, dmap, n = red.energy, red.lifter.dof_map_device(), red.size
+        diag = E.hessian_diag(u, dof_map=dmap, n_out=n, dtype=torch.float32)
+        x = torch.zeros_like(b)
+        nbytes = L.tatva_batch_slot_workspace(E.op.handle, E.ncomp, n)
+        ws = torch.empty(int(nbytes), dtype=torch.uint8, device="cuda")
+        nat.check(L.tatva_batch_start(B, k, E.op.handle, ctypes.byref(E._desc), nat.dptr(u),
+                                      nat.dptr(dmap), n, nat.dptr(diag), nat.dptr(b), nat.dptr(x),
+                                      tol, 2000, nat.dptr(ws), ws.numel(), s))
+        keep.append((diag, ws))
+        xs.append(x)
+    stats, running = (nat.PcgStats * len(problems))(), ctypes.c_int32(1)
+    for _ in range(300):
+        nat.check(L.tatva_batch_iterate(B, 8, s))
+        nat.check(L.tatva_batch_poll(B, stats, ctypes.byref(running), s))
+        if running.value == 0:
+            break
+    assert running.value == 0
+    assert all(st.reserved != 0 and st.status == 0 for st in stats)
+    for k in range(len(problems)):
+        nat.check(L.tatva_batch_release(B, k))
+    nat.check(L.tatva_batch_destroy(B))
+    return xs, [st.iterations for st in stats]
+
+
+def clamped(mesh, density, end):
+    """(reduced energy, state, right-hand side) with the nodes ``end`` fixed."""
+    import torch
+
+    E = ta.Operator(mesh, ta.Hexahedron8()).energy(density)
+    nc = E.ncomp
+    L = lifter.Lifter(E.size, lifter.Fixed((end[:, None] * nc + np.arange(nc)).ravel(), 0.0))
+    g = torch.Generator(device="cuda").manual_seed(E.size)
+    u = 1e-4 * torch.randn(E.size, dtype=torch.float32, device="cuda", generator=g)
+    red = E.reduced(L)
+    return red, u, torch.randn(red.size, dtype=torch.float32, device="cuda", generator=g)
+
+
+def test_batch_class_of_mixed_densities_and_geometries():
+    """Hex8 slots of every density on boxes, parallelepipeds and general elements, three
+    launch classes of three densities each: every slot as alone, bit for bit, and its
+    residual as test_matfree_pcg_step_by_nodes."""
+    import torch
+
+    problems = [clamped(mesh, density, np.where(ta.Mesh.box(shape).coords[:, 2] == 0.0)[0])
+                for shape, mesh in (((6, 5, 7), ta.Mesh.box((6, 5, 7))),
+                                    ((6, 5, 7), parallelepipeds((6, 5, 7))),
+                                    ((9, 6, 8), ta.Mesh.box((9, 6, 8), jitter=0.1)))
+                for density in (PO, LE, NH)]
+    together, its = batch_solve(problems)
+    for (red, u, b), x, it in zip(problems, together, its):
+        (alone,), (it_alone,) = batch_solve([(red, u, b)])
+        assert it == it_alone and torch.equal(x, alone)
+        r = b.double() - red.hvp_full_state(u.double(), x.double())
+        assert float(r.norm() / b.double().norm()) < 2e-4
+
+
+@pytest.mark.parametrize("density", [LE, NH, PO], ids=["le", "nh", "poisson"])
+def test_matfree_pcg_dot_of_tiles_of_many_nodes(density):
+    """Tiles of more than 512 local nodes (a beam one element thick: 1028), whose dot reads
+    v again past the first two of a thread: iterations within 10 % of the FP64 PCG's (a
+    wrong dot is a wrong step length) and the residual as test_matfree_pcg_step_by_nodes,
+    single and batched."""
+    from tatva_amd import solvers
+
+    mesh = ta.Mesh.box((515, 1, 1), lengths=(515.0, 1.0, 1.0))
+    red, u, b = clamped(mesh, density, np.where(mesh.coords[:, 2] == 0.0)[0])
+    lay = red.op.device_layout()
+    assert lay["max_local"] > 1024 and lay["n_tiles"] >= 2
+    cm = sparse.ColoredMatrix.from_csr(
+        red.lifter.adapt_sparsity(sparse.pattern_from_mesh(mesh, red.ncomp)))
+    data = sparse._HessianAssembler(red.grad, cm).assemble_full_state(u.double(), red.lifter)
+    H = sps.csr_matrix((to_np(data), to_np(cm.indices), to_np(cm.indptr)), shape=cm.shape)
+    b64 = to_np(b).astype(float)
+    want = fem.pcg(H, b64, tol=1e-4)[1]
+    single, info = solvers.pcg_matfree(red, u, b, tol=1e-4)
+    assert info.converged
+    (batched,), (its,) = batch_solve([(red, u, b)])
+    for x, it in ((single, info.iterations), (batched, its)):
+        assert abs(it - want) <= max(2, 0.1 * want)
+        assert np.linalg.norm(b64 - H @ to_np(x).astype(float)) < 2e-4 * np.linalg.norm(b64)
