@@ -84,6 +84,7 @@ template <int CTRL>
 __device__ __forceinline__ double dpp_move(double v) {
   return __hiloint2double(dpp_move<CTRL>(__double2hiint(v)), dpp_move<CTRL>(__double2loint(v)));
 }
+constexpr int kDppQuadFirst = 0x00;    // quad_perm [0, 0, 0, 0]
 constexpr int kDppXor1 = 0xB1;         // quad_perm [1, 0, 3, 2]
 constexpr int kDppXor2 = 0x4E;         // quad_perm [2, 3, 0, 1]
 constexpr int kDppHalfMirror = 0x141;  // lane ^ 7 inside each group of 8

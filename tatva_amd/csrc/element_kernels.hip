@@ -78,6 +78,12 @@ __global__ __launch_bounds__(kBlock) void k_weights(int64_t n_elem, const double
   for (int q = 0; q < quad.nq; ++q) out[e * quad.nq + q] = qp_detJ<KIND>(X, quad.xi[q]) * quad.w[q];
 }
 
+// Lane 0's value in every group of eight lanes (s: the lane in its group).
+__device__ __forceinline__ double first_of_eight(double v, int s) {
+  const double low = dpp_move<kDppQuadFirst>(v), high = dpp_move<kDppHalfMirror>(low);
+  return s < 4 ? low : high;
+}
+
 // Values (GRAD false) or gradients of a nodal field of NC components at the
 // quadrature points: out[(e * nq + q) * L + ...], L = NC or NC * D.  Hex8: eight
 // lanes an element, lane s loads one node for all eight and takes the points s,
@@ -116,12 +122,16 @@ __global__ __launch_bounds__(kBlock) void k_point_field(int64_t n_elem, const do
     wave_lds_sync();
   };
   if constexpr (kHex) {
+    // Gradients take the differences to the element's first node (the derivatives sum to
+    // zero), exact or nearly: summed as they are, coordinates of 1 on elements of 1/64
+    // leave rounding of some 64 last places in J.
     const int64_t g = conn[e * 8 + hex_bin(s)];
 #pragma unroll
-    for (int j = 0; j < 3; ++j)
-      if constexpr (GRAD) staged[lane * kStage + j] = coords[g * 3 + j];
-#pragma unroll
-    for (int c = 0; c < NC; ++c) staged[lane * kStage + 3 + c] = u[g * NC + c];
+    for (int j = 0; j < kStage; ++j) {
+      if (!GRAD && j < 3) continue;
+      const double v = j < 3 ? coords[g * 3 + j] : u[g * NC + j - 3];
+      staged[lane * kStage + j] = GRAD ? v - first_of_eight(v, s) : v;
+    }
     wave_lds_sync();
     const double *nodes = staged + (lane - s) * kStage;
     for (int q0 = 0; q0 < quad.nq; q0 += 8) {
@@ -131,7 +141,7 @@ __global__ __launch_bounds__(kBlock) void k_point_field(int64_t n_elem, const do
       if constexpr (GRAD) {
         double J[3][3] = {}, H[NC][3] = {}, inv[3][3];
 #pragma unroll
-        for (int a = 0; a < 8; ++a) {
+        for (int a = 1; a < 8; ++a) {
           double d[3];
           pt.dN(a, d);
 #pragma unroll

@@ -763,3 +763,31 @@ def test_matfree_pcg_dot_of_tiles_of_many_nodes(density):
     for x, it in ((single, info.iterations), (batched, its)):
         assert abs(it - want) <= max(2, 0.1 * want)
         assert np.linalg.norm(b64 - H @ to_np(x).astype(float)) < 2e-4 * np.linalg.norm(b64)
+
+
+def test_point_gradients_do_not_lose_the_coordinates_places():
+    """Gradients on small elements far from the origin (edges 1/64 at 100, 50, -70) against
+    80-bit arithmetic: the differences of an element's coordinates are exact, so J and the
+    natural gradients carry the rounding of some eight operations each and the inverse a
+    few more; 20 last places relative to the largest gradient bound them, where sums of the
+    coordinates themselves would leave 100 / (1/64) = 6400."""
+    mesh = ta.Mesh.box((6, 5, 7), lengths=(6 / 64, 5 / 64, 7 / 64), origin=(100.0, 50.0, -70.0),
+                       jitter=0.1, seed=3)
+    op = ta.Operator(mesh, ta.Hexahedron8())
+    u = np.random.default_rng(1).uniform(1.0, 2.0, (mesh.n_nodes, 3))
+    X, U = (a[mesh.elements].astype(np.longdouble) for a in (mesh.coords, u))
+    s = op.element._reference_nodes().astype(np.longdouble)
+    q = op.element.quad_points.astype(np.longdouble)
+    f = 1 + s[None] * q[:, None]  # (point, node, axis)
+    dN = np.stack([s[:, k] / 8 * np.prod(np.delete(f, k, axis=2), axis=2) for k in range(3)], axis=2)
+    J = np.einsum("qak,eaj->eqkj", dN, X)
+    H = np.einsum("qak,eac->eqkc", dN, U)
+    inv = np.empty_like(J)  # cofactors
+    for i in range(3):
+        for j in range(3):
+            a, b, c, d = (i + 1) % 3, (i + 2) % 3, (j + 1) % 3, (j + 2) % 3
+            inv[..., j, i] = J[..., a, c] * J[..., b, d] - J[..., a, d] * J[..., b, c]
+    det = np.einsum("...k,...k->...", J[..., 0, :], inv[..., :, 0])
+    ref = np.einsum("eqjk,eqkc->eqcj", inv / det[..., None, None], H)
+    err = np.max(np.abs(to_np(op.grad(u)).astype(np.longdouble) - ref))
+    assert err < 20 * np.finfo(float).eps * np.max(np.abs(ref))
