@@ -409,8 +409,10 @@ def device_gb_in_use():
     return (total - free) / 1e9
 
 
-def mesh_is_affine(op):
-    return bool(op.device_layout().get("hex_affine"))
+def geometry_cache_bytes(op):
+    """Bytes per element of the affine Hex8 geometry cache (0: the mesh is not affine)."""
+    lay = op.device_layout()
+    return 20 if lay.get("hex_box") else 44 if lay.get("hex_affine") else 0
 
 
 def hvp_tile_bytes(op, dens_ncomp=3, cached_lin=0, geo=False, defer_n=0, mapped=True):
@@ -583,15 +585,15 @@ def headline(args):
     # with the cache the PCG reads the linearisation (F^-1 and mu - lambda ln J: 10
     # floats per quadrature point) instead of the state
     cached = args.lin_cache != "never"     # the headline mesh is Hex8
-    geo = not args.no_geo_cache and mesh_is_affine(op)
+    geo = 0 if args.no_geo_cache else geometry_cache_bytes(op)
     defer = not args.no_defer
     full_vec = not args.no_full_vectors
     n_vec = mesh.n_nodes * 3 if full_vec else n_free   # length of the CG vectors
-    tile_bytes, lay = hvp_tile_bytes(op, cached_lin=10 if cached else 0, geo=20 if geo else False,
+    tile_bytes, lay = hvp_tile_bytes(op, cached_lin=10 if cached else 0, geo=geo,
                                      defer_n=n_vec if defer else 0, mapped=not full_vec)
     hbm_rate = tile_bytes / (tile_us * 1e-6) / 1e9 if tile_us else None
     # the profile's counters are those of the default kernel on this workload
-    default_kernel = n == 160 and not cached and geo and defer and full_vec
+    default_kernel = n == 160 and not cached and geo == 20 and defer and full_vec
     prof = profile_counters(HEADLINE_PROFILE) if default_kernel else {}
     valu = prof.get("valu_wave_instructions_per_launch")
     traffic = prof.get("hbm_bytes_per_launch")
@@ -632,7 +634,7 @@ def headline(args):
             "algorithmic_bytes": tile_bytes,
             "hbm_achieved_gbs": hbm_rate,
             "hbm_frac": hbm_rate / HBM_PEAK_GBS if hbm_rate else None,
-            "geometry_cache": geo,
+            "geometry_cache": bool(geo),
             "deferred_cg_update": defer,
             "full_length_cg_vectors": full_vec,
             "avg_launch_us": tile_us,

@@ -354,8 +354,8 @@ int tatva_pcg_matfree_f32_mapped(tatva_mesh *mesh, const tatva_density *density,
 
 /* A batch runs many matrix-free FP32 Jacobi-PCG solves (each with its own
  * mesh, density, constraints, state, tolerance) in shared launches: one tile
- * assembly and one gather launch per (element kind, density kind, quadrature)
- * class and one vector launch per iteration for all slots.  No counterpart
+ * assembly launch per (element kind, quadrature, Hex8 geometry) class, whatever
+ * its slots' densities, and one step launch per iteration for all slots.  No counterpart
  * in the reference (it is the serving loop's solver; the linear algebra is the
  * same as tatva_pcg_matfree_f32).  A slot's arithmetic does not depend on the
  * other slots, so its result is identical alone and in any mix. */

@@ -7,8 +7,8 @@
 // elements' vectors in registers and sums them per local node, then writes the
 // tile's node sums to its slots of a partial buffer.  The per-tile sum runs
 // one element color at a time into LDS accumulators (no two elements of a
-// color share a node; colors are separated by barriers) for Tri3 and Hex8
-// (6-13 colors a tile); Tet4 tiles have ~30 colors, so there every element
+// color share a node; colors are separated by barriers) for Tri3 (6-8 colors
+// a tile); in Hex8 and Tet4 tiles (up to 15 and ~30 colors) every element
 // writes its vector to LDS and each local node adds its entries in ascending
 // (slot, node) order from a per-tile incidence list (two barriers).
 // A node gather adds, per node, the slots of the tiles containing it in tile
@@ -43,7 +43,7 @@ struct TileSet {
   const int32_t *slot_ptr;   // (n_nodes + 1) node -> its slots
   const int32_t *slot_pos;   // (n_slots) node-major position of each tile slot's sums
   const int32_t *tnodes;     // (n_slots) global node of each slot
-  // Tet4 only: entries (slot * nne + a) of each local node, ascending, at
+  // Hex8 and Tet4: entries (slot * nne + a) of each local node, ascending, at
   // inc_list[tile * kTile * nne + ...]; local node j ends at inc_end[node_ptr + j]
   const uint16_t *inc_end;   // (n_slots)
   const uint16_t *inc_list;  // (n_tiles * kTile * nne)
