@@ -158,6 +158,34 @@ __global__ __launch_bounds__(kBlock) void k_point_field(int64_t n_elem, const do
 #pragma unroll
           for (int j = 0; j < 3; ++j)
             mine[lane * L + c * 3 + j] = H[c][0] * inv[j][0] + H[c][1] * inv[j][1] + H[c][2] * inv[j][2];
+        // an infinite value at a node: its gradients are infinite, not NaN as the
+        // differences and the zeros of the inverse make them
+        double finite = 0.0;
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+          for (int k = 0; k < 3; ++k) finite += 0.0 * H[c][k];
+        if (finite != 0.0) {
+#pragma unroll 1
+          for (int a = 0; a < 8; ++a) {
+            const int i = hex_bin(a);
+            const double sx = (i & 1) ? 1.0 : -1.0, sy = (i & 2) ? 1.0 : -1.0,
+                         sz = (i & 4) ? 1.0 : -1.0;
+            const double d[3] = {0.125 * sx * (1.0 + sy * y) * (1.0 + sz * z),
+                                 0.125 * sy * (1.0 + sx * x) * (1.0 + sz * z),
+                                 0.125 * sz * (1.0 + sx * x) * (1.0 + sy * y)};
+            const int64_t n = conn[e * 8 + a];
+#pragma unroll
+            for (int j = 0; j < 3; ++j) {
+              const double B = inv[j][0] * d[0] + inv[j][1] * d[1] + inv[j][2] * d[2];
+#pragma unroll
+              for (int c = 0; c < NC; ++c) {
+                double *g = mine + lane * L + c * 3 + j;
+                *g = (a > 0 ? *g : 0.0) + B * u[n * NC + c];
+              }
+            }
+          }
+        }
       } else {
 #pragma unroll
         for (int c = 0; c < NC; ++c) {

@@ -765,6 +765,22 @@ def test_matfree_pcg_dot_of_tiles_of_many_nodes(density):
         assert np.linalg.norm(b64 - H @ to_np(x).astype(float)) < 2e-4 * np.linalg.norm(b64)
 
 
+def shape_gradients(mesh, el):
+    """dN_a/dx_j at the points, (element, point, j, a), in 80-bit arithmetic."""
+    X = mesh.coords[mesh.elements].astype(np.longdouble)
+    s, q = el._reference_nodes().astype(np.longdouble), el.quad_points.astype(np.longdouble)
+    f = 1 + s[None] * q[:, None]  # (point, node, axis)
+    dN = np.stack([s[:, k] / 8 * np.prod(np.delete(f, k, axis=2), axis=2) for k in range(3)], axis=2)
+    J = np.einsum("qak,eaj->eqkj", dN, X)
+    inv = np.empty_like(J)  # cofactors
+    for i in range(3):
+        for j in range(3):
+            a, b, c, d = (i + 1) % 3, (i + 2) % 3, (j + 1) % 3, (j + 2) % 3
+            inv[..., j, i] = J[..., a, c] * J[..., b, d] - J[..., a, d] * J[..., b, c]
+    det = np.einsum("...k,...k->...", J[..., 0, :], inv[..., :, 0])
+    return np.einsum("eqjk,qak->eqja", inv / det[..., None, None], dN)
+
+
 def test_point_gradients_do_not_lose_the_coordinates_places():
     """Gradients on small elements far from the origin (edges 1/64 at 100, 50, -70) against
     80-bit arithmetic: the differences of an element's coordinates are exact, so J and the
@@ -775,19 +791,26 @@ def test_point_gradients_do_not_lose_the_coordinates_places():
                        jitter=0.1, seed=3)
     op = ta.Operator(mesh, ta.Hexahedron8())
     u = np.random.default_rng(1).uniform(1.0, 2.0, (mesh.n_nodes, 3))
-    X, U = (a[mesh.elements].astype(np.longdouble) for a in (mesh.coords, u))
-    s = op.element._reference_nodes().astype(np.longdouble)
-    q = op.element.quad_points.astype(np.longdouble)
-    f = 1 + s[None] * q[:, None]  # (point, node, axis)
-    dN = np.stack([s[:, k] / 8 * np.prod(np.delete(f, k, axis=2), axis=2) for k in range(3)], axis=2)
-    J = np.einsum("qak,eaj->eqkj", dN, X)
-    H = np.einsum("qak,eac->eqkc", dN, U)
-    inv = np.empty_like(J)  # cofactors
-    for i in range(3):
-        for j in range(3):
-            a, b, c, d = (i + 1) % 3, (i + 2) % 3, (j + 1) % 3, (j + 2) % 3
-            inv[..., j, i] = J[..., a, c] * J[..., b, d] - J[..., a, d] * J[..., b, c]
-    det = np.einsum("...k,...k->...", J[..., 0, :], inv[..., :, 0])
-    ref = np.einsum("eqjk,eqkc->eqcj", inv / det[..., None, None], H)
+    ref = np.einsum("eqja,eac->eqcj", shape_gradients(mesh, op.element), u[mesh.elements].astype(np.longdouble))
     err = np.max(np.abs(to_np(op.grad(u)).astype(np.longdouble) - ref))
     assert err < 20 * np.finfo(float).eps * np.max(np.abs(ref))
+
+
+@pytest.mark.parametrize("nc", [1, 2, 3])
+@pytest.mark.parametrize("points", [2, 3])
+@pytest.mark.parametrize("jitter", [0.0, 0.1])
+def test_point_gradients_of_infinite_values(jitter, points, nc):
+    """A node's infinite value makes the gradients around it infinite, with the signs of
+    its shape gradients (NaN where two disagree or the value is NaN), and no others."""
+    mesh, el = ta.Mesh.box((4, 3, 5), jitter=jitter, seed=5), ta.Hexahedron8(*gauss(points))
+    u = np.random.default_rng(0).standard_normal((mesh.n_nodes, nc))
+    u[37, 0], u[38, nc - 1], u[60, 0], u[0, nc - 1], u[11, 0] = np.inf, np.inf, -np.inf, -np.inf, np.nan
+    got = to_np(ta.Operator(mesh, el).grad(u))
+    B = shape_gradients(mesh, el).astype(float)
+    with np.errstate(invalid="ignore"):
+        ref = (B[:, :, None] * np.moveaxis(u[mesh.elements], 1, 2)[:, None, :, None]).sum(axis=-1)
+    assert np.isinf(ref).any() and np.isnan(ref).any()
+    for of in (np.isnan, np.isposinf, np.isneginf):
+        assert np.array_equal(of(got), of(ref))
+    finite = np.isfinite(ref)
+    assert rel_err(got[finite], ref[finite]) < RTOL
