@@ -92,7 +92,13 @@ __device__ __forceinline__ double first_of_eight(double v, int s) {
 // per element storing 72 bytes at a time at a stride of 576 took 96.5 us for the
 // gradients of three components on 64 x 61 x 67 Hex8, now 47.7 us (171 MB of output
 // and mesh, 3.6 TB/s).
-template <int KIND, int NC, bool GRAD>
+// Hex8 gradients take the nodes' differences to the element's first one (the derivatives
+// sum to zero), exact or nearly: summed as they are, coordinates of 1 on elements of 1/64
+// leave rounding of some 64 last places in J.  MANY (rules of more than eight points): the
+// nodes are staged as differences (27 points on 40^3: 35 us, 40 with the lanes
+// subtracting at every eight points); else the lanes subtract what they read (eight
+// points on 64 x 61 x 67, map of perf/cases.py: 98.9 us, 100.3 staged).
+template <int KIND, int NC, bool GRAD, bool MANY>
 __global__ __launch_bounds__(kBlock) void k_point_field(int64_t n_elem, const double *__restrict__ coords,
                                                         const int32_t *__restrict__ conn,
                                                         QuadRule quad, const double *__restrict__ u,
@@ -122,15 +128,12 @@ __global__ __launch_bounds__(kBlock) void k_point_field(int64_t n_elem, const do
     wave_lds_sync();
   };
   if constexpr (kHex) {
-    // Gradients take the differences to the element's first node (the derivatives sum to
-    // zero), exact or nearly: summed as they are, coordinates of 1 on elements of 1/64
-    // leave rounding of some 64 last places in J.
     const int64_t g = conn[e * 8 + hex_bin(s)];
 #pragma unroll
     for (int j = 0; j < kStage; ++j) {
       if (!GRAD && j < 3) continue;
       const double v = j < 3 ? coords[g * 3 + j] : u[g * NC + j - 3];
-      staged[lane * kStage + j] = GRAD ? v - first_of_eight(v, s) : v;
+      staged[lane * kStage + j] = GRAD && MANY ? v - first_of_eight(v, s) : v;
     }
     wave_lds_sync();
     const double *nodes = staged + (lane - s) * kStage;
@@ -142,14 +145,17 @@ __global__ __launch_bounds__(kBlock) void k_point_field(int64_t n_elem, const do
         double J[3][3] = {}, H[NC][3] = {}, inv[3][3];
 #pragma unroll
         for (int a = 1; a < 8; ++a) {
-          double d[3];
+          double d[3], v[3 + NC];
           pt.dN(a, d);
+#pragma unroll
+          for (int j = 0; j < 3 + NC; ++j)
+            v[j] = MANY ? nodes[a * kStage + j] : nodes[a * kStage + j] - nodes[j];
 #pragma unroll
           for (int k = 0; k < 3; ++k) {
 #pragma unroll
-            for (int j = 0; j < 3; ++j) J[k][j] += d[k] * nodes[a * kStage + j];
+            for (int j = 0; j < 3; ++j) J[k][j] += d[k] * v[j];
 #pragma unroll
-            for (int c = 0; c < NC; ++c) H[c][k] += d[k] * nodes[a * kStage + 3 + c];
+            for (int c = 0; c < NC; ++c) H[c][k] += d[k] * v[3 + c];
           }
         }
         det_inv(J, inv);
@@ -1355,8 +1361,15 @@ static bool launch_point_field(const tatva_mesh *m, int nc, const double *u, dou
   const auto go = [&](auto ncc) {
     constexpr int NC = decltype(ncc)::value;
     if (K == TATVA_HEX8 && m->quad.nq < kPointFieldMin<GRAD, NC>) return false;
-    k_point_field<K, NC, GRAD><<<grid_for(m->n_elements, kElems), kBlock, 0, s>>>(
-        m->n_elements, m->coords, m->conn, m->quad, u, out);
+    const auto launch = [&](auto many) {
+      k_point_field<K, NC, GRAD, decltype(many)::value>
+          <<<grid_for(m->n_elements, kElems), kBlock, 0, s>>>(m->n_elements, m->coords, m->conn,
+                                                             m->quad, u, out);
+    };
+    if (K == TATVA_HEX8 && GRAD && m->quad.nq > 8)
+      launch(std::bool_constant<K == TATVA_HEX8 && GRAD>{});
+    else
+      launch(std::false_type{});
     return true;
   };
   if (nc == 1) return go(std::integral_constant<int, 1>{});
