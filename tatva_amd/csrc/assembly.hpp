@@ -19,6 +19,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <cmath>
 #include <cstdint>
 #include <type_traits>
 
@@ -688,7 +689,11 @@ __device__ __forceinline__ void hex8_element(const double (&X)[8][3], const T (&
 // diagonal of the Jacobian (zero linear modes would not say so: their sums round,
 // and hide shears of the coordinates' last place), else 0.
 inline int hex_affine_host(const double (&X)[8][3]) {
-  int kind = 2;
+  bool box = true;
+  for (int a = 0; a < 8; ++a)
+    for (int j = 0; j < 3; ++j) box &= X[a][j] == X[(hex_bin(a) >> j) & 1 ? 6 : 0][j];
+  for (int j = 0; j < 3; ++j) box &= std::isfinite(8.0 * std::fabs(X[0][j]) + 8.0 * std::fabs(X[6][j]));
+  if (box) return 2;  // (its modes are exactly zero: equal sums and differences)
   for (int j = 0; j < 3; ++j) {
     double v[8];
     for (int a = 0; a < 8; ++a) v[hex_bin(a)] = X[a][j];
@@ -700,10 +705,8 @@ inline int hex_affine_host(const double (&X)[8][3]) {
           v[b | h] = hi - lo;
         }
     if (v[3] != 0.0 || v[5] != 0.0 || v[6] != 0.0 || v[7] != 0.0) return 0;
-    for (int a = 0; a < 8; ++a)
-      if (X[a][j] != ((hex_bin(a) >> j) & 1 ? X[6][j] : X[0][j])) kind = 1;
   }
-  return kind;
+  return 1;
 }
 
 // ------------------------------------------------------ tile assembly ------
